@@ -379,12 +379,14 @@ int plan_nodal(lulesh_ctx *c, int cz) {
     (void)hipGraphExecDestroy(c->graph);
     c->graph = nullptr;
   }
+  c->b.nodal_wide = 0;
   for (InstDesc &I : c->inst) {
     const NodalTile t = nodal_tile(I.s, c->tile_lo, c->tile_hi);
     I.etx = t.etx;
     I.ety = t.ety;
     I.tx = t.tx;
     I.ty = t.ty;
+    if (nodal_patch_wide(t)) c->b.nodal_wide = 1;
   }
   // default: auto_depth, balanced per instance; an explicit depth applies
   // unchanged to all instances

@@ -1,6 +1,9 @@
 // Correctly rounded FP64 cube root for the GPU kernels (and, compiled for
 // the host, for its test harness).  Any correctly rounded cube root returns
-// the same bits, so the method only decides the speed:
+// the same bits, so the method only decides the speed.  Arguments between
+// 2^-60 and 2^60 -- every element volume in practice -- take cbrt_mid below
+// (about 30 instructions instead of 130); what it cannot decide, and every
+// other argument, takes this general path:
 //
 //   1. x = t * 2^(3q) with t in [1, 8); a single-precision seed refined by
 //      two Newton steps y -= (y^3 - t) c, c ~ 1/(3 y^2) from a single-
@@ -87,9 +90,59 @@ LULESH_CBRT_FN int64_t cbrt_exact_k(uint64_t X, int64_t K) {
   return K;
 }
 
+// single-precision x^(1/3) of a normal x, to a relative 2^-19 for
+// 2^-60 <= x <= 2^60 (log2 to one ulp of at most 2^-18, a third of it, exp2)
+LULESH_CBRT_FN float cbrt_seed(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(x) * 0.333333343267440796f);
+#else
+  return cbrtf(x);
+#endif
+}
+
+// The cube root of 2^-60 <= x <= 2^60 without taking x apart; *decided says
+// whether the result is known to be the correctly rounded one.
+//   seed       y0 within a relative 2^-19;
+//   Newton     y = y0 - (y0^3 - x) c, c = 1 / (3 y0^2) to 2^-22, leaves a
+//              relative error below 2^-37;
+//   residual   r = x - y^3 with y^2 = y2 + e2 and y2 y = y3 + e3 exact by
+//              fused multiply-adds (x - y3 is exact): error below 2^-87 x;
+//   d = r / (3 y^2), c refined once (it belongs to y0, so it is within
+//              2^-18 before and 2^-36 after): the root is y + d within
+//              2^-73 y (d's own error, and the d^2 / y that Newton drops).
+// y + d is the correct rounding if y + (d - m) and y + (d + m) round alike
+// for m = 2^-71 y >= that error; they differ for one x in 2^17, which the
+// caller hands to the general path.
+LULESH_CBRT_FN double cbrt_mid(double x, bool *decided) {
+  const double y0 = (double)cbrt_seed((float)x);
+  const double s0 = y0 * y0;
+  double c = (double)cbrt_rcpf((float)(3.0 * s0));
+  const double y = fma(-fma(s0, y0, -x), c, y0);
+  const double y2 = y * y, e2 = fma(y, y, -y2);
+  const double y3 = y2 * y, e3 = fma(y2, y, -y3);
+  const double r = fma(-e2, y, (x - y3) - e3);
+  c = c * fma(-(3.0 * y2), c, 2.0);
+  const double d = r * c;
+  const double m = y * 4.2351647362715017e-22;  // 2^-71
+  const double lo = y + (d - m), hi = y + (d + m);
+  *decided = lo == hi;
+  return lo;
+}
+
+LULESH_CBRT_FN double cbrt_general(double x, bool exact_only, int64_t *slow);
+
 // the cube root, correctly rounded; for tests, `exact_only` skips the fast
-// decision and `*slow` counts the calls the exact path decided
+// decisions and `*slow` counts the calls the exact path decided
 LULESH_CBRT_FN double cbrt_cr(double x, bool exact_only = false, int64_t *slow = nullptr) {
+  if (!exact_only && x >= 8.6736173798840355e-19 && x <= 1152921504606846976.0) {
+    bool decided;
+    const double y = cbrt_mid(x, &decided);
+    if (decided) return y;
+  }
+  return cbrt_general(x, exact_only, slow);
+}
+
+LULESH_CBRT_FN double cbrt_general(double x, bool exact_only, int64_t *slow) {
   if (x == 0.0 || !isfinite(x)) return x + x;
   double ax = fabs(x);
   int sub = 0;

@@ -1,12 +1,11 @@
 // MI355X (gfx950) kernels of one LULESH Lagrange leap-frog cycle, FP64.
 //
-// One cycle = five launches on the context stream:
-//   k_force  element-parallel: stress corner forces (integrateStressForElems)
-//            and Flanagan-Belytschko hourglass corner forces
-//            (calcHourglassControlForElems + calcFBHourglassForceForElems)
-//   k_node   node-parallel: fixed-order corner gather (stress sum, then
-//            hourglass sum, as the reference sums them), acceleration,
-//            symmetry-plane BCs, velocity, position
+// One cycle = four launches on the context stream:
+//   k_nodal  stress corner forces (integrateStressForElems), Flanagan-
+//            Belytschko hourglass corner forces (calcHourglassControlForElems
+//            + calcFBHourglassForceForElems), their fixed-order sums at the
+//            nodes (stress, then hourglass, as the reference sums them),
+//            acceleration, symmetry-plane BCs, velocity, position
 //   k_kin    element-parallel: calcKinematicsForElems + the deviatoric loop
 //            + calcMonotonicQGradientsForElems
 //   k_qeos   element-parallel: calcMonotonicQRegionForElems, the QStop check,
@@ -15,8 +14,8 @@
 //            reduced to one minimum per block
 //   k_dt     one block: the final minima (calcTimeConstraintsForElems) and,
 //            in driver-loop mode, the loop test and the next timeIncrement!
-// No atomics touch field data: corners are written once and gathered in the
-// reference's order, so the FP64 result is deterministic run to run.
+// No atomics touch field data: a node sums its corners in the reference's
+// order, so the FP64 result is deterministic run to run.
 #include "lulesh_elem.h"
 #include "lulesh_kernels.h"
 
@@ -370,8 +369,70 @@ __global__ void k_run_begin(Batch B) {
 // Elements on tile edges are computed by every tile that needs them
 // (17x15x(cz+1) per 16x14xcz nodes for an inner 17 x 15 tile): no corner
 // force ever goes to HBM.
+//
+// What bounds it: FP64 issue.  A wave needs about 1,500 vector instructions
+// per element plane (6,000 cycles of a SIMD, whose two waves belong to two
+// workgroups), and a wave alone waits for as long again unless its memory
+// and LDS accesses are few and early.  Hence the node ring (a plane is
+// fetched once per tile, one plane ahead, instead of 24 16-byte gathers per
+// element, which kept the address path busy for 700 cycles per wave and
+// plane), the element values and nodal mass asked for a phase ahead, and
+// LDS reads without branches.  Timestamps inside the kernel at s=192: 19,000
+// cycles per plane for the workgroup issued first before, 12,500 now.  At
+// s=192 a launch takes 496 us against 615 (27 TFLOP/s of the 1,430 additions
+// and products per element and plane), the batch of 64 domains 403 against
+// 500, s=63 36 against 39.  243 VGPRs and 78 KB of LDS: two workgroups per
+// CU by either.
 // ---------------------------------------------------------------------------
+// Corner forces in LDS: [corner q of the bottom face][element slot][x y z of
+// corner q, x y z of corner q + 4 above it], so that a node takes what one
+// element gives it in three 16-byte reads (the 48-byte stride spreads
+// sixteen lanes over all 64 banks).  Slot BLOCK holds zeros.
+constexpr int LDS_PAIR = (BLOCK + 1) * 6;  // doubles per corner q
+LDEV int lds_at(int q, int slot) { return q * LDS_PAIR + slot * 6; }
+LDEV void lds_put(double *lds, int slot, const double (&F)[8][3]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    double2 *p = (double2 *)(lds + lds_at(q, slot));
+    p[0] = make_double2(F[q][0], F[q][1]);
+    p[1] = make_double2(F[q][2], F[q + 4][0]);
+    p[2] = make_double2(F[q + 4][1], F[q + 4][2]);
+  }
+}
+// one phase of a node's sums: the bottom corners of its four elements end
+// the sum c of its own plane, their top corners start the sum n of the next
+LDEV void lds_fold(const double *lds, int p00, int p10, int p01, int p11, double &c0, double &c1,
+                   double &c2, double &n0, double &n1, double &n2) {
+  const int at4[4] = {p00, p10, p01, p11};
+  double2 v[4][3];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const double2 *p = (const double2 *)(lds + at4[k]);
+    v[k][0] = p[0]; v[k][1] = p[1]; v[k][2] = p[2];
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    c0 = c0 + v[k][0].x; c1 = c1 + v[k][0].y; c2 = c2 + v[k][1].x;
+    n0 = n0 + v[k][1].y; n1 = n1 + v[k][2].x; n2 = n2 + v[k][2].y;
+  }
+}
+
+// The node planes the element and node lanes of a tile read, kept in LDS:
+// the (etx + 1) x (ety + 1) nodes around its elements, six arrays of
+// `NPATCH` doubles per plane (NODAL_PATCH, or NODAL_PATCH_WIDE for tiles
+// whose patch is larger: one workgroup per CU instead of two).
+// the values of one node array at an element's eight corners: the bottom
+// nodes from plane b, the top ones from plane t of the ring (rows of w)
+LDEV void hex_patch(const double *b, const double *t, int p, int w, double (&out)[8]) {
+  out[0] = b[p]; out[1] = b[p + 1]; out[3] = b[p + w]; out[2] = b[p + w + 1];
+  out[4] = t[p]; out[5] = t[p + 1]; out[7] = t[p + w]; out[6] = t[p + w + 1];
+}
+
+// QK: the quirk bits Q1 | Q2 known at compile time, -1: taken from the batch
+template <int QK, int NPATCH>
 __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
+  // values a thread fetches of the patch nodes past BLOCK
+  constexpr int XV = (6 * (NPATCH - 1 - BLOCK) + BLOCK - 1) / BLOCK;
   // XCD-aware order: the dispatcher deals workgroups round-robin over the 8
   // XCDs, and the host's table gives each XCD a contiguous run of blocks
   // (neighbouring tiles, whose halos then share its L2; -8 % at s=192)
@@ -381,7 +442,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   const InstDesc I = B.inst[inst_];
   DevScalars *sc = B.sc + inst_;
   if (B.gated && !sc->active) return;
-  const int s = I.s, quirks = B.quirks, keep_aux = B.keep_aux;
+  const int s = I.s, quirks = QK < 0 ? B.quirks : QK, keep_aux = B.keep_aux;
   const int etx = I.etx, ety = I.ety;
   const DevFields f = slice(B.f, I);
   const int lb = vb - I.gb0;
@@ -407,13 +468,18 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   const bool node_col = tj < ety && ni < iend && nj < jend;
   // the four elements around the node column, in ascending id order:
   // (ni-1,nj-1) (ni,nj-1) (ni-1,nj) (ni,nj) at lanes (ti+oi-1, tj+oj-1) ..
-  // (ti+oi, tj+oj); each is read only where it exists, which keeps every
-  // read inside the tile (a node column the tile owns has its elements
-  // among the tile's lanes)
+  // (ti+oi, tj+oj); where one does not exist, the slot that holds zeros
+  // stands in for it (a node column the tile owns has its elements among
+  // the tile's lanes).  Adding that zero changes no bit, and every lane's
+  // reads are unconditional: all of a phase's are in flight together
+  // instead of one exec-masked group after the other.
   const bool h00 = ni >= 1 && nj >= 1, h10 = ni < s && nj >= 1;
   const bool h01 = ni >= 1 && nj < s, h11 = ni < s && nj < s;
-  const int l00 = (tj + oj - 1) * etx + (ti + oi - 1), l10 = l00 + 1, l01 = l00 + etx,
-            l11 = l00 + etx + 1;
+  const int l00 = (tj + oj - 1) * etx + (ti + oi - 1);
+  const int p00 = lds_at(2, node_col && h00 ? l00 : BLOCK);
+  const int p10 = lds_at(3, node_col && h10 ? l00 + 1 : BLOCK);
+  const int p01 = lds_at(1, node_col && h01 ? l00 + etx : BLOCK);
+  const int p11 = lds_at(0, node_col && h11 ? l00 + etx + 1 : BLOCK);
   // corner of the node in element (ox,oy) = node offset inside it:
   // (1,1)->2, (0,1)->3, (1,0)->1, (0,0)->0 at the bottom; +4 at the top
 
@@ -423,10 +489,45 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   const bool hg_on = hourg > 0.0;
   const double dt = sc->deltatime, u_cut = sc->u_cut;
 
-  __shared__ double lds[24 * BLOCK];  // [corner][component][element slot]
+  // [corner of the bottom face][element slot, slot BLOCK zero][bottom xyz, top xyz]
+  __shared__ __align__(16) double lds[LDS_PAIR * 4];
+  if (t < 24) lds[lds_at(t / 6, BLOCK) + t % 6] = 0.0;
+  // Two node planes of the tile, [plane & 1][x y z xd yd zd][node]: the
+  // (etx + 1) x (ety + 1) nodes around its elements.  An element takes its
+  // eight nodes from here, so a plane is fetched once per tile (six 8-byte
+  // loads per thread) instead of 24 paired 16-byte gathers per element.
+  __shared__ double ring[2][6][NPATCH];
+  const int pw = etx + 1, np = pw * (ety + 1);
+  const uint32_t us1 = (uint32_t)s1, node_plane = us1 * us1;
+  // What this thread fetches of a plane: the six values of patch node t,
+  // and the values t, t + BLOCK .. of the patch nodes past BLOCK (array by
+  // array), all clamped into the domain
+  const int pa = t < np ? t : np - 1;
+  auto node_of = [&](int p) {
+    const int i = i0 - oi + p % pw, j = j0 - oj + p / pw;
+    return (uint32_t)(j < s ? j : s) * us1 + (uint32_t)(i < s ? i : s);
+  };
+  const uint32_t na = node_of(pa);
+  uint32_t nx[XV];
+  int px[XV];  // where it goes in a plane of the ring, -1: nothing
+  const double *xsrc[XV];
+#pragma unroll
+  for (int k = 0; k < XV; ++k) {
+    const int xn = np - BLOCK, xi = t + k * BLOCK, xc = xn > 0 ? xi / xn : 6;
+    nx[k] = 0;
+    px[k] = -1;
+    xsrc[k] = in.x;
+    if (xc < 6) {
+      const int p = BLOCK + xi % xn;
+      nx[k] = node_of(p);
+      px[k] = xc * NPATCH + p;
+      xsrc[k] = xc == 0 ? in.x : xc == 1 ? in.y : xc == 2 ? in.z : xc == 3 ? in.xd : xc == 4 ? in.yd : in.zd;
+    }
+  }
+  const int pe = tj < ety ? tj * pw + ti : 0;               // the element's first node
+  const int po = tj < ety ? (tj + oj) * pw + ti + oi : 0;   // the own node column
 
   double cs0 = 0.0, cs1 = 0.0, cs2 = 0.0, ch0 = 0.0, ch1 = 0.0, ch2 = 0.0;  // node plane ek
-  double ns0 = 0.0, ns1 = 0.0, ns2 = 0.0, nh0 = 0.0, nh1 = 0.0, nh2 = 0.0;  // node plane ek+1
 
   // Issue order.  A CU holds two k_nodal workgroups, one wave of each per
   // SIMD, and a SIMD issues the older wave first when both are ready, so a
@@ -438,183 +539,165 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   const int lead_end = k0 - 1 + (11 * (k1 - k0 + 1)) / 20;
   if ((int)(blockIdx.x >> 3) >= B.nodal_lead) __builtin_amdgcn_s_setprio(1);
 
-  for (int ek = k0 - 1; ek < k1; ++ek) {
-    const bool plane = ek >= 0 && ek < s;
+  // Element and node addresses are clamped into the domain, so that every
+  // lane loads without a branch; lanes without an element or node column of
+  // their own use none of it.
+  const uint32_t ce = (uint32_t)(ej < s ? ej : s - 1) * (uint32_t)s + (uint32_t)(ei < s ? ei : s - 1);
+  const uint32_t cn = (uint32_t)(nj < s1 ? nj : s) * us1 + (uint32_t)(ni < s1 ? ni : s);
+  const uint32_t elem_plane = (uint32_t)s * (uint32_t)s;
+  // the first element plane; node planes ek0 and ek0 + 1 and the first
+  // plane's element values
+  const int ek0 = k0 > 0 ? k0 - 1 : 0;
+  for (int k = 0; k < 2; ++k) {
+    const uint32_t o = ((uint32_t)(ek0 + k) * node_plane + na) * 8u;
+    double(*r)[NPATCH] = ring[(ek0 + k) & 1];
+    const double a0 = at(in.x, o), a1 = at(in.y, o), a2 = at(in.z, o);
+    const double a3 = at(in.xd, o), a4 = at(in.yd, o), a5 = at(in.zd, o);
+    r[0][pa] = a0; r[1][pa] = a1; r[2][pa] = a2; r[3][pa] = a3; r[4][pa] = a4; r[5][pa] = a5;
+#pragma unroll
+    for (int j = 0; j < XV; ++j)
+      if (px[j] >= 0) (&r[0][0])[px[j]] = xsrc[j][(uint32_t)(ek0 + k) * node_plane + nx[j]];
+  }
+  double vp, vq, vv, vvolo, vss, vem;
+  {
+    const uint32_t eo = ((uint32_t)ek0 * elem_plane + ce) * 8u;
+    vp = at(f.p, eo); vq = at(f.q, eo); vv = at(f.v, eo);
+    vvolo = at(f.volo, eo); vss = at(f.ss, eo); vem = at(f.elemMass, eo);
+  }
+  __syncthreads();
+
+  for (int ek = ek0; ek < k1; ++ek) {
+    const bool plane = ek < s;
     if (ek == lead_end) __builtin_amdgcn_s_setprio(0);
+    // asked for now, used after this plane's arithmetic: node plane ek + 2
+    // (for the next element plane) and the nodal mass of plane ek
+    const bool more = ek + 1 < k1 && ek + 1 < s;
+    double a0, a1, a2, a3, a4, a5, ax[XV];
+    if (more) {
+      const uint32_t o = ((uint32_t)(ek + 2) * node_plane + na) * 8u;
+      a0 = at(in.x, o); a1 = at(in.y, o); a2 = at(in.z, o);
+      a3 = at(in.xd, o); a4 = at(in.yd, o); a5 = at(in.zd, o);
+#pragma unroll
+      for (int j = 0; j < XV; ++j)
+        if (px[j] >= 0) ax[j] = xsrc[j][(uint32_t)(ek + 2) * node_plane + nx[j]];
+    }
+    const uint32_t no = ((uint32_t)ek * node_plane + cn) * 8u;
+    const double mass = at(f.nodalMass, no);
     double hgf[8][3];
     if (plane && elem_col) {
-      const int64_t e = ((int64_t)ek * s + ej) * s + ei;
-      const uint32_t eo = (uint32_t)e * 8u;
-      uint32_t nid[4];
-      hex_pairs(((uint32_t)ek * (uint32_t)s1 + (uint32_t)ej) * (uint32_t)s1 + (uint32_t)ei,
-                (uint32_t)s1, nid);
+      const double(*rb)[NPATCH] = ring[ek & 1], (*rt)[NPATCH] = ring[(ek + 1) & 1];
       double X[8], Y[8], Z[8];
-      gather8p(in.x, nid, X); gather8p(in.y, nid, Y); gather8p(in.z, nid, Z);
+      hex_patch(rb[0], rt[0], pe, pw, X);
+      hex_patch(rb[1], rt[1], pe, pw, Y);
+      hex_patch(rb[2], rt[2], pe, pw, Z);
       // stress corners, src/domain.jl:1097-1108 (sig from 963-969)
-      const double detJ = jacobian_volume(X, Y, Z);
-      if (detJ <= 0.0) raise(sc, ERR_EARLY_VOLUME);
+      if (jacobian_volume64(X, Y, Z) <= 0.0) raise(sc, ERR_EARLY_VOLUME);
       {
         double B[8][3];
-        node_normals(X, Y, Z, quirks, B);
-        const double ms = -((-at(f.p, eo)) - at(f.q, eo));
+        node_normals16(X, Y, Z, quirks, B);
+        const double ms = (-((-vp) - vq)) * 0.0625;
 #pragma unroll
         for (int n = 0; n < 8; ++n)
 #pragma unroll
-          for (int c = 0; c < 3; ++c) lds[(n * 3 + c) * BLOCK + t] = ms * B[n][c];
+          for (int c = 0; c < 3; ++c) B[n][c] = ms * B[n][c];
+        lds_put(lds, t, B);
       }
       // hourglass corners, src/domain.jl:1707-1729 and 1505-1639
-      const double v = at(f.v, eo);
-      const double determ = at(f.volo, eo) * v;
-      if (v <= 0.0) raise(sc, ERR_HG_VOLUME);
+      const double determ = vvolo * vv;
+      if (vv <= 0.0) raise(sc, ERR_HG_VOLUME);
       if (hg_on) {
-        // Mode-major form of the same arithmetic: for each hourglass mode m
-        // the column hourgam[.][m], its three projections h_c[m] and the
-        // running sums sum_m hourgam[n][m] h_c[m] (m = 0..3 in order, as the
-        // reference's 4-term sums fold) -- fewer values live at once.
-        double dvdx[8], dvdy[8], dvdz[8];
-        volume_derivative(X, Y, Z, quirks, dvdx, dvdy, dvdz);
-        double hmx[4], hmy[4], hmz[4];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          double hx = X[0] * gam(0, m), hy = Y[0] * gam(0, m), hz = Z[0] * gam(0, m);
-#pragma unroll
-          for (int n = 1; n < 8; ++n) {
-            hx = hx + X[n] * gam(n, m);
-            hy = hy + Y[n] * gam(n, m);
-            hz = hz + Z[n] * gam(n, m);
-          }
-          hmx[m] = hx; hmy[m] = hy; hmz[m] = hz;
-        }
-        const double volinv = 1.0 / determ;
-        double VX[8], VY[8], VZ[8];
-        gather8p(in.xd, nid, VX); gather8p(in.yd, nid, VY); gather8p(in.zd, nid, VZ);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          double g[8];
-#pragma unroll
-          for (int n = 0; n < 8; ++n)
-            g[n] = gam(n, m) - volinv * (((dvdx[n] * hmx[m]) + (dvdy[n] * hmy[m])) + (dvdz[n] * hmz[m]));
-          double h0 = g[0] * VX[0], h1 = g[0] * VY[0], h2 = g[0] * VZ[0];
-#pragma unroll
-          for (int n = 1; n < 8; ++n) {
-            h0 = h0 + g[n] * VX[n];
-            h1 = h1 + g[n] * VY[n];
-            h2 = h2 + g[n] * VZ[n];
-          }
-#pragma unroll
-          for (int n = 0; n < 8; ++n) {
-            if (m == 0) {
-              hgf[n][0] = g[n] * h0;
-              hgf[n][1] = g[n] * h1;
-              hgf[n][2] = g[n] * h2;
-            } else {
-              hgf[n][0] = hgf[n][0] + g[n] * h0;
-              hgf[n][1] = hgf[n][1] + g[n] * h1;
-              hgf[n][2] = hgf[n][2] + g[n] * h2;
-            }
-          }
-        }
         const double volume13 = cbrt_cr(determ);
-        const double coefficient = ((((-hourg) * 0.01) * at(f.ss, eo)) * at(f.elemMass, eo)) / volume13;
+        const double coefficient = ((((-hourg) * 0.01) * vss) * vem) / volume13;
+        // the 36 edge sums the face normals and the volume derivatives have
+        // in common are formed twice: kept over both, they alone hold 72
+        // registers and the kernel needs 294
+#pragma unroll
+        for (int n = 0; n < 8; ++n) pin3(X[n], Y[n], Z[n]);
+        double hmx[4], hmy[4], hmz[4];
+        hourglass_modes(X, hmx);
+        hourglass_modes(Y, hmy);
+        hourglass_modes(Z, hmz);
+        const double volinv = 1.0 / determ;
+        double g[8][4], h[4][3];
 #pragma unroll
         for (int n = 0; n < 8; ++n) {
-          hgf[n][0] = coefficient * hgf[n][0];
-          hgf[n][1] = coefficient * hgf[n][1];
-          hgf[n][2] = coefficient * hgf[n][2];
+          const int vo = pe + (n == 1 || n == 2 || n == 5 || n == 6 ? 1 : 0) + (n == 2 || n == 3 || n == 6 || n == 7 ? pw : 0);
+          const double(*rv)[NPATCH] = n < 4 ? rb : rt;
+          const double vx = rv[3][vo], vy = rv[4][vo], vz = rv[5][vo];
+          double dx, dy, dz;
+          volume_derivative_node(X, Y, Z, quirks, n, dx, dy, dz);
+#pragma unroll
+          for (int m = 0; m < 4; ++m) {
+            g[n][m] = gam(n, m) - volinv * (((dx * hmx[m]) + (dy * hmy[m])) + (dz * hmz[m]));
+            if (n == 0) {
+              h[m][0] = g[n][m] * vx; h[m][1] = g[n][m] * vy; h[m][2] = g[n][m] * vz;
+            } else {
+              h[m][0] = h[m][0] + g[n][m] * vx;
+              h[m][1] = h[m][1] + g[n][m] * vy;
+              h[m][2] = h[m][2] + g[n][m] * vz;
+            }
+          }
+          pin3(h[0][0], h[1][0], h[2][0]);
         }
+#pragma unroll
+        for (int n = 0; n < 8; ++n)
+#pragma unroll
+          for (int c = 0; c < 3; ++c)
+            hgf[n][c] = coefficient * (((g[n][0] * h[0][c] + g[n][1] * h[1][c]) + g[n][2] * h[2][c]) + g[n][3] * h[3][c]);
       }
     }
     __syncthreads();
     // stress: finish node plane ek with the bottom corners of plane ek, start
     // node plane ek+1 with its top corners (plane ek precedes plane ek+1)
-    if (node_col && plane) {
-      if (ek >= k0) {
-#define LULESH_ACC(flag, slot, corner)                                  \
-  if (flag) {                                                           \
-    cs0 = cs0 + lds[((corner) * 3 + 0) * BLOCK + (slot)];               \
-    cs1 = cs1 + lds[((corner) * 3 + 1) * BLOCK + (slot)];               \
-    cs2 = cs2 + lds[((corner) * 3 + 2) * BLOCK + (slot)];               \
-  }
-        LULESH_ACC(h00, l00, 2) LULESH_ACC(h10, l10, 3) LULESH_ACC(h01, l01, 1)
-        LULESH_ACC(h11, l11, 0)
-#undef LULESH_ACC
-      }
-      if (ek + 1 < k1) {
-#define LULESH_ACC(flag, slot, corner)                                  \
-  if (flag) {                                                           \
-    ns0 = ns0 + lds[((corner) * 3 + 0) * BLOCK + (slot)];               \
-    ns1 = ns1 + lds[((corner) * 3 + 1) * BLOCK + (slot)];               \
-    ns2 = ns2 + lds[((corner) * 3 + 2) * BLOCK + (slot)];               \
-  }
-        LULESH_ACC(h00, l00, 6) LULESH_ACC(h10, l10, 7) LULESH_ACC(h01, l01, 5)
-        LULESH_ACC(h11, l11, 4)
-#undef LULESH_ACC
-      }
+    double ns0 = 0.0, ns1 = 0.0, ns2 = 0.0, nh0 = 0.0, nh1 = 0.0, nh2 = 0.0;
+    if (plane) lds_fold(lds, p00, p10, p01, p11, cs0, cs1, cs2, ns0, ns1, ns2);
+    const double(*ro)[NPATCH] = ring[ek & 1];
+    const double ox = ro[0][po], oy = ro[1][po], oz = ro[2][po];
+    const double oxd = ro[3][po], oyd = ro[4][po], ozd = ro[5][po];
+    __syncthreads();
+    if (hg_on && plane && elem_col) lds_put(lds, t, hgf);
+    // every wave is past its reads of node plane ek: plane ek + 2 takes its
+    // place, and the next plane's element values are asked for
+    if (more) {
+      double(*r)[NPATCH] = ring[ek & 1];
+      r[0][pa] = a0; r[1][pa] = a1; r[2][pa] = a2; r[3][pa] = a3; r[4][pa] = a4; r[5][pa] = a5;
+#pragma unroll
+      for (int j = 0; j < XV; ++j)
+        if (px[j] >= 0) (&r[0][0])[px[j]] = ax[j];
+      const uint32_t eo = ((uint32_t)(ek + 1) * elem_plane + ce) * 8u;
+      vp = at(f.p, eo); vq = at(f.q, eo); vv = at(f.v, eo);
+      vvolo = at(f.volo, eo); vss = at(f.ss, eo); vem = at(f.elemMass, eo);
     }
     __syncthreads();
-    if (hg_on) {
-      if (plane && elem_col) {
-#pragma unroll
-        for (int n = 0; n < 8; ++n)
-#pragma unroll
-          for (int c = 0; c < 3; ++c) lds[(n * 3 + c) * BLOCK + t] = hgf[n][c];
-      }
-      __syncthreads();
-      if (node_col && plane) {
-        if (ek >= k0) {
-#define LULESH_ACC(flag, slot, corner)                                  \
-  if (flag) {                                                           \
-    ch0 = ch0 + lds[((corner) * 3 + 0) * BLOCK + (slot)];               \
-    ch1 = ch1 + lds[((corner) * 3 + 1) * BLOCK + (slot)];               \
-    ch2 = ch2 + lds[((corner) * 3 + 2) * BLOCK + (slot)];               \
-  }
-          LULESH_ACC(h00, l00, 2) LULESH_ACC(h10, l10, 3) LULESH_ACC(h01, l01, 1)
-          LULESH_ACC(h11, l11, 0)
-#undef LULESH_ACC
-        }
-        if (ek + 1 < k1) {
-#define LULESH_ACC(flag, slot, corner)                                  \
-  if (flag) {                                                           \
-    nh0 = nh0 + lds[((corner) * 3 + 0) * BLOCK + (slot)];               \
-    nh1 = nh1 + lds[((corner) * 3 + 1) * BLOCK + (slot)];               \
-    nh2 = nh2 + lds[((corner) * 3 + 2) * BLOCK + (slot)];               \
-  }
-          LULESH_ACC(h00, l00, 6) LULESH_ACC(h10, l10, 7) LULESH_ACC(h01, l01, 5)
-          LULESH_ACC(h11, l11, 4)
-#undef LULESH_ACC
-        }
-      }
-      __syncthreads();
-    }
+    if (hg_on && plane) lds_fold(lds, p00, p10, p01, p11, ch0, ch1, ch2, nh0, nh1, nh2);
+    __syncthreads();
     // node plane ek is complete: calcAccelerationForNodes ..
     // calcPositionForNodes for it
     if (node_col && ek >= k0) {
-      const uint32_t no = (((uint32_t)ek * (uint32_t)s1 + (uint32_t)nj) * (uint32_t)s1 + (uint32_t)ni) * 8u;
       double fx = cs0, fy = cs1, fz = cs2;
       if (hg_on) {
         fx = fx + ch0;
         fy = fy + ch1;
         fz = fz + ch2;
       }
-      const double mass = at(f.nodalMass, no);
       double xdd = fx / mass, ydd = fy / mass, zdd = fz / mass;
       // symmetry planes: the col 0, row 0 and plane 0 node sets
       // (src/domain.jl:773-791, 1787-1806)
       if (ni == 0) xdd = 0.0;
       if (nj == 0) ydd = 0.0;
       if (ek == 0) zdd = 0.0;
-      double xd = at(in.xd, no) + xdd * dt;
+      double xd = oxd + xdd * dt;
       if (fabs(xd) < u_cut) xd = 0.0;
-      double yd = at(in.yd, no) + ydd * dt;
+      double yd = oyd + ydd * dt;
       if (fabs(yd) < u_cut) yd = 0.0;
-      double zd = at(in.zd, no) + zdd * dt;
+      double zd = ozd + zdd * dt;
       if (fabs(zd) < u_cut) zd = 0.0;
       at(out.xd, no) = xd;
       at(out.yd, no) = yd;
       at(out.zd, no) = zd;
-      at(out.x, no) = at(in.x, no) + xd * dt;
-      at(out.y, no) = at(in.y, no) + yd * dt;
-      at(out.z, no) = at(in.z, no) + zd * dt;
+      at(out.x, no) = ox + xd * dt;
+      at(out.y, no) = oy + yd * dt;
+      at(out.z, no) = oz + zd * dt;
       if (keep_aux) {
         at(f.fx, no) = fx; at(f.fy, no) = fy; at(f.fz, no) = fz;
         at(f.xdd, no) = xdd; at(f.ydd, no) = ydd; at(f.zdd, no) = zdd;
@@ -622,7 +705,6 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
     }
     cs0 = ns0; cs1 = ns1; cs2 = ns2;
     ch0 = nh0; ch1 = nh1; ch2 = nh2;
-    ns0 = ns1 = ns2 = nh0 = nh1 = nh2 = 0.0;
   }
   // the instance's last workgroup to finish makes the node set just written
   // current: every workgroup of the instance has then started (and read
@@ -1100,7 +1182,7 @@ static inline unsigned per_inst_grid(int n) { return (unsigned)((n + 63) / 64); 
 
 int nodal_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_nodal, BLOCK, 0) != hipSuccess || n < 1)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_nodal<3, NODAL_PATCH>, BLOCK, 0) != hipSuccess || n < 1)
     n = 1;
   return n;
 }
@@ -1123,7 +1205,14 @@ hipError_t launch_kernel(int id, hipStream_t st, const Batch &b) {
   switch (id) {
     case KID_NODAL:
       // glaunch workgroups, dealt to blocks by the XCD-aware order table
-      hipLaunchKernelGGL(k_nodal, dim3(b.glaunch), dim3(BLOCK), 0, st, b);
+      if (b.nodal_wide)
+        hipLaunchKernelGGL((k_nodal<-1, NODAL_PATCH_WIDE>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
+      else if ((b.quirks & (Q1 | Q2)) == (Q1 | Q2))
+        hipLaunchKernelGGL((k_nodal<Q1 | Q2, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
+      else if ((b.quirks & (Q1 | Q2)) == 0)
+        hipLaunchKernelGGL((k_nodal<0, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
+      else
+        hipLaunchKernelGGL((k_nodal<-1, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
       break;
     case KID_KIN:
       hipLaunchKernelGGL(k_kin, dim3(b.kin_launch), dim3(KIN_CHUNK), 0, st, b);

@@ -51,6 +51,12 @@ inline NodalTile nodal_tile(int s, int lo = 16, int hi = 32) {
   }
   return best;
 }
+// k_nodal keeps the (etx + 1) x (ety + 1) nodes around a tile's elements in
+// LDS; this many fit beside a second workgroup on the CU.  Every tile of the
+// default widths fits (at most 297 nodes); narrower or wider ones up to 387
+// take the kernel's wide form.
+constexpr int NODAL_PATCH = 298, NODAL_PATCH_WIDE = 388;
+inline bool nodal_patch_wide(const NodalTile &t) { return (t.etx + 1) * (t.ety + 1) >= NODAL_PATCH; }
 // z-chunks of a column.  Node plane k takes the corners of element planes
 // k-1 and k, so a chunk marches one element plane more than it owns node
 // planes, except where there is none below (node plane 0) or above (node
