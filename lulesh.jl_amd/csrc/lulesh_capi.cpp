@@ -408,6 +408,11 @@ int plan_nodal(lulesh_ctx *c, int cz) {
     for (int ch = 0; ch < k.chunks; ++ch)
       gplanes.insert(gplanes.end(), I.tx * I.ty, nodal_chunk_planes(k, ch, I.s));
   }
+  // one small domain at the default geometry: a workgroup per node plane
+  c->b.one = c->inst[0];
+  c->b.ptile = plane_tile(c->inst[0].s);
+  c->b.nodal_planes = c->n == 1 && automatic && c->tile_lo == 16 && c->tile_hi == 32 &&
+                      nodal_planes_fit(c->inst[0].s, (int64_t)c->cus * c->nodal_per_cu);
   c->b.gblocks = gb;
   c->gblock_host = std::move(gblock_inst);
   c->gplanes_host = std::move(gplanes);

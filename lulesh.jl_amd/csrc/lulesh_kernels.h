@@ -77,6 +77,9 @@ struct Batch {
   const int *qeos_order;    // k_qeos block run by each launched workgroup, -1: none
   int eblocks, nblocks, gblocks;
   int glaunch;              // k_nodal workgroups launched (a multiple of 8)
+  int nodal_planes;         // one small domain: k_nodal_planes with tile ptile
+  NodalTile ptile;
+  InstDesc one;             // the instance of a batch of one, by value
   int nodal_wide;           // some tile's node patch needs the wide k_nodal (nodal_patch_wide)
   int nodal_lead;           // CUs per XCD: k_nodal workgroups dealt to an XCD
                             // before its CUs hold one each

@@ -428,6 +428,81 @@ LDEV void hex_patch(const double *b, const double *t, int p, int w, double (&out
   out[4] = t[p]; out[5] = t[p + 1]; out[7] = t[p + w]; out[6] = t[p + w + 1];
 }
 
+// The hourglass columns g[n][m] = Gamma[n][m] - (dV/dx_n . projection m) / V
+// and their velocity projections h[m] = sum_n g[n][m] v_n of an element,
+// node by node (src/domain.jl:1516-1600): node n's volume derivative and
+// velocity are used and dropped before the next node's, every sum in the
+// reference's order.
+template <int NPATCH>
+LDEV void hourglass_gh(double (&X)[8], double (&Y)[8], double (&Z)[8], const double (*rb)[NPATCH],
+                       const double (*rt)[NPATCH], int pe, int pw, int quirks, double volinv,
+                       double (&g)[8][4], double (&h)[4][3]) {
+  // the 36 edge sums the face normals and the volume derivatives have in
+  // common are formed twice: kept over both, they alone hold 72 registers
+  // and k_nodal needs 294
+#pragma unroll
+  for (int n = 0; n < 8; ++n) pin3(X[n], Y[n], Z[n]);
+  double hmx[4], hmy[4], hmz[4];
+  hourglass_modes(X, hmx);
+  hourglass_modes(Y, hmy);
+  hourglass_modes(Z, hmz);
+#pragma unroll
+  for (int n = 0; n < 8; ++n) {
+    const bool right = n == 1 || n == 2 || n == 5 || n == 6, back = n == 2 || n == 3 || n == 6 || n == 7;
+    const double(*rv)[NPATCH] = n < 4 ? rb : rt;
+    const int vo = pe + (right ? 1 : 0) + (back ? pw : 0);
+    const double vx = rv[3][vo], vy = rv[4][vo], vz = rv[5][vo];
+    double dx, dy, dz;
+    volume_derivative_node(X, Y, Z, quirks, n, dx, dy, dz);
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+      g[n][m] = gam(n, m) - volinv * (((dx * hmx[m]) + (dy * hmy[m])) + (dz * hmz[m]));
+      if (n == 0) {
+        h[m][0] = g[n][m] * vx; h[m][1] = g[n][m] * vy; h[m][2] = g[n][m] * vz;
+      } else {
+        h[m][0] = h[m][0] + g[n][m] * vx;
+        h[m][1] = h[m][1] + g[n][m] * vy;
+        h[m][2] = h[m][2] + g[n][m] * vz;
+      }
+    }
+    pin3(h[0][0], h[1][0], h[2][0]);
+  }
+}
+LDEV double hourglass_force(const double (&g)[4], const double (&h)[4][3], int c, double coefficient) {
+  return coefficient * (((g[0] * h[0][c] + g[1] * h[1][c]) + g[2] * h[2][c]) + g[3] * h[3][c]);
+}
+// acceleration, symmetry planes, velocity and position of one node
+// (src/domain.jl:1781-1838), written to the other node set
+struct NodeOld {
+  double mass, x, y, z, xd, yd, zd;
+};
+LDEV void node_update(const NodeSet &out, const DevFields &f, uint32_t no, int ni, int nj, int k,
+                      double fx, double fy, double fz, const NodeOld &o, double dt, double u_cut,
+                      int keep_aux) {
+  double xdd = fx / o.mass, ydd = fy / o.mass, zdd = fz / o.mass;
+  // symmetry planes: the col 0, row 0 and plane 0 node sets
+  // (src/domain.jl:773-791, 1787-1806)
+  if (ni == 0) xdd = 0.0;
+  if (nj == 0) ydd = 0.0;
+  if (k == 0) zdd = 0.0;
+  double xd = o.xd + xdd * dt;
+  if (fabs(xd) < u_cut) xd = 0.0;
+  double yd = o.yd + ydd * dt;
+  if (fabs(yd) < u_cut) yd = 0.0;
+  double zd = o.zd + zdd * dt;
+  if (fabs(zd) < u_cut) zd = 0.0;
+  at(out.xd, no) = xd;
+  at(out.yd, no) = yd;
+  at(out.zd, no) = zd;
+  at(out.x, no) = o.x + xd * dt;
+  at(out.y, no) = o.y + yd * dt;
+  at(out.z, no) = o.z + zd * dt;
+  if (keep_aux) {
+    at(f.fx, no) = fx; at(f.fy, no) = fy; at(f.fz, no) = fz;
+    at(f.xdd, no) = xdd; at(f.ydd, no) = ydd; at(f.zdd, no) = zdd;
+  }
+}
+
 // QK: the quirk bits Q1 | Q2 known at compile time, -1: taken from the batch
 template <int QK, int NPATCH>
 __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
@@ -608,42 +683,13 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
       if (hg_on) {
         const double volume13 = cbrt_cr(determ);
         const double coefficient = ((((-hourg) * 0.01) * vss) * vem) / volume13;
-        // the 36 edge sums the face normals and the volume derivatives have
-        // in common are formed twice: kept over both, they alone hold 72
-        // registers and the kernel needs 294
-#pragma unroll
-        for (int n = 0; n < 8; ++n) pin3(X[n], Y[n], Z[n]);
-        double hmx[4], hmy[4], hmz[4];
-        hourglass_modes(X, hmx);
-        hourglass_modes(Y, hmy);
-        hourglass_modes(Z, hmz);
-        const double volinv = 1.0 / determ;
         double g[8][4], h[4][3];
-#pragma unroll
-        for (int n = 0; n < 8; ++n) {
-          const int vo = pe + (n == 1 || n == 2 || n == 5 || n == 6 ? 1 : 0) + (n == 2 || n == 3 || n == 6 || n == 7 ? pw : 0);
-          const double(*rv)[NPATCH] = n < 4 ? rb : rt;
-          const double vx = rv[3][vo], vy = rv[4][vo], vz = rv[5][vo];
-          double dx, dy, dz;
-          volume_derivative_node(X, Y, Z, quirks, n, dx, dy, dz);
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            g[n][m] = gam(n, m) - volinv * (((dx * hmx[m]) + (dy * hmy[m])) + (dz * hmz[m]));
-            if (n == 0) {
-              h[m][0] = g[n][m] * vx; h[m][1] = g[n][m] * vy; h[m][2] = g[n][m] * vz;
-            } else {
-              h[m][0] = h[m][0] + g[n][m] * vx;
-              h[m][1] = h[m][1] + g[n][m] * vy;
-              h[m][2] = h[m][2] + g[n][m] * vz;
-            }
-          }
-          pin3(h[0][0], h[1][0], h[2][0]);
-        }
+        hourglass_gh(X, Y, Z, rb, rt, pe, pw, quirks, 1.0 / determ, g, h);
 #pragma unroll
         for (int n = 0; n < 8; ++n)
 #pragma unroll
           for (int c = 0; c < 3; ++c)
-            hgf[n][c] = coefficient * (((g[n][0] * h[0][c] + g[n][1] * h[1][c]) + g[n][2] * h[2][c]) + g[n][3] * h[3][c]);
+            hgf[n][c] = hourglass_force(g[n], h, c, coefficient);
       }
     }
     __syncthreads();
@@ -680,28 +726,8 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
         fy = fy + ch1;
         fz = fz + ch2;
       }
-      double xdd = fx / mass, ydd = fy / mass, zdd = fz / mass;
-      // symmetry planes: the col 0, row 0 and plane 0 node sets
-      // (src/domain.jl:773-791, 1787-1806)
-      if (ni == 0) xdd = 0.0;
-      if (nj == 0) ydd = 0.0;
-      if (ek == 0) zdd = 0.0;
-      double xd = oxd + xdd * dt;
-      if (fabs(xd) < u_cut) xd = 0.0;
-      double yd = oyd + ydd * dt;
-      if (fabs(yd) < u_cut) yd = 0.0;
-      double zd = ozd + zdd * dt;
-      if (fabs(zd) < u_cut) zd = 0.0;
-      at(out.xd, no) = xd;
-      at(out.yd, no) = yd;
-      at(out.zd, no) = zd;
-      at(out.x, no) = ox + xd * dt;
-      at(out.y, no) = oy + yd * dt;
-      at(out.z, no) = oz + zd * dt;
-      if (keep_aux) {
-        at(f.fx, no) = fx; at(f.fy, no) = fy; at(f.fz, no) = fz;
-        at(f.xdd, no) = xdd; at(f.ydd, no) = ydd; at(f.zdd, no) = zdd;
-      }
+      node_update(out, f, no, ni, nj, ek, fx, fy, fz, NodeOld{mass, ox, oy, oz, oxd, oyd, ozd}, dt,
+                  u_cut, keep_aux);
     }
     cs0 = ns0; cs1 = ns1; cs2 = ns2;
     ch0 = nh0; ch1 = nh1; ch2 = nh2;
@@ -714,6 +740,180 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
     __syncthreads();
     if (t == 0) {
       if (atomicAdd(&sc->nodal_done, 1) == I.gbn - 1) {
+        sc->nodal_done = 0;
+        sc->parity = par ^ 1;
+      }
+    }
+  }
+}
+
+// lagrangeNodal of a single small domain: one node plane per workgroup, the
+// element planes below and above it computed side by side.
+//
+// On a domain that leaves the chip mostly idle a launch of k_nodal lasts as
+// long as one wave's march, at least two element planes one after the other
+// (4.5 us each).  Here a workgroup's first two waves take the plane below
+// the node plane and the other two the plane above, so both take one plane's
+// time; each keeps only the corners that touch the node plane, which leaves
+// room to stage stress and hourglass corners together: one barrier instead
+// of four per plane.  The arithmetic and every sum's order are k_nodal's.
+// It does twice k_nodal's element work per node plane, so it is used only
+// while its workgroups all run at once (nodal_planes_fit).  Event-timed
+// launches: s=8 10.1 us against the march's 17.6, s=16 10.8 against 17.8,
+// s=30 15.3 against 17.9.  Bound by one wave's latency: launch, the loads of
+// the patch, 7,500 cycles of arithmetic, one fold.
+constexpr int PLANE_LANES = BLOCK / 2;  // element lanes per element plane
+template <int QK>
+__global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
+  DevScalars *sc = B.sc;
+  if (B.gated && !sc->active) return;
+  const InstDesc &I = B.one;
+  const DevFields &f = B.f;
+  const int s = I.s, s1 = s + 1, etx = B.ptile.etx, ety = B.ptile.ety;
+  const int tx = blockIdx.x, ty = blockIdx.y, k = blockIdx.z;
+  const int i0 = tx == 0 ? 0 : etx + (tx - 1) * (etx - 1);
+  const int j0 = ty == 0 ? 0 : ety + (ty - 1) * (ety - 1);
+  const int oi = tx != 0, oj = ty != 0;
+  const int iend = tx == B.ptile.tx - 1 ? s + 1 : i0 + etx - oi;
+  const int jend = ty == B.ptile.ty - 1 ? s + 1 : j0 + ety - oj;
+  const int t = threadIdx.x, l = t % PLANE_LANES;
+  const int upper = __builtin_amdgcn_readfirstlane(t / PLANE_LANES);
+  const int ti = l % etx, tj = l / etx;
+  const int ei = i0 - oi + ti, ej = j0 - oj + tj, ek = k - 1 + upper;
+  const bool elem = tj < ety && ei < s && ej < s && ek >= 0 && ek < s;
+  const int ni = i0 + ti, nj = j0 + tj;
+  const bool node = upper && tj < ety && ni < iend && nj < jend;
+
+  const int par = sc->parity;
+  const NodeSet in = pick(f, par), out = pick(f, par ^ 1);
+  const double hourg = sc->hgcoef;
+  const bool hg_on = hourg > 0.0;
+  const double dt = sc->deltatime, u_cut = sc->u_cut;
+
+  // three node planes around k (those outside the domain repeat the edge)
+  __shared__ double patch[3][6][PLANE_PATCH];
+  // [corner mod 4][lane, slot BLOCK zero][stress xyz, hourglass xyz]
+  __shared__ __align__(16) double lds[LDS_PAIR * 4];
+  const int pw = etx + 1, np = pw * (ety + 1);
+  const uint32_t us1 = (uint32_t)s1, node_plane = us1 * us1;
+  double nv[2][6];
+  int at_[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int m = t + j * BLOCK, pl = m / np, p = m % np;
+    at_[j] = pl < 3 ? pl * 6 * PLANE_PATCH + p : -1;
+    const int i = i0 - oi + p % pw, jj = j0 - oj + p / pw;
+    const int kk = k - 1 + pl;
+    const uint32_t o = ((uint32_t)(kk < 0 ? 0 : kk < s ? kk : s) * node_plane +
+                        (uint32_t)(jj < s ? jj : s) * us1 + (uint32_t)(i < s ? i : s)) * 8u;
+    nv[j][0] = at(in.x, o); nv[j][1] = at(in.y, o); nv[j][2] = at(in.z, o);
+    nv[j][3] = at(in.xd, o); nv[j][4] = at(in.yd, o); nv[j][5] = at(in.zd, o);
+  }
+  const uint32_t eo = ((uint32_t)(ek < 0 ? 0 : ek < s ? ek : s - 1) * ((uint32_t)s * (uint32_t)s) +
+                       (uint32_t)(ej < s ? ej : s - 1) * (uint32_t)s + (uint32_t)(ei < s ? ei : s - 1)) * 8u;
+  const double vp = at(f.p, eo), vq = at(f.q, eo), vv = at(f.v, eo);
+  const double vvolo = at(f.volo, eo), vss = at(f.ss, eo), vem = at(f.elemMass, eo);
+  const uint32_t no = ((uint32_t)k * node_plane + (uint32_t)(nj < s1 ? nj : s) * us1 +
+                       (uint32_t)(ni < s1 ? ni : s)) * 8u;
+  const double mass = at(f.nodalMass, no);
+  if (t < 24) lds[lds_at(t / 6, BLOCK) + t % 6] = 0.0;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+    if (at_[j] >= 0) {
+      double *r = &patch[0][0][0] + at_[j];
+#pragma unroll
+      for (int c = 0; c < 6; ++c) r[c * PLANE_PATCH] = nv[j][c];
+    }
+  __syncthreads();
+
+  if (elem) {
+    const double(*rb)[PLANE_PATCH] = patch[upper], (*rt)[PLANE_PATCH] = patch[upper + 1];
+    const int pe = tj * pw + ti;
+    const int quirks = QK;
+    double X[8], Y[8], Z[8];
+    hex_patch(rb[0], rt[0], pe, pw, X);
+    hex_patch(rb[1], rt[1], pe, pw, Y);
+    hex_patch(rb[2], rt[2], pe, pw, Z);
+    if (jacobian_volume64(X, Y, Z) <= 0.0) raise(sc, ERR_EARLY_VOLUME);
+    double2 *p[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) p[q] = (double2 *)(lds + lds_at(q, t));
+    double z[4];
+    {
+      double N[8][3];
+      node_normals16(X, Y, Z, quirks, N);
+      const double ms = (-((-vp) - vq)) * 0.0625;
+      // the corners on the node plane: the top ones of the element below,
+      // the bottom ones of the element above
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const double a = upper ? N[q][0] : N[q + 4][0], b = upper ? N[q][1] : N[q + 4][1];
+        z[q] = ms * (upper ? N[q][2] : N[q + 4][2]);
+        p[q][0] = make_double2(ms * a, ms * b);
+      }
+    }
+    const double determ = vvolo * vv;
+    if (vv <= 0.0) raise(sc, ERR_HG_VOLUME);
+    if (hg_on) {
+      const double volume13 = cbrt_cr(determ);
+      const double coefficient = ((((-hourg) * 0.01) * vss) * vem) / volume13;
+      double g[8][4], h[4][3];
+      hourglass_gh(X, Y, Z, rb, rt, pe, pw, quirks, 1.0 / determ, g, h);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        double gq[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) gq[m] = upper ? g[q][m] : g[q + 4][m];
+        p[q][1] = make_double2(z[q], hourglass_force(gq, h, 0, coefficient));
+        p[q][2] = make_double2(hourglass_force(gq, h, 1, coefficient),
+                               hourglass_force(gq, h, 2, coefficient));
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        p[q][1] = make_double2(z[q], 0.0);
+        p[q][2] = make_double2(0.0, 0.0);
+      }
+    }
+  }
+  __syncthreads();
+  if (node) {
+    // the element plane below, then the one above, each in (row, col) order
+    const int l00 = (tj + oj - 1) * etx + (ti + oi - 1);
+    double cs0 = 0.0, cs1 = 0.0, cs2 = 0.0, ch0 = 0.0, ch1 = 0.0, ch2 = 0.0;
+    double2 v[8][3];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      const int dj = (w >> 1) & 1, di = w & 1, up = w >> 2;
+      const int x = ni - 1 + di, y = nj - 1 + dj, zk = k - 1 + up;
+      const bool there = x >= 0 && x < s && y >= 0 && y < s && zk >= 0 && zk < s;
+      const int q = dj ? (di ? 0 : 1) : (di ? 3 : 2);
+      const double2 *r = (const double2 *)(lds + lds_at(q, there ? up * PLANE_LANES + l00 + dj * etx + di : BLOCK));
+      v[w][0] = r[0]; v[w][1] = r[1]; v[w][2] = r[2];
+    }
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      cs0 = cs0 + v[w][0].x; cs1 = cs1 + v[w][0].y; cs2 = cs2 + v[w][1].x;
+      ch0 = ch0 + v[w][1].y; ch1 = ch1 + v[w][2].x; ch2 = ch2 + v[w][2].y;
+    }
+    if (hg_on) {
+      cs0 = cs0 + ch0;
+      cs1 = cs1 + ch1;
+      cs2 = cs2 + ch2;
+    }
+    const int po = (tj + oj) * pw + ti + oi;
+    node_update(out, f, no, ni, nj, k, cs0, cs1, cs2,
+                NodeOld{mass, patch[1][0][po], patch[1][1][po], patch[1][2][po], patch[1][3][po],
+                        patch[1][4][po], patch[1][5][po]},
+                dt, u_cut, B.keep_aux);
+  }
+  // as in k_nodal: the last workgroup to finish makes the set just written
+  // current
+  if (B.flip) {
+    __syncthreads();
+    if (t == 0) {
+      const int last = (int)(gridDim.x * gridDim.y * gridDim.z) - 1;
+      if (atomicAdd(&sc->nodal_done, 1) == last) {
         sc->nodal_done = 0;
         sc->parity = par ^ 1;
       }
@@ -1205,14 +1405,24 @@ hipError_t launch_kernel(int id, hipStream_t st, const Batch &b) {
   switch (id) {
     case KID_NODAL:
       // glaunch workgroups, dealt to blocks by the XCD-aware order table
-      if (b.nodal_wide)
+      if (b.nodal_planes) {
+        const dim3 g(b.ptile.tx, b.ptile.ty, b.one.s + 1);
+        switch (b.quirks & (Q1 | Q2)) {
+          case 0: hipLaunchKernelGGL(k_nodal_planes<0>, g, dim3(BLOCK), 0, st, b); break;
+          case Q1: hipLaunchKernelGGL(k_nodal_planes<Q1>, g, dim3(BLOCK), 0, st, b); break;
+          case Q2: hipLaunchKernelGGL(k_nodal_planes<Q2>, g, dim3(BLOCK), 0, st, b); break;
+          default: hipLaunchKernelGGL((k_nodal_planes<Q1 | Q2>), g, dim3(BLOCK), 0, st, b); break;
+        }
+      } else if (b.nodal_wide) {
         hipLaunchKernelGGL((k_nodal<-1, NODAL_PATCH_WIDE>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
-      else if ((b.quirks & (Q1 | Q2)) == (Q1 | Q2))
-        hipLaunchKernelGGL((k_nodal<Q1 | Q2, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
-      else if ((b.quirks & (Q1 | Q2)) == 0)
-        hipLaunchKernelGGL((k_nodal<0, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
-      else
-        hipLaunchKernelGGL((k_nodal<-1, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
+      } else {
+        switch (b.quirks & (Q1 | Q2)) {
+          case 0: hipLaunchKernelGGL((k_nodal<0, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
+          case Q1: hipLaunchKernelGGL((k_nodal<Q1, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
+          case Q2: hipLaunchKernelGGL((k_nodal<Q2, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
+          default: hipLaunchKernelGGL((k_nodal<Q1 | Q2, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
+        }
+      }
       break;
     case KID_KIN:
       hipLaunchKernelGGL(k_kin, dim3(b.kin_launch), dim3(KIN_CHUNK), 0, st, b);

@@ -232,6 +232,9 @@ int run(const lulesh_device_domain *dom, double *scalars, hipStream_t st, int de
   B.nblocks = I.nbn;
   B.gblocks = c.gb;
   B.glaunch = c.glaunch;
+  B.one = I;
+  B.ptile = plane_tile(nx);
+  B.nodal_planes = nodal_planes_fit(nx, (int64_t)d.cus * d.nodal_per_cu);
   B.nodal_wide = nodal_patch_wide(c.tile) ? 1 : 0;
   B.nodal_lead = d.cus / 8 > 1 ? d.cus / 8 : 1;
   B.sc = (DevScalars *)(base + c.off_sc);

@@ -57,6 +57,28 @@ inline NodalTile nodal_tile(int s, int lo = 16, int hi = 32) {
 // take the kernel's wide form.
 constexpr int NODAL_PATCH = 298, NODAL_PATCH_WIDE = 388;
 inline bool nodal_patch_wide(const NodalTile &t) { return (t.etx + 1) * (t.ety + 1) >= NODAL_PATCH; }
+// k_nodal_planes, the form for one small domain: a workgroup per tile and
+// node plane, half its threads for the element plane below and half for the
+// one above, so a tile has at most BLOCK / 2 element lanes (8 to 16 wide)
+// and its patch at most 153 nodes, three planes of which the workgroup's
+// threads fetch in two passes.
+constexpr int PLANE_PATCH = 154;
+inline NodalTile plane_tile(int s) {
+  NodalTile best{0, 0, 0, 0};
+  for (int a = 8; a <= 16; ++a) {
+    const int b = BLOCK / 2 / a;
+    const int tx = nodal_span(s, a), ty = nodal_span(s, b);
+    if (best.etx == 0 || tx * ty < best.tx * best.ty) best = NodalTile{a, b, tx, ty};
+  }
+  return best;
+}
+// Whether it is the faster form: all its workgroups resident at once.  On
+// 512 slots that is s <= 34 (420 workgroups, 16.2 us a launch against the
+// march's 18.9); at s=36 (555) it takes 20.5 us against 18.7.
+inline bool nodal_planes_fit(int s, int64_t slots) {
+  const NodalTile t = plane_tile(s);
+  return (int64_t)t.tx * t.ty * (s + 1) <= slots;
+}
 // z-chunks of a column.  Node plane k takes the corners of element planes
 // k-1 and k, so a chunk marches one element plane more than it owns node
 // planes, except where there is none below (node plane 0) or above (node
