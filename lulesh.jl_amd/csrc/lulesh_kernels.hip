@@ -379,10 +379,10 @@ __global__ void k_run_begin(Batch B) {
 // plane), the element values and nodal mass asked for a phase ahead, and
 // LDS reads without branches.  Timestamps inside the kernel at s=192: 19,000
 // cycles per plane for the workgroup issued first before, 12,500 now.  At
-// s=192 a launch takes 496 us against 615 (27 TFLOP/s of the 1,430 additions
-// and products per element and plane), the batch of 64 domains 403 against
-// 500, s=63 36 against 39.  243 VGPRs and 78 KB of LDS: two workgroups per
-// CU by either.
+// s=192 a launch takes 487 us against 615 (26 TFLOP/s with the 1,430
+// additions and products per element and plane, halo included), the batch of
+// 64 domains 396 against 500, s=63 36 against 39.  252 VGPRs and 78 KB of
+// LDS: two workgroups per CU by either.
 // ---------------------------------------------------------------------------
 // Corner forces in LDS: [corner q of the bottom face][element slot][x y z of
 // corner q, x y z of corner q + 4 above it], so that a node takes what one
@@ -421,6 +421,11 @@ LDEV void lds_fold(const double *lds, int p00, int p10, int p01, int p11, double
 // the (etx + 1) x (ety + 1) nodes around its elements, six arrays of
 // `NPATCH` doubles per plane (NODAL_PATCH, or NODAL_PATCH_WIDE for tiles
 // whose patch is larger: one workgroup per CU instead of two).
+// an LDS read the compiler neither moves past pinned values nor merges
+LDEV double lds_read(const double *p) {
+  typedef __attribute__((address_space(3))) const volatile double lds_double;
+  return *(lds_double *)p;
+}
 // the values of one node array at an element's eight corners: the bottom
 // nodes from plane b, the top ones from plane t of the ring (rows of w)
 LDEV void hex_patch(const double *b, const double *t, int p, int w, double (&out)[8]) {
@@ -446,12 +451,24 @@ LDEV void hourglass_gh(double (&X)[8], double (&Y)[8], double (&Z)[8], const dou
   hourglass_modes(X, hmx);
   hourglass_modes(Y, hmy);
   hourglass_modes(Z, hmz);
-#pragma unroll
-  for (int n = 0; n < 8; ++n) {
+  // node n + 1's velocity is asked for before node n's arithmetic (a
+  // volatile read stays on its side of the statements that pin values), and
+  // one wait per node leaves the run of FP64 instructions aligned: k_nodal
+  // at s=192 501 -> 487 us
+  double v[2][3];
+  auto velocity = [&](int n) {
     const bool right = n == 1 || n == 2 || n == 5 || n == 6, back = n == 2 || n == 3 || n == 6 || n == 7;
     const double(*rv)[NPATCH] = n < 4 ? rb : rt;
     const int vo = pe + (right ? 1 : 0) + (back ? pw : 0);
-    const double vx = rv[3][vo], vy = rv[4][vo], vz = rv[5][vo];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) v[n & 1][c] = lds_read(&rv[3 + c][vo]);
+  };
+  velocity(0);
+#pragma unroll
+  for (int n = 0; n < 8; ++n) {
+    double &vx = v[n & 1][0], &vy = v[n & 1][1], &vz = v[n & 1][2];
+    pin3(vx, vy, vz);
+    if (n < 7) velocity(n + 1);
     double dx, dy, dz;
     volume_derivative_node(X, Y, Z, quirks, n, dx, dy, dz);
 #pragma unroll
