@@ -29,6 +29,9 @@ struct DevScalars {
   int parity;           // which NodeSet holds the current x..zd
   int nodal_done;       // k_nodal workgroups of this instance finished in the
                         // running launch (the last one flips parity, resets it)
+  int dt_pending;       // the last cycle's end (constraints, loop test, next dt)
+                        // is still to be taken (defer_dt)
+  int err_nodal[2];     // under defer_dt, what the nodal launch of each parity raised
 };
 
 // node positions and velocities; two sets, ping-ponged by the fused nodal
@@ -92,6 +95,8 @@ struct Batch {
   int gated;                // kernels skip instances whose active flag is 0
   int keep_aux;             // also write fx.., xdd.., dxx.., ql, qq
   int loop_mode;            // k_dt: 1 driver-loop test and next dt, 2 next dt always
+  int defer_dt;             // the nodal kernel takes the previous cycle's end, k_dt only
+                            // what is still pending
   int flip;                 // k_nodal makes the node set it wrote current
   double *dt_record;        // k_time_increment (k_dt in loop_mode 2) stores each instance-0 dt here
   int64_t dt_base;          // ... at index cycle - 1 - dt_base (if non-null)

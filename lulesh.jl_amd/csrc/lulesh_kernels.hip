@@ -79,7 +79,8 @@ LDEV T &at(T *base, uint32_t boff) {
   return *(T *)((char *)base + boff);
 }
 
-LDEV void raise(DevScalars *sc, int code) { atomicMin(&sc->err, code); }
+LDEV void raise(int *err, int code) { atomicMin(err, code); }
+LDEV void raise(DevScalars *sc, int code) { raise(&sc->err, code); }
 
 // Stores of k_kin's and k_qeos' outputs that do not keep their lines in the
 // caches: the next kernel reads them back from memory anyway, and with the
@@ -172,28 +173,140 @@ static_assert(KIN_CHUNK == 64, "k_kin workgroups are one wave");
   const int64_t n = (int64_t)(blockIdx.x - I.nb0) * BLOCK + threadIdx.x;       \
   const DevFields f = slice((B).f, I);
 
-// timeIncrement!, src/domain.jl:920-961
-LDEV void time_increment(DevScalars *sc) {
-  double targetdt = sc->stoptime - sc->time;
-  if (sc->dtfixed <= 0.0 && sc->cycle != 0) {
-    const double olddt = sc->deltatime;
+// timeIncrement!, src/domain.jl:920-961, from given time constraints
+struct TimeStep {
+  double time, deltatime;
+  long long cycle;
+};
+LDEV TimeStep next_time_step(const DevScalars &S, double dtcourant, double dthydro) {
+  TimeStep r{S.time, S.deltatime, S.cycle};
+  double targetdt = S.stoptime - r.time;
+  if (S.dtfixed <= 0.0 && r.cycle != 0) {
+    const double olddt = r.deltatime;
     double gnewdt = __builtin_huge_val();
-    if (sc->dtcourant < gnewdt) gnewdt = sc->dtcourant / 2.0;
-    if (sc->dthydro < gnewdt) gnewdt = (sc->dthydro * 2.0) / 3.0;
+    if (dtcourant < gnewdt) gnewdt = dtcourant / 2.0;
+    if (dthydro < gnewdt) gnewdt = (dthydro * 2.0) / 3.0;
     double newdt = gnewdt;
     const double ratio = newdt / olddt;
     if (ratio >= 1.0) {
-      if (ratio < sc->deltatimemultlb) newdt = olddt;
-      else if (ratio > sc->deltatimemultub) newdt = olddt * sc->deltatimemultub;
+      if (ratio < S.deltatimemultlb) newdt = olddt;
+      else if (ratio > S.deltatimemultub) newdt = olddt * S.deltatimemultub;
     }
-    newdt = jmin(newdt, sc->dtmax);
-    sc->deltatime = newdt;
+    newdt = jmin(newdt, S.dtmax);
+    r.deltatime = newdt;
   }
-  if (sc->deltatime < targetdt && targetdt < (4.0 * sc->deltatime) / 3.0)
-    targetdt = (2.0 * sc->deltatime) / 3.0;
-  if (targetdt < sc->deltatime) sc->deltatime = targetdt;
-  sc->time = sc->time + sc->deltatime;
-  sc->cycle = sc->cycle + 1;
+  if (r.deltatime < targetdt && targetdt < (4.0 * r.deltatime) / 3.0)
+    targetdt = (2.0 * r.deltatime) / 3.0;
+  if (targetdt < r.deltatime) r.deltatime = targetdt;
+  r.time = r.time + r.deltatime;
+  r.cycle = r.cycle + 1;
+  return r;
+}
+LDEV void store(DevScalars *sc, const TimeStep &ts) {
+  sc->time = ts.time;
+  sc->deltatime = ts.deltatime;
+  sc->cycle = ts.cycle;
+}
+LDEV void time_increment(DevScalars *sc) {
+  store(sc, next_time_step(*sc, sc->dtcourant, sc->dthydro));
+}
+// the driver loop's test (examples/benchmark.jl:82,95)
+LDEV bool loop_goes_on(const DevScalars *sc, int err) {
+  return err == ERR_NONE && sc->cycle < sc->num_iters && sc->time < sc->stoptime;
+}
+// The error code the loop test sees when a nodal launch makes it: what that
+// launch itself raises goes to err_nodal[parity] (a workgroup that starts
+// late must not take it for the previous cycle's), what the previous one
+// raised is in err_nodal[parity ^ 1].
+LDEV int previous_err(const DevScalars *sc, int par) {
+  const int e = par ? sc->err_nodal[0] : sc->err_nodal[1];
+  return e < sc->err ? e : sc->err;
+}
+LDEV void gather_errs(DevScalars *sc) {
+  int e = sc->err;
+  e = sc->err_nodal[0] < e ? sc->err_nodal[0] : e;
+  e = sc->err_nodal[1] < e ? sc->err_nodal[1] : e;
+  sc->err = e;
+  sc->err_nodal[0] = sc->err_nodal[1] = ERR_NONE;
+}
+
+// The end of the previous cycle of the driver loop, taken at the head of the
+// next one (B.defer_dt: one domain whose partial minima are few).  k_dt on
+// its own is a launch of one workgroup, 4-5 us of a small domain's cycle of
+// 29 with the gap before it; here every workgroup of the nodal launch folds the partial minima for
+// itself, beside its own first loads, and the last one to finish stores the
+// scalars (all the others have read the old ones by then).  A cycle of the
+// device loop at s=16 takes 28.6 -> 26.2 us, s=48 54.1 -> 51.3, s=64 70.4 ->
+// 67.9, s=96 142.3 -> 141.7.  Each wave's minimum goes through LDS and a
+// barrier the kernel has anyway (dt_fold_wave, then dt_fold_take).
+struct DtFold {
+  double courant, hydro;
+};
+LDEV DtFold dt_fold_load(const Batch &B, int ebn) {
+  const double2 *__restrict__ p = (const double2 *)B.dtpart;
+  double a = 1.0e+20, b = 1.0e+20;
+  for (int i = threadIdx.x; i < ebn; i += BLOCK) {
+    const double2 v = p[i];
+    a = v.x < a ? v.x : a;
+    b = v.y < b ? v.y : b;
+  }
+  return DtFold{a, b};
+}
+LDEV void dt_fold_wave(DtFold d, double (*m)[2]) {
+  double a = d.courant, b = d.hydro;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const double oa = __shfl_xor(a, off, 64), ob = __shfl_xor(b, off, 64);
+    a = oa < a ? oa : a;
+    b = ob < b ? ob : b;
+  }
+  if ((threadIdx.x & 63) == 0) {
+    m[threadIdx.x >> 6][0] = a;
+    m[threadIdx.x >> 6][1] = b;
+  }
+}
+LDEV DtFold dt_fold_take(const DevScalars &S, const double (*m)[2]) {
+  double a = m[0][0], b = m[0][1];
+#pragma unroll
+  for (int w = 1; w < BLOCK / 64; ++w) {
+    a = m[w][0] < a ? m[w][0] : a;
+    b = m[w][1] < b ? m[w][1] : b;
+  }
+  return DtFold{a < 1.0e+20 ? a : S.dtcourant, b < 1.0e+20 ? b : S.dthydro};
+}
+// what the last workgroup to finish stores
+struct DtNow {
+  DtFold d;
+  TimeStep ts;
+};
+// what a nodal workgroup that defers keeps of it in LDS
+struct DtShared {
+  double m[BLOCK / 64][2];
+  DtNow now;
+};
+LDEV DtShared &dt_shared() {
+  __shared__ DtShared d;
+  return d;
+}
+LDEV DtNow dt_now_of(const DevScalars &S, bool fold, const double (*m)[2]) {
+  if (!fold) return DtNow{DtFold{S.dtcourant, S.dthydro}, TimeStep{S.time, S.deltatime, S.cycle}};
+  const DtFold d = dt_fold_take(S, m);
+  return DtNow{d, next_time_step(S, d.courant, d.hydro)};
+}
+// A nodal workgroup of a loop that has ended: the constraints are folded all
+// the same, and the last workgroup stores them.
+LDEV void dt_fold_end(DevScalars *sc, int last, double (*m)[2], const Batch &B, int ebn) {
+  dt_fold_wave(dt_fold_load(B, ebn), m);
+  __syncthreads();
+  if (threadIdx.x == 0 && atomicAdd(&sc->nodal_done, 1) == last) {
+    const DtFold d = dt_fold_take(*sc, m);
+    sc->nodal_done = 0;
+    sc->dtcourant = d.courant;
+    sc->dthydro = d.hydro;
+    gather_errs(sc);
+    sc->active = 0;
+    sc->dt_pending = 0;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -321,6 +434,8 @@ __global__ void k_init_scalars(Batch B) {
   sc->num_iters = 0;
   sc->parity = 0;
   sc->nodal_done = 0;
+  sc->dt_pending = 0;
+  sc->err_nodal[0] = sc->err_nodal[1] = ERR_NONE;
 }
 
 // ---------------------------------------------------------------------------
@@ -342,6 +457,8 @@ __global__ void k_run_begin(Batch B) {
   DevScalars *sc = B.sc + i;
   sc->num_iters = B.num_iters;
   sc->err = ERR_NONE;
+  sc->err_nodal[0] = sc->err_nodal[1] = ERR_NONE;
+  sc->dt_pending = 0;
   const int go = sc->time < sc->stoptime;
   sc->active = go;
   if (go) time_increment(sc);
@@ -520,8 +637,24 @@ LDEV void node_update(const NodeSet &out, const DevFields &f, uint32_t no, int n
   }
 }
 
+// The instance's last workgroup to finish makes the node set just written
+// current: every workgroup of the instance has then started (and read the
+// old parity and scalars), and the next kernel sees the new ones (a kernel
+// boundary orders the stores; no fence is needed inside a launch).
+LDEV void nodal_finish(const Batch &B, DevScalars *sc, int par, const DtNow *now) {
+  if (now) {
+    sc->dtcourant = now->d.courant;
+    sc->dthydro = now->d.hydro;
+    store(sc, now->ts);
+    sc->dt_pending = 1;
+  }
+  sc->nodal_done = 0;
+  sc->parity = par ^ 1;
+}
+
 // QK: the quirk bits Q1 | Q2 known at compile time, -1: taken from the batch
-template <int QK, int NPATCH>
+// DEFER: one domain whose previous cycle's end is taken here (B.defer_dt)
+template <int QK, int NPATCH, bool DEFER>
 __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   // values a thread fetches of the patch nodes past BLOCK
   constexpr int XV = (6 * (NPATCH - 1 - BLOCK) + BLOCK - 1) / BLOCK;
@@ -530,8 +663,8 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   // (neighbouring tiles, whose halos then share its L2; -8 % at s=192)
   const int vb = B.gblock_order[blockIdx.x];
   if (vb < 0) return;
-  const int inst_ = B.gblock_inst[vb];
-  const InstDesc I = B.inst[inst_];
+  const int inst_ = DEFER ? 0 : B.gblock_inst[vb];
+  const InstDesc I = DEFER ? B.one : B.inst[inst_];
   DevScalars *sc = B.sc + inst_;
   if (B.gated && !sc->active) return;
   const int s = I.s, quirks = QK < 0 ? B.quirks : QK, keep_aux = B.keep_aux;
@@ -579,7 +712,22 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   const NodeSet in = pick(f, par), out = pick(f, par ^ 1);
   const double hourg = sc->hgcoef;
   const bool hg_on = hourg > 0.0;
-  const double dt = sc->deltatime, u_cut = sc->u_cut;
+  const double u_cut = sc->u_cut;
+  const double dt = sc->deltatime;
+  int *const err = DEFER ? &sc->err_nodal[par] : &sc->err;
+  [[maybe_unused]] DevScalars S;
+  [[maybe_unused]] bool fold = false;
+  if constexpr (DEFER) {
+    S = *sc;
+    fold = S.dt_pending;
+    if (fold) {
+      if (!loop_goes_on(sc, previous_err(sc, par))) {
+        dt_fold_end(sc, I.gbn - 1, dt_shared().m, B, I.ebn);
+        return;
+      }
+      dt_fold_wave(dt_fold_load(B, I.ebn), dt_shared().m);
+    }
+  }
 
   // [corner of the bottom face][element slot, slot BLOCK zero][bottom xyz, top xyz]
   __shared__ __align__(16) double lds[LDS_PAIR * 4];
@@ -657,6 +805,11 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
     vvolo = at(f.volo, eo); vss = at(f.ss, eo); vem = at(f.elemMass, eo);
   }
   __syncthreads();
+  // (read in the first plane's node update, several barriers from here)
+  if constexpr (DEFER) {
+    const DtNow w = dt_now_of(S, fold, dt_shared().m);
+    if (t == 0) dt_shared().now = w;
+  }
 
   for (int ek = ek0; ek < k1; ++ek) {
     const bool plane = ek < s;
@@ -683,7 +836,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
       hex_patch(rb[1], rt[1], pe, pw, Y);
       hex_patch(rb[2], rt[2], pe, pw, Z);
       // stress corners, src/domain.jl:1097-1108 (sig from 963-969)
-      if (jacobian_volume64(X, Y, Z) <= 0.0) raise(sc, ERR_EARLY_VOLUME);
+      if (jacobian_volume64(X, Y, Z) <= 0.0) raise(err, ERR_EARLY_VOLUME);
       {
         double B[8][3];
         node_normals16(X, Y, Z, quirks, B);
@@ -696,7 +849,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
       }
       // hourglass corners, src/domain.jl:1707-1729 and 1505-1639
       const double determ = vvolo * vv;
-      if (vv <= 0.0) raise(sc, ERR_HG_VOLUME);
+      if (vv <= 0.0) raise(err, ERR_HG_VOLUME);
       if (hg_on) {
         const double volume13 = cbrt_cr(determ);
         const double coefficient = ((((-hourg) * 0.01) * vss) * vem) / volume13;
@@ -743,22 +896,21 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
         fy = fy + ch1;
         fz = fz + ch2;
       }
-      node_update(out, f, no, ni, nj, ek, fx, fy, fz, NodeOld{mass, ox, oy, oz, oxd, oyd, ozd}, dt,
+      double step = dt;
+      if constexpr (DEFER) step = dt_shared().now.ts.deltatime;
+      node_update(out, f, no, ni, nj, ek, fx, fy, fz, NodeOld{mass, ox, oy, oz, oxd, oyd, ozd}, step,
                   u_cut, keep_aux);
     }
     cs0 = ns0; cs1 = ns1; cs2 = ns2;
     ch0 = nh0; ch1 = nh1; ch2 = nh2;
   }
-  // the instance's last workgroup to finish makes the node set just written
-  // current: every workgroup of the instance has then started (and read
-  // the old parity), and the next kernel sees the new one (a kernel
-  // boundary orders the stores; no fence is needed inside this launch)
   if (B.flip) {
     __syncthreads();
     if (t == 0) {
       if (atomicAdd(&sc->nodal_done, 1) == I.gbn - 1) {
-        sc->nodal_done = 0;
-        sc->parity = par ^ 1;
+        const DtNow *now = nullptr;
+        if constexpr (DEFER) now = &dt_shared().now;
+        nodal_finish(B, sc, par, now);
       }
     }
   }
@@ -805,7 +957,20 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
   const NodeSet in = pick(f, par), out = pick(f, par ^ 1);
   const double hourg = sc->hgcoef;
   const bool hg_on = hourg > 0.0;
-  const double dt = sc->deltatime, u_cut = sc->u_cut;
+  const double u_cut = sc->u_cut;
+  const int last = (int)(gridDim.x * gridDim.y * gridDim.z) - 1;
+  DtShared &dts = dt_shared();
+  const bool fold = B.defer_dt && sc->dt_pending;
+  int *const err = B.defer_dt ? &sc->err_nodal[par] : &sc->err;
+  const DevScalars S = *sc;
+  DtFold mine{1.0e+20, 1.0e+20};
+  if (fold) {
+    if (!loop_goes_on(sc, previous_err(sc, par))) {
+      dt_fold_end(sc, last, dts.m, B, I.ebn);
+      return;
+    }
+    mine = dt_fold_load(B, I.ebn);
+  }
 
   // three node planes around k (those outside the domain repeat the edge)
   __shared__ double patch[3][6][PLANE_PATCH];
@@ -834,6 +999,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
                        (uint32_t)(ni < s1 ? ni : s)) * 8u;
   const double mass = at(f.nodalMass, no);
   if (t < 24) lds[lds_at(t / 6, BLOCK) + t % 6] = 0.0;
+  if (fold) dt_fold_wave(mine, dts.m);
 #pragma unroll
   for (int j = 0; j < 2; ++j)
     if (at_[j] >= 0) {
@@ -842,6 +1008,10 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
       for (int c = 0; c < 6; ++c) r[c * PLANE_PATCH] = nv[j][c];
     }
   __syncthreads();
+  if (B.defer_dt) {
+    const DtNow w = dt_now_of(S, fold, dts.m);
+    if (t == 0) dts.now = w;
+  }
 
   if (elem) {
     const double(*rb)[PLANE_PATCH] = patch[upper], (*rt)[PLANE_PATCH] = patch[upper + 1];
@@ -851,7 +1021,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
     hex_patch(rb[0], rt[0], pe, pw, X);
     hex_patch(rb[1], rt[1], pe, pw, Y);
     hex_patch(rb[2], rt[2], pe, pw, Z);
-    if (jacobian_volume64(X, Y, Z) <= 0.0) raise(sc, ERR_EARLY_VOLUME);
+    if (jacobian_volume64(X, Y, Z) <= 0.0) raise(err, ERR_EARLY_VOLUME);
     double2 *p[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) p[q] = (double2 *)(lds + lds_at(q, t));
@@ -870,7 +1040,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
       }
     }
     const double determ = vvolo * vv;
-    if (vv <= 0.0) raise(sc, ERR_HG_VOLUME);
+    if (vv <= 0.0) raise(err, ERR_HG_VOLUME);
     if (hg_on) {
       const double volume13 = cbrt_cr(determ);
       const double coefficient = ((((-hourg) * 0.01) * vss) * vem) / volume13;
@@ -922,18 +1092,14 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
     node_update(out, f, no, ni, nj, k, cs0, cs1, cs2,
                 NodeOld{mass, patch[1][0][po], patch[1][1][po], patch[1][2][po], patch[1][3][po],
                         patch[1][4][po], patch[1][5][po]},
-                dt, u_cut, B.keep_aux);
+                B.defer_dt ? dts.now.ts.deltatime : S.deltatime, u_cut, B.keep_aux);
   }
   // as in k_nodal: the last workgroup to finish makes the set just written
   // current
   if (B.flip) {
     __syncthreads();
     if (t == 0) {
-      const int last = (int)(gridDim.x * gridDim.y * gridDim.z) - 1;
-      if (atomicAdd(&sc->nodal_done, 1) == last) {
-        sc->nodal_done = 0;
-        sc->parity = par ^ 1;
-      }
+      if (atomicAdd(&sc->nodal_done, 1) == last) nodal_finish(B, sc, par, B.defer_dt ? &dts.now : nullptr);
     }
   }
 }
@@ -1320,6 +1486,7 @@ __global__ __launch_bounds__(1024) void k_dt(Batch B) {
   const InstDesc I = B.inst[blockIdx.x];
   DevScalars *sc = B.sc + blockIdx.x;
   if (B.gated && !sc->active) return;
+  if (B.defer_dt && !sc->dt_pending) return;
   const int loop_mode = B.loop_mode;
   // (courant, hydro) pairs, 16-byte aligned; four independent loads in
   // flight per thread (a minimum does not depend on the order it is taken in)
@@ -1365,8 +1532,10 @@ __global__ __launch_bounds__(1024) void k_dt(Batch B) {
   if (a < 1.0e+20) sc->dtcourant = a;
   if (b < 1.0e+20) sc->dthydro = b;
   if (loop_mode == 1) {
-    const int go = (sc->err == ERR_NONE) && (sc->cycle < sc->num_iters) && (sc->time < sc->stoptime);
+    if (B.defer_dt) gather_errs(sc);
+    const bool go = loop_goes_on(sc, sc->err);
     sc->active = go;
+    sc->dt_pending = 0;
     if (go) time_increment(sc);
   } else if (loop_mode == 2) {
     time_increment(sc);
@@ -1399,7 +1568,7 @@ static inline unsigned per_inst_grid(int n) { return (unsigned)((n + 63) / 64); 
 
 int nodal_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_nodal<3, NODAL_PATCH>, BLOCK, 0) != hipSuccess || n < 1)
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_nodal<3, NODAL_PATCH, false>, BLOCK, 0) != hipSuccess || n < 1)
     n = 1;
   return n;
 }
@@ -1418,6 +1587,17 @@ hipError_t launch_math(hipStream_t st, int op, const double *a, const double *b,
   return hipGetLastError();
 }
 
+template <bool DEFER>
+static void launch_nodal(hipStream_t st, const Batch &b) {
+  const dim3 g(b.glaunch), w(BLOCK);
+  switch (b.quirks & (Q1 | Q2)) {
+    case 0: hipLaunchKernelGGL((k_nodal<0, NODAL_PATCH, DEFER>), g, w, 0, st, b); break;
+    case Q1: hipLaunchKernelGGL((k_nodal<Q1, NODAL_PATCH, DEFER>), g, w, 0, st, b); break;
+    case Q2: hipLaunchKernelGGL((k_nodal<Q2, NODAL_PATCH, DEFER>), g, w, 0, st, b); break;
+    default: hipLaunchKernelGGL((k_nodal<Q1 | Q2, NODAL_PATCH, DEFER>), g, w, 0, st, b); break;
+  }
+}
+
 hipError_t launch_kernel(int id, hipStream_t st, const Batch &b) {
   switch (id) {
     case KID_NODAL:
@@ -1431,14 +1611,11 @@ hipError_t launch_kernel(int id, hipStream_t st, const Batch &b) {
           default: hipLaunchKernelGGL((k_nodal_planes<Q1 | Q2>), g, dim3(BLOCK), 0, st, b); break;
         }
       } else if (b.nodal_wide) {
-        hipLaunchKernelGGL((k_nodal<-1, NODAL_PATCH_WIDE>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
+        hipLaunchKernelGGL((k_nodal<-1, NODAL_PATCH_WIDE, false>), dim3(b.glaunch), dim3(BLOCK), 0, st, b);
+      } else if (b.defer_dt) {
+        launch_nodal<true>(st, b);
       } else {
-        switch (b.quirks & (Q1 | Q2)) {
-          case 0: hipLaunchKernelGGL((k_nodal<0, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
-          case Q1: hipLaunchKernelGGL((k_nodal<Q1, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
-          case Q2: hipLaunchKernelGGL((k_nodal<Q2, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
-          default: hipLaunchKernelGGL((k_nodal<Q1 | Q2, NODAL_PATCH>), dim3(b.glaunch), dim3(BLOCK), 0, st, b); break;
-        }
+        launch_nodal<false>(st, b);
       }
       break;
     case KID_KIN:

@@ -167,6 +167,8 @@ bool set_scalars(DevScalars &S, const double *v) {
   S.active = 0;
   S.parity = 0;
   S.nodal_done = 0;
+  S.dt_pending = 0;
+  S.err_nodal[0] = S.err_nodal[1] = ERR_NONE;
   return true;
 }
 
@@ -261,6 +263,7 @@ int run(const lulesh_device_domain *dom, double *scalars, hipStream_t st, int de
   B.gated = 0;
   B.keep_aux = 0;
   B.loop_mode = 0;
+  B.defer_dt = 0;
   B.flip = 1;
   B.dt_record = nullptr;
   B.dt_base = 0;
