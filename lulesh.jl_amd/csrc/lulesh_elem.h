@@ -42,10 +42,6 @@ LDEV double jmin(double x, double y) {
   bool takey = (y < x) || (signbit(y) > signbit(x));
   return takey ? (isnan(x) ? x : y) : (isnan(y) ? y : x);
 }
-LDEV double jmax(double x, double y) {
-  bool takey = (y > x) || (signbit(y) < signbit(x));
-  return takey ? (isnan(x) ? x : y) : (isnan(y) ? y : x);
-}
 
 // correctly rounded cube root: cbrt_cr (lulesh_cbrt.h)
 
@@ -80,58 +76,42 @@ LDEV double elem_volume(const double (&x)[8], const double (&y)[8], const double
 }
 
 // ---------------------------------------------------------------------------
-// calcElemShapeFunctionDerivatives, src/domain.jl:1932-2021.  Only the four
-// independent rows of b are produced (rows 5..8 are their negations and no
-// caller needs them); returns the Jacobian volume.
+// calcElemShapeFunctionDerivatives, src/domain.jl:1932-2021.  Powers of two
+// factor out of every product and sum exactly, so the .125 of each
+// derivative is left out here and in what is formed from them.
 // ---------------------------------------------------------------------------
-struct Jac {
-  double fjxxi, fjxet, fjxze, fjyxi, fjyet, fjyze, fjzxi, fjzet, fjzze;
-};
-LDEV Jac jacobian(const double (&x)[8], const double (&y)[8], const double (&z)[8]) {
-  Jac j;
-  j.fjxxi = .125 * ((((x[6] - x[0]) + (x[5] - x[3])) - (x[7] - x[1])) - (x[4] - x[2]));
-  j.fjxet = .125 * ((((x[6] - x[0]) - (x[5] - x[3])) + (x[7] - x[1])) - (x[4] - x[2]));
-  j.fjxze = .125 * ((((x[6] - x[0]) + (x[5] - x[3])) + (x[7] - x[1])) + (x[4] - x[2]));
-  j.fjyxi = .125 * ((((y[6] - y[0]) + (y[5] - y[3])) - (y[7] - y[1])) - (y[4] - y[2]));
-  j.fjyet = .125 * ((((y[6] - y[0]) - (y[5] - y[3])) + (y[7] - y[1])) - (y[4] - y[2]));
-  j.fjyze = .125 * ((((y[6] - y[0]) + (y[5] - y[3])) + (y[7] - y[1])) + (y[4] - y[2]));
-  j.fjzxi = .125 * ((((z[6] - z[0]) + (z[5] - z[3])) - (z[7] - z[1])) - (z[4] - z[2]));
-  j.fjzet = .125 * ((((z[6] - z[0]) - (z[5] - z[3])) + (z[7] - z[1])) - (z[4] - z[2]));
-  j.fjzze = .125 * ((((z[6] - z[0]) + (z[5] - z[3])) + (z[7] - z[1])) + (z[4] - z[2]));
-  return j;
-}
-// 64 x the Jacobian volume: the stress integration keeps only its sign, and
-// powers of two factor out of every product and sum exactly, so the .125 of
-// each derivative is left out
-LDEV double jacobian_volume64(const double (&x)[8], const double (&y)[8], const double (&z)[8]) {
 #define LULESH_J(v, xi, et, ze)                                                     \
   const double v##60 = v[6] - v[0], v##53 = v[5] - v[3], v##71 = v[7] - v[1],       \
                v##42 = v[4] - v[2];                                                 \
   const double xi = ((v##60 + v##53) - v##71) - v##42,                              \
                et = ((v##60 - v##53) + v##71) - v##42,                              \
                ze = ((v##60 + v##53) + v##71) + v##42
+// 64 x the Jacobian volume: the stress integration keeps only its sign
+LDEV double jacobian_volume64(const double (&x)[8], const double (&y)[8], const double (&z)[8]) {
   LULESH_J(x, xxi, xet, xze);
   LULESH_J(y, yxi, yet, yze);
   LULESH_J(z, zxi, zet, zze);
-#undef LULESH_J
   const double cx = (zxi * yze) - (yxi * zze);
   const double cy = (xxi * zze) - (zxi * xze);
   const double cz = (yxi * xze) - (xxi * yze);
   return ((xet * cx) + (yet * cy)) + (zet * cz);
 }
-// b[n][c] for n = 0..3 and the volume
-LDEV double shape_derivatives4(const double (&x)[8], const double (&y)[8], const double (&z)[8],
-                               double (&b)[4][3]) {
-  const Jac j = jacobian(x, y, z);
-  const double cjxxi = (j.fjyet * j.fjzze) - (j.fjzet * j.fjyze);
-  const double cjxet = -(j.fjyxi * j.fjzze) + (j.fjzxi * j.fjyze);
-  const double cjxze = (j.fjyxi * j.fjzet) - (j.fjzxi * j.fjyet);
-  const double cjyxi = -(j.fjxet * j.fjzze) + (j.fjzet * j.fjxze);
-  const double cjyet = (j.fjxxi * j.fjzze) - (j.fjzxi * j.fjxze);
-  const double cjyze = -(j.fjxxi * j.fjzet) + (j.fjzxi * j.fjxet);
-  const double cjzxi = (j.fjxet * j.fjyze) - (j.fjyet * j.fjxze);
-  const double cjzet = -(j.fjxxi * j.fjyze) + (j.fjyxi * j.fjxze);
-  const double cjzze = (j.fjxxi * j.fjyet) - (j.fjyxi * j.fjxet);
+// 64 b[n][c] for n = 0..3 (rows 5..8 are their negations and no caller needs
+// them); returns 64 x the Jacobian volume
+LDEV double shape_derivatives4_64(const double (&x)[8], const double (&y)[8], const double (&z)[8],
+                                  double (&b)[4][3]) {
+  LULESH_J(x, xxi, xet, xze);
+  LULESH_J(y, yxi, yet, yze);
+  LULESH_J(z, zxi, zet, zze);
+  const double cjxxi = (yet * zze) - (zet * yze);
+  const double cjxet = -(yxi * zze) + (zxi * yze);
+  const double cjxze = (yxi * zet) - (zxi * yet);
+  const double cjyxi = -(xet * zze) + (zet * xze);
+  const double cjyet = (xxi * zze) - (zxi * xze);
+  const double cjyze = -(xxi * zet) + (zxi * xet);
+  const double cjzxi = (xet * yze) - (yet * xze);
+  const double cjzet = -(xxi * yze) + (yxi * xze);
+  const double cjzze = (xxi * yet) - (yxi * xet);
   b[0][0] = ((-cjxxi) - cjxet) - cjxze;
   b[1][0] = (cjxxi - cjxet) - cjxze;
   b[2][0] = (cjxxi + cjxet) - cjxze;
@@ -144,8 +124,9 @@ LDEV double shape_derivatives4(const double (&x)[8], const double (&y)[8], const
   b[1][2] = (cjzxi - cjzet) - cjzze;
   b[2][2] = (cjzxi + cjzet) - cjzze;
   b[3][2] = ((-cjzxi) + cjzet) - cjzze;
-  return 8.0 * (((j.fjxet * cjxet) + (j.fjyet * cjyet)) + (j.fjzet * cjzet));
+  return ((xet * cjxet) + (yet * cjyet)) + (zet * cjzet);
 }
+#undef LULESH_J
 
 // ---------------------------------------------------------------------------
 // sumElemFaceNormal (src/domain.jl:971-989) and calcElemNodeNormals
@@ -280,19 +261,24 @@ LDEV double area_face(double x0, double x1, double x2, double x3, double y0, dou
   return ((((fx * fx) + (fy * fy)) + (fz * fz)) * (((gx * gx) + (gy * gy)) + (gz * gz))) -
          (fg * fg);
 }
+// The reference's chain of Julia max from 0.0 is the largest of the six and
+// 0, or NaN if one of them is: one v_max_f64 each and three tests for NaN
+// instead of a dozen selects per link.
 LDEV double char_length(const double (&x)[8], const double (&y)[8], const double (&z)[8],
                         double volume) {
-  double cl = 0.0;
 #define LULESH_AF(a, b, c, d) \
-  cl = jmax(area_face(x[a], x[b], x[c], x[d], y[a], y[b], y[c], y[d], z[a], z[b], z[c], z[d]), cl)
-  LULESH_AF(0, 1, 2, 3);
-  LULESH_AF(4, 5, 6, 7);
-  LULESH_AF(0, 1, 5, 4);
-  LULESH_AF(1, 2, 6, 5);
-  LULESH_AF(2, 3, 7, 6);
-  LULESH_AF(3, 0, 4, 7);
+  area_face(x[a], x[b], x[c], x[d], y[a], y[b], y[c], y[d], z[a], z[b], z[c], z[d])
+  const double a0 = LULESH_AF(0, 1, 2, 3), a1 = LULESH_AF(4, 5, 6, 7);
+  double cl = __builtin_fmax(0.0, __builtin_fmax(a0, a1));
+  bool nan = __builtin_isunordered(a0, a1);
+  const double a2 = LULESH_AF(0, 1, 5, 4), a3 = LULESH_AF(1, 2, 6, 5);
+  cl = __builtin_fmax(cl, __builtin_fmax(a2, a3));
+  nan = nan || __builtin_isunordered(a2, a3);
+  const double a4 = LULESH_AF(2, 3, 7, 6), a5 = LULESH_AF(3, 0, 4, 7);
+  cl = __builtin_fmax(cl, __builtin_fmax(a4, a5));
+  nan = nan || __builtin_isunordered(a4, a5);
 #undef LULESH_AF
-  return (4.0 * volume) / sqrt(cl);
+  return nan ? __builtin_nan("") : (4.0 * volume) / sqrt(cl);
 }
 
 // diagonal of calcElemVelocityGradient (src/domain.jl:2023-2043); the

@@ -1106,6 +1106,13 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
 
 // calcKinematicsForElems (src/domain.jl:2099-2147), the deviatoric loop
 // (2156-2171) and calcMonotonicQGradientsForElems (2175-2320)
+//
+// Bound by its memory pattern (the same 24 gathers, 2 reads and 10 writes
+// alone take 240 us at s=192) and the vector instructions beside it.  Without
+// the power-of-two scalings and the select chains of Julia's max: s=192 281
+// -> 270 us, batch 209 -> 202, s=96 34.0 -> 32.0.  Fetching a 256-element
+// chunk's node rows once into LDS instead (10 loads per thread and plane, one
+// barrier) takes 320 us: the loads no longer run under other waves' work.
 __global__ __launch_bounds__(KIN_CHUNK) void k_kin(Batch B) {
   // the chunk of one element plane this workgroup runs: kin_table bands
   // the planes so that an XCD's consecutive chunks climb one band of the
@@ -1149,7 +1156,8 @@ __global__ __launch_bounds__(KIN_CHUNK) void k_kin(Batch B) {
       YS[n] = Y[n] - dt2 * YV[n];
       ZS[n] = Z[n] - dt2 * ZV[n];
     }
-    const double detJ = shape_derivatives4(XS, YS, ZS, b);
+    // (64 x detJ and 64 x b: the factors cancel exactly)
+    const double detJ = shape_derivatives4_64(XS, YS, ZS, b);
     const double inv_detJ = 1.0 / detJ;
     const double d1 = inv_detJ * vgrad_term(b, 0, XV);
     const double d2 = inv_detJ * vgrad_term(b, 1, YV);
@@ -1168,46 +1176,33 @@ __global__ __launch_bounds__(KIN_CHUNK) void k_kin(Batch B) {
   const double ptiny = 1.e-36;
   const double vol = volo * vnew;
   const double norm = 1.0 / (vol + ptiny);
-  const double dxj = -0.25 * (sum4(X[0], X[1], X[5], X[4]) - sum4(X[3], X[2], X[6], X[7]));
-  const double dyj = -0.25 * (sum4(Y[0], Y[1], Y[5], Y[4]) - sum4(Y[3], Y[2], Y[6], Y[7]));
-  const double dzj = -0.25 * (sum4(Z[0], Z[1], Z[5], Z[4]) - sum4(Z[3], Z[2], Z[6], Z[7]));
-  const double dxi = 0.25 * (sum4(X[1], X[2], X[6], X[5]) - sum4(X[0], X[3], X[7], X[4]));
-  const double dyi = 0.25 * (sum4(Y[1], Y[2], Y[6], Y[5]) - sum4(Y[0], Y[3], Y[7], Y[4]));
-  const double dzi = 0.25 * (sum4(Z[1], Z[2], Z[6], Z[5]) - sum4(Z[0], Z[3], Z[7], Z[4]));
-  const double dxk = 0.25 * (sum4(X[4], X[5], X[6], X[7]) - sum4(X[0], X[1], X[2], X[3]));
-  const double dyk = 0.25 * (sum4(Y[4], Y[5], Y[6], Y[7]) - sum4(Y[0], Y[1], Y[2], Y[3]));
-  const double dzk = 0.25 * (sum4(Z[4], Z[5], Z[6], Z[7]) - sum4(Z[0], Z[1], Z[2], Z[3]));
-  double ax, ay, az, dxv, dyv, dzv;
-  // zeta: i cross j
-  ax = (dyi * dzj) - (dzi * dyj);
-  ay = (dzi * dxj) - (dxi * dzj);
-  az = (dxi * dyj) - (dyi * dxj);
-  st_nt(f.delx_zeta, eo, vol / sqrt((((ax * ax) + (ay * ay)) + (az * az)) + ptiny));
-  ax = ax * norm; ay = ay * norm; az = az * norm;
-  dxv = 0.25 * (sum4(XV[4], XV[5], XV[6], XV[7]) - sum4(XV[0], XV[1], XV[2], XV[3]));
-  dyv = 0.25 * (sum4(YV[4], YV[5], YV[6], YV[7]) - sum4(YV[0], YV[1], YV[2], YV[3]));
-  dzv = 0.25 * (sum4(ZV[4], ZV[5], ZV[6], ZV[7]) - sum4(ZV[0], ZV[1], ZV[2], ZV[3]));
-  st_nt(f.delv_zeta, eo, ((ax * dxv) + (ay * dyv)) + (az * dzv));
-  // xi: j cross k
-  ax = (dyj * dzk) - (dzj * dyk);
-  ay = (dzj * dxk) - (dxj * dzk);
-  az = (dxj * dyk) - (dyj * dxk);
-  st_nt(f.delx_xi, eo, vol / sqrt((((ax * ax) + (ay * ay)) + (az * az)) + ptiny));
-  ax = ax * norm; ay = ay * norm; az = az * norm;
-  dxv = 0.25 * (sum4(XV[1], XV[2], XV[6], XV[5]) - sum4(XV[0], XV[3], XV[7], XV[4]));
-  dyv = 0.25 * (sum4(YV[1], YV[2], YV[6], YV[5]) - sum4(YV[0], YV[3], YV[7], YV[4]));
-  dzv = 0.25 * (sum4(ZV[1], ZV[2], ZV[6], ZV[5]) - sum4(ZV[0], ZV[3], ZV[7], ZV[4]));
-  st_nt(f.delv_xi, eo, ((ax * dxv) + (ay * dyv)) + (az * dzv));
-  // eta: k cross i
-  ax = (dyk * dzi) - (dzk * dyi);
-  ay = (dzk * dxi) - (dxk * dzi);
-  az = (dxk * dyi) - (dyk * dxi);
-  st_nt(f.delx_eta, eo, vol / sqrt((((ax * ax) + (ay * ay)) + (az * az)) + ptiny));
-  ax = ax * norm; ay = ay * norm; az = az * norm;
-  dxv = -0.25 * (sum4(XV[0], XV[1], XV[5], XV[4]) - sum4(XV[3], XV[2], XV[6], XV[7]));
-  dyv = -0.25 * (sum4(YV[0], YV[1], YV[5], YV[4]) - sum4(YV[3], YV[2], YV[6], YV[7]));
-  dzv = -0.25 * (sum4(ZV[0], ZV[1], ZV[5], ZV[4]) - sum4(ZV[3], ZV[2], ZV[6], ZV[7]));
-  st_nt(f.delv_eta, eo, ((ax * dxv) + (ay * dyv)) + (az * dzv));
+  // Four times the reference's side differences d' = 4 d: powers of two
+  // factor out exactly, so an area vector is a' = 16 a, sqrt(a.a + ptiny) =
+  // sqrt(a'.a' + 256 ptiny) / 16, and a.dv norm = a'.dv' (norm / 64).
+  const double ptiny256 = 256.0 * 1.e-36, norm64 = norm * 0.015625, vol16 = vol * 16.0;
+#define LULESH_SIDE(v, a, b, c, d, e, f, g, h) (sum4(v[a], v[b], v[c], v[d]) - sum4(v[e], v[f], v[g], v[h]))
+#define LULESH_ETA(v) (-LULESH_SIDE(v, 0, 1, 5, 4, 3, 2, 6, 7))
+#define LULESH_XI(v) LULESH_SIDE(v, 1, 2, 6, 5, 0, 3, 7, 4)
+#define LULESH_ZETA(v) LULESH_SIDE(v, 4, 5, 6, 7, 0, 1, 2, 3)
+  const double dxj = LULESH_ETA(X), dyj = LULESH_ETA(Y), dzj = LULESH_ETA(Z);
+  const double dxi = LULESH_XI(X), dyi = LULESH_XI(Y), dzi = LULESH_XI(Z);
+  const double dxk = LULESH_ZETA(X), dyk = LULESH_ZETA(Y), dzk = LULESH_ZETA(Z);
+  auto gradient = [&](double ux, double uy, double uz, double wx, double wy, double wz, double dvx,
+                      double dvy, double dvz, double *delx, double *delv) {
+    const double ax = (uy * wz) - (uz * wy);
+    const double ay = (uz * wx) - (ux * wz);
+    const double az = (ux * wy) - (uy * wx);
+    st_nt(delx, eo, vol16 / sqrt((((ax * ax) + (ay * ay)) + (az * az)) + ptiny256));
+    st_nt(delv, eo, (((ax * norm64) * dvx) + ((ay * norm64) * dvy)) + ((az * norm64) * dvz));
+  };
+  // zeta: i cross j, xi: j cross k, eta: k cross i
+  gradient(dxi, dyi, dzi, dxj, dyj, dzj, LULESH_ZETA(XV), LULESH_ZETA(YV), LULESH_ZETA(ZV), f.delx_zeta, f.delv_zeta);
+  gradient(dxj, dyj, dzj, dxk, dyk, dzk, LULESH_XI(XV), LULESH_XI(YV), LULESH_XI(ZV), f.delx_xi, f.delv_xi);
+  gradient(dxk, dyk, dzk, dxi, dyi, dzi, LULESH_ETA(XV), LULESH_ETA(YV), LULESH_ETA(ZV), f.delx_eta, f.delv_eta);
+#undef LULESH_SIDE
+#undef LULESH_ETA
+#undef LULESH_XI
+#undef LULESH_ZETA
 }
 
 // neighbour ids exactly as setupElementConnectivities stores them
