@@ -94,7 +94,8 @@ __global__ __launch_bounds__(BLOCK) void a_qeos(AdjArgs A) {
     for (int sd = 0; sd < 2; ++sd) {
       src[d][sd] = bc_source(bc, d, sd);
       tgt[d][sd] = read_target(d, sd, e, A.s, A.E, A.q3);
-      const double val = src[d][sd] == 0 ? dvs[d][tgt[d][sd]] : (src[d][sd] == 1 ? qi.dv[d] : 0.0);
+      const double there = dvs[d][tgt[d][sd]];  // (read before the mask is known)
+      const double val = src[d][sd] == 0 ? there : (src[d][sd] == 1 ? qi.dv[d] : 0.0);
       if (sd == 0) qi.dm[d] = val;
       else qi.dp[d] = val;
     }
@@ -166,76 +167,96 @@ __global__ __launch_bounds__(BLOCK) void a_kin(AdjArgs A) {
   if (e >= A.E) return;
   const DevFields &f = A.f;
   const NodeSet S = A.cur;
-  // own delv adjoint plus what the elements that read this delv sent back
+  // Own delv adjoint plus what the elements that read this delv sent back:
+  // by read_target, the next element's minus read (and element 0's, which
+  // reads element 1), the last element's plus read under quirk Q3 or the
+  // previous element's without it, and along eta and zeta the neighbour's
+  // minus and plus reads (the last eta row's plus reads wrap to the first).
+  // With a branch per candidate and 48 eight-byte node loads a launch took
+  // 10.2 us at s=24 and 13.7 at s=48, now 7.1 and 12.4.
+  const uint32_t ue = (uint32_t)e, us = (uint32_t)A.s, s2 = us * us, uE = (uint32_t)A.E;
+  const uint32_t eo = ue * 8u;
   double l6[6];
-  for (int d = 0; d < 3; ++d) {
-    double acc = A.ldvs[(int64_t)d * A.E + e];
-    for (int sd = 0; sd < 2; ++sd) {
-      const double *nb = A.nbr + (int64_t)(d * 2 + sd) * A.E;
-      // readers of e are among these candidates; each is checked exactly
-      const int64_t s = A.s, s2 = (int64_t)A.s * A.s, E = A.E;
-      const int64_t step = d == 0 ? 1 : (d == 1 ? s : s2);
-      const int64_t cand[5] = {e - step, e + step, d == 1 ? e + (E - s) : -1,
-                               d == 0 && e == 1 ? 0 : -1, d == 0 && e == E - 2 ? E - 1 : -1};
-      for (int k = 0; k < 5; ++k) {
-        const int64_t i = cand[k];
-        if (i < 0 || i >= E || i == e) continue;
-        bool dup = false;
-        for (int k2 = 0; k2 < k; ++k2) dup = dup || cand[k2] == i;
-        if (dup) continue;
-        if (read_target(d, sd, i, s, E, A.q3) == e) acc += nb[i];
-      }
-    }
-    l6[3 + d] = acc;
-    l6[d] = A.ldx[(int64_t)d * A.E + e];
+  {
+    auto sent = [&](int q, bool there, uint32_t i) {
+      const double x = at(A.nbr + (int64_t)q * A.E, there ? i * 8u : 0u);
+      return there ? x : 0.0;
+    };
+    const double own[3] = {at(A.ldvs, eo), at(A.ldvs + A.E, eo), at(A.ldvs + 2 * A.E, eo)};
+    const double x0 = sent(0, ue == 1u, 0u), x1 = sent(0, ue + 1u < uE, ue + 1u);
+    const double x2 = A.q3 ? sent(1, ue + 2u == uE, uE - 1u) : sent(1, ue >= 1u, ue - 1u);
+    const double y0 = sent(2, ue + us < uE, ue + us);
+    const bool wraps = ue < us && uE > us;
+    const double y1 = sent(3, ue >= us || wraps, ue >= us ? ue - us : ue + (uE - us));
+    const double z0 = sent(4, ue + s2 < uE, ue + s2), z1 = sent(5, ue >= s2, ue - s2);
+    l6[0] = at(A.ldx, eo); l6[1] = at(A.ldx + A.E, eo); l6[2] = at(A.ldx + 2 * A.E, eo);
+    l6[3] = ((own[0] + x0) + x1) + x2;
+    l6[4] = (own[1] + y0) + y1;
+    l6[5] = (own[2] + z0) + z1;
   }
-  int64_t nid[8];
-  elem_nodes_a(e, A.s, nid);
   double X[8], Y[8], Z[8], VX[8], VY[8], VZ[8];
-  for (int n = 0; n < 8; ++n) {
-    X[n] = S.x[nid[n]]; Y[n] = S.y[nid[n]]; Z[n] = S.z[nid[n]];
-    VX[n] = S.xd[nid[n]]; VY[n] = S.yd[nid[n]]; VZ[n] = S.zd[nid[n]];
+  {
+    const uint32_t s1 = us + 1u, col = ue % us, rest = ue / us;
+    uint32_t nid[4];
+    hex_pairs(((rest / us) * s1 + rest % us) * s1 + col, s1, nid);
+    gather8p(S.x, nid, X); gather8p(S.y, nid, Y); gather8p(S.z, nid, Z);
+    gather8p(S.xd, nid, VX); gather8p(S.yd, nid, VY); gather8p(S.zd, nid, VZ);
   }
   double lX[8] = {0}, lY[8] = {0}, lZ[8] = {0}, lVX[8] = {0}, lVY[8] = {0}, lVZ[8] = {0};
-  const double volo = f.volo[e];
-  double lvnew = A.lvnew[e] + A.lvnew_delv[e];  // delv = vnew - v
-  lvnew += lulesh_adj::monoq_grad_rev(X, Y, Z, VX, VY, VZ, volo, f.vnew[e], l6, lX, lY, lZ, lVX,
+  const double volo = at(f.volo, eo);
+  double lvnew = at(A.lvnew, eo) + at(A.lvnew_delv, eo);  // delv = vnew - v
+  lvnew += lulesh_adj::monoq_grad_rev(X, Y, Z, VX, VY, VZ, volo, at(f.vnew, eo), l6, lX, lY, lZ, lVX,
                                       lVY, lVZ);
   lulesh_adj::volume_grad_rev(X, Y, Z, lvnew / volo, lX, lY, lZ);
   double *cr = A.corner;
+#pragma unroll
   for (int n = 0; n < 8; ++n) {
-    cr[(int64_t)(0 * 8 + n) * A.E + e] = lX[n];
-    cr[(int64_t)(1 * 8 + n) * A.E + e] = lY[n];
-    cr[(int64_t)(2 * 8 + n) * A.E + e] = lZ[n];
-    cr[(int64_t)(3 * 8 + n) * A.E + e] = lVX[n];
-    cr[(int64_t)(4 * 8 + n) * A.E + e] = lVY[n];
-    cr[(int64_t)(5 * 8 + n) * A.E + e] = lVZ[n];
+    at(cr + (int64_t)(0 * 8 + n) * A.E, eo) = lX[n];
+    at(cr + (int64_t)(1 * 8 + n) * A.E, eo) = lY[n];
+    at(cr + (int64_t)(2 * 8 + n) * A.E, eo) = lZ[n];
+    at(cr + (int64_t)(3 * 8 + n) * A.E, eo) = lVX[n];
+    at(cr + (int64_t)(4 * 8 + n) * A.E, eo) = lVY[n];
+    at(cr + (int64_t)(5 * 8 + n) * A.E, eo) = lVZ[n];
   }
 }
 
 // corner of element (ei,ej,ek) that node (i,j,k) occupies
 LDEV int corner_of_a(int ox, int oy, int oz) { return 4 * oz + (oy ? (ox ? 2 : 3) : (ox ? 1 : 0)); }
 
-// sum over the node's corners of comp c (0..5) of the corner buffer
-LDEV void gather_corners(const AdjArgs &A, const double *corner, int64_t n, double out[6]) {
-  const int s = A.s;
-  const int64_t s1 = s + 1;
-  const int i = (int)(n % s1), j = (int)((n / s1) % s1), k = (int)(n / (s1 * s1));
-  for (int c = 0; c < 6; ++c) out[c] = 0.0;
-  for (int dk = -1; dk <= 0; ++dk) {
-    const int ek = k + dk;
-    if (ek < 0 || ek >= s) continue;
-    for (int dj = -1; dj <= 0; ++dj) {
-      const int ej = j + dj;
-      if (ej < 0 || ej >= s) continue;
-      for (int di = -1; di <= 0; ++di) {
-        const int ei = i + di;
-        if (ei < 0 || ei >= s) continue;
-        const int64_t e = ((int64_t)ek * s + ej) * s + ei;
-        const int cn = corner_of_a(-di, -dj, -dk);
-        for (int c = 0; c < 6; ++c) out[c] += corner[(int64_t)(c * 8 + cn) * A.E + e];
-      }
+// The eight elements around node (i, j, k), in ascending order: byte offset
+// of each in an element array and whether it exists (a missing one reads
+// element 0 and adds zero).
+struct NodeElems {
+  uint32_t off[8];
+  bool has[8];
+  LDEV NodeElems(int i, int j, int k, int s) {
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      const int ei = i - 1 + (w & 1), ej = j - 1 + ((w >> 1) & 1), ek = k - 1 + (w >> 2);
+      has[w] = ei >= 0 && ei < s && ej >= 0 && ej < s && ek >= 0 && ek < s;
+      off[w] = has[w] ? (((uint32_t)ek * (uint32_t)s + (uint32_t)ej) * (uint32_t)s + (uint32_t)ei) * 8u : 0u;
     }
+  }
+};
+// Sum over a node's corners of comp c (0..5) of a corner buffer.  The reads
+// are unconditional, sixteen in flight together: with a branch per element
+// a_node1 waited for sixteen groups of six one after the other, 8.0 us a
+// launch at s=24 against 5.9 now.  From s=48 on (18.7 us) what bounds it is
+// the 96 values per element it reads back, at 5 TB/s.
+LDEV void gather_corners(const AdjArgs &A, const double *corner, const NodeElems &ne, double out[6]) {
+#pragma unroll 2
+  for (int c = 0; c < 6; ++c) {
+    const double *p = corner + (int64_t)(c * 8) * A.E;
+    double v[8];
+#pragma unroll
+    for (int w = 0; w < 8; ++w) {
+      const int cn = corner_of_a(1 - (w & 1), 1 - ((w >> 1) & 1), 1 - (w >> 2));
+      v[w] = at(p + (int64_t)cn * A.E, ne.off[w]);
+    }
+    double sum = 0.0;
+#pragma unroll
+    for (int w = 0; w < 8; ++w) sum += ne.has[w] ? v[w] : 0.0;
+    out[c] = sum;
   }
 }
 
@@ -243,17 +264,18 @@ LDEV void gather_corners(const AdjArgs &A, const double *corner, int64_t n, doub
 __global__ __launch_bounds__(BLOCK) void a_node1(AdjArgs A) {
   const int64_t n = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (n >= A.N) return;
+  const int s1 = A.s + 1, un = (int)n;
+  const int i = un % s1, j = (un / s1) % s1, k = un / (s1 * s1);
+  const NodeElems ne(i, j, k, A.s);
   double g[6];
   if (A.force_pending) {
     // what a_node2 of the later cycle would add: corner_f into the node state
-    gather_corners(A, A.corner_f, n, g);
+    gather_corners(A, A.corner_f, ne, g);
     A.lx[n] += g[0]; A.ly[n] += g[1]; A.lz[n] += g[2];
     A.lxd[n] += g[3]; A.lyd[n] += g[4]; A.lzd[n] += g[5];
   }
-  gather_corners(A, A.corner, n, g);
+  gather_corners(A, A.corner, ne, g);
   const double dt = A.dt;
-  const int64_t s1 = A.s + 1;
-  const int i = (int)(n % s1), j = (int)((n / s1) % s1), k = (int)(n / (s1 * s1));
   const double mass = A.f.nodalMass[n];
   double *lxs[3] = {A.lx, A.ly, A.lz};
   double *lvs[3] = {A.lxd, A.lyd, A.lzd};
@@ -361,8 +383,10 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void
 __global__ __launch_bounds__(BLOCK) void a_node2(AdjArgs A) {
   const int64_t n = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (n >= A.N) return;
+  const int s1 = A.s + 1, un = (int)n;
+  const NodeElems ne(un % s1, (un / s1) % s1, un / (s1 * s1), A.s);
   double g[6];
-  gather_corners(A, A.corner_f, n, g);
+  gather_corners(A, A.corner_f, ne, g);
   A.lx[n] += g[0];
   A.ly[n] += g[1];
   A.lz[n] += g[2];

@@ -37,6 +37,40 @@ constexpr uint32_t ZETA_P = 0x38000, ZETA_P_SYMM = 0x08000, ZETA_P_FREE = 0x1000
 
 constexpr int Q1 = 1, Q2 = 2, Q3 = 4;
 
+// An element's 8 nodes as 4 adjacent pairs (n, n+1) -- nodes (0,1) (3,2)
+// (4,5) (7,6) of the hex order of buildMesh! -- each pair one 16-byte load
+// at a 32-bit byte offset from a uniform base (node arrays of a context stay
+// below 4 GiB).  o[] = byte offsets of nodes 0, 3, 4, 7.
+LDEV void hex_pairs(uint32_t n0, uint32_t s1, uint32_t (&o)[4]) {
+  const uint32_t P = s1 * s1;
+  o[0] = n0 * 8u;
+  o[1] = (n0 + s1) * 8u;
+  o[2] = (n0 + P) * 8u;
+  o[3] = (n0 + P + s1) * 8u;
+}
+
+LDEV double2 ld_pair(const double *base, uint32_t boff) {
+  const double *p = (const double *)__builtin_assume_aligned((const char *)base + boff, 8);
+  double2 v;
+  __builtin_memcpy(&v, p, 16);
+  return v;
+}
+
+LDEV void gather8p(const double *__restrict__ base, const uint32_t (&o)[4], double (&out)[8]) {
+  const double2 a = ld_pair(base, o[0]), b = ld_pair(base, o[1]), c = ld_pair(base, o[2]),
+                d = ld_pair(base, o[3]);
+  out[0] = a.x; out[1] = a.y;
+  out[3] = b.x; out[2] = b.y;
+  out[4] = c.x; out[5] = c.y;
+  out[7] = d.x; out[6] = d.y;
+}
+
+// element of a field at a 32-bit byte offset from a uniform base
+template <typename T>
+LDEV T &at(T *base, uint32_t boff) {
+  return *(T *)((char *)base + boff);
+}
+
 // Julia 1.7 Base.min for Float64 (NaN-propagating, -0 < +0)
 LDEV double jmin(double x, double y) {
   bool takey = (y < x) || (signbit(y) > signbit(x));
