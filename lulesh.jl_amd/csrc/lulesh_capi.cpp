@@ -325,12 +325,14 @@ int ensure_regions(lulesh_ctx *c) {
 // a batch keeps the plain cut (the balanced one measured slower there).
 bool balanced_cut(const lulesh_ctx *c) { return c->n == 1; }
 
-// Default z-march depth for the context's instances (auto_depth, with a
-// round of CUs x resident k_nodal workgroups per CU).
+// Default z-march depth for the context's instances (auto_depth_one for a
+// single domain; auto_depth, with a round of CUs x resident k_nodal
+// workgroups per CU, for a batch).
 int auto_depth(const lulesh_ctx *c) {
   std::vector<NodalPlanInst> pi;
   pi.reserve(c->inst.size());
   for (const InstDesc &I : c->inst) pi.push_back({I.s, NodalTile{I.etx, I.ety, I.tx, I.ty}});
+  if (c->n == 1) return auto_depth_one(pi[0], c->cus, c->nodal_per_cu);
   return lulesh::auto_depth(pi.data(), pi.size(), (int64_t)c->cus * c->nodal_per_cu,
                             balanced_cut(c));
 }

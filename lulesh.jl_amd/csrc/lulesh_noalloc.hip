@@ -75,7 +75,7 @@ Carve carve(int nx, const DeviceScratch &d) {
   c.eb = (int)((c.E + BLOCK - 1) / BLOCK);
   c.tile = nodal_tile(nx);
   const NodalPlanInst pi{nx, c.tile};
-  c.cut = depth_cut(nx, auto_depth(&pi, 1, (int64_t)d.cus * d.nodal_per_cu, true), true);
+  c.cut = depth_cut(nx, auto_depth_one(pi, d.cus, d.nodal_per_cu), true);
   c.gb = nodal_blocks(c.tile, c.cut);
   // one instance, its blocks taken as equally heavy (under the balanced
   // cut only the last chunk marches fewer planes): nodal_order's XCD runs

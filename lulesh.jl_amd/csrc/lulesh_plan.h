@@ -160,6 +160,31 @@ inline int auto_depth(const NodalPlanInst *insts, size_t n, int64_t slots, bool 
   return best;
 }
 
+// The same for one domain, where a launch may also leave CUs to a single
+// workgroup: a launch of p planes takes about 9.8 + 4.4 p us with at most one
+// workgroup on a CU and 10.4 + 6.4 p us with two (s=36 to 64, depths 1 to 8).
+// auto_depth takes the two for equal and, with few blocks, doubles up CUs
+// where fewer, deeper chunks on a CU each are faster: launches at s=48 29.6
+// -> 26.9 us (depth 2, 288 workgroups -> depth 3, 192), s=52 30.6 -> 27.9,
+// s=40 23.0 -> 22.4; from s=56 on both choose alike.
+inline int auto_depth_one(const NodalPlanInst &I, int64_t cus, int64_t per_cu) {
+  if (cus < 1) cus = 1;
+  const int64_t slots = per_cu > 1 ? cus * per_cu : cus;
+  int best = 2;
+  int64_t best_cost = -1;
+  for (int d = 1; d <= I.s + 1; ++d) {
+    const NodalCut k = depth_cut(I.s, d, true);
+    const int64_t total = nodal_blocks(I.t, k);
+    const int64_t planes = k.cz + 1, rounds = (total + slots - 1) / slots;
+    const int64_t cost = total <= cus ? 98 + 44 * planes : 104 + 64 * planes * rounds;
+    if (best_cost < 0 || cost < best_cost) {
+      best = d;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 // k_nodal dispatch order.  The dispatcher deals a launch's workgroups
 // round-robin over the eight XCDs (workgroup g to XCD g % 8), each with its
 // own L2.  XCD x gets the x-th of eight contiguous runs of the block order
