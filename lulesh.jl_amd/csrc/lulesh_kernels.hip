@@ -1171,17 +1171,18 @@ __global__ __launch_bounds__(KIN_CHUNK) void k_kin(Batch B) {
 #undef LULESH_ZETA
 }
 
-// neighbour ids exactly as setupElementConnectivities stores them
-// (src/domain.jl:793-820), 0-based
-LDEV int64_t nb_xim(int64_t e) { return e == 0 ? 1 : e - 1; }
-LDEV int64_t nb_xip(int64_t e, int64_t E) { return e < E - 1 ? e + 1 : E - 1; }
-LDEV int64_t nb_etam(int64_t e, int64_t s) { return e < s ? e : e - s; }
-LDEV int64_t nb_etap(int64_t e, int64_t s, int64_t E) { return e < E - s ? e + s : e - (E - s); }
-LDEV int64_t nb_zetam(int64_t e, int64_t s2) { return e < s2 ? e : e - s2; }
-LDEV int64_t nb_zetap(int64_t e, int64_t s2, int64_t E) { return e < E - s2 ? e + s2 : e; }
-// a read the reference would make out of bounds (only reachable with an
-// uploaded elemBC that marks a boundary face interior, or s = 1) is clamped
-LDEV int64_t clampi(int64_t i, int64_t E) { return i < 0 ? 0 : (i >= E ? E - 1 : i); }
+// Neighbour ids as setupElementConnectivities stores them
+// (src/domain.jl:793-820), 0-based, its odd entries included; a read the
+// reference would make out of bounds (only reachable with an uploaded elemBC
+// that marks a boundary face interior, or s = 1) is clamped.
+LDEV uint32_t nb_xim(uint32_t e, uint32_t E) { return e ? e - 1u : (E > 1u ? 1u : 0u); }
+LDEV uint32_t nb_xip(uint32_t e, uint32_t E, bool q3) {
+  const uint32_t nb = e < E - 1u ? e + 1u : E - 1u;
+  return q3 ? (nb ? nb - 1u : 0u) : nb;
+}
+LDEV uint32_t nb_minus(uint32_t e, uint32_t step) { return e < step ? e : e - step; }  // eta, zeta
+LDEV uint32_t nb_etap(uint32_t e, uint32_t s, uint32_t E) { return e < E - s ? e + s : e - (E - s); }
+LDEV uint32_t nb_zetap(uint32_t e, uint32_t s2, uint32_t E) { return e < E - s2 ? e + s2 : e; }
 
 // block-wide minimum of two values (64-wide wavefronts, BLOCK threads)
 LDEV void block_min2(double &a, double &b) {
@@ -1210,7 +1211,14 @@ LDEV void block_min2(double &a, double &b) {
 // time; the reference's element-wise temporaries never mix elements),
 // updateVolumesForElems (2912-2930) and the per-element terms of
 // calcCourantConstraintForElems / calcHydroConstraintForElems (2964-3054)
-template <bool COST>
+//
+// EARLY: every value the element may need is read up front.  A small launch
+// lasts as long as its chain of waits and is shorter that way (s=16 9.1 ->
+// 8.7 us, s=48 10.8 -> 10.3); a large one streams, and the values held over
+// the limiter cost it resident waves (s=96 30.9 -> 31.6, s=192 198 -> 203).
+// The line lies at 1024 blocks: s=64 (1024) 14.3 -> 13.85, s=72 (1458) alike.
+constexpr int QEOS_EARLY = 1024;
+template <bool COST, bool EARLY>
 __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
   LULESH_ELEM_PREAMBLE_T(B, qeos_order)
   if (B.gated && !sc->active) return;  // uniform over the block
@@ -1221,64 +1229,57 @@ __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
     const double ptiny = 1e-36;
     const double mult = sc->monoq_limiter_mult, maxslope = sc->monoq_max_slope;
     const uint32_t bc = ld_nt(&f.elemBC[e]);
-    const double dvxi = f.delv_xi[e], dveta = f.delv_eta[e], dvzeta = f.delv_zeta[e];
+    // The six neighbours' values are read before the boundary mask is known
+    // (their ids are valid whatever it says), so nothing waits for it first:
+    // s=16 9.6 -> 8.9 us a launch, s=48 11.3 -> 10.8, large domains alike.
+    const uint32_t ue = (uint32_t)e, uE = (uint32_t)E, us = (uint32_t)s, s2 = us * us;
+    const uint32_t eo = ue * 8u;
+    const double dvxi = at(f.delv_xi, eo), dveta = at(f.delv_eta, eo), dvzeta = at(f.delv_zeta, eo);
+    const double nxim = at(f.delv_xi, nb_xim(ue, uE) * 8u), nxip = at(f.delv_xi, nb_xip(ue, uE, quirks & Q3) * 8u);
+    const double netam = at(f.delv_eta, nb_minus(ue, us) * 8u), netap = at(f.delv_eta, nb_etap(ue, us, uE) * 8u);
+    const double nzetam = at(f.delv_zeta, nb_minus(ue, s2) * 8u), nzetap = at(f.delv_zeta, nb_zetap(ue, s2, uE) * 8u);
+    double early[12];
+    if constexpr (EARLY) {
+      const double *src[12] = {f.vdov, f.volo, f.vnew, f.delx_xi, f.delx_eta, f.delx_zeta,
+                               f.elemMass, f.v, f.arealg, f.e, f.p, f.q};
+#pragma unroll
+      for (int k = 0; k < 12; ++k) early[k] = ld_nt(&src[k][e]);
+    }
+    auto own = [&](int k, const double *p) { return EARLY ? early[k] : ld_nt(&p[e]); };
     bool bad = false;
-    double delvm = 0.0, delvp = 0.0;
-    uint32_t c;
-    // xi
-    c = bc & XI_M;
-    if (c == 0 || c == XI_M_COMM) delvm = f.delv_xi[clampi(nb_xim(e), E)];
-    else if (c == XI_M_SYMM) delvm = dvxi;
-    else if (c == XI_M_FREE) delvm = 0.0;
-    else { delvm = 0.0; bad = true; }
-    c = bc & XI_P;
-    if (c == 0 || c == XI_P_COMM) {
-      const int64_t nb = nb_xip(e, E);  // stored 0-based id
-      delvp = (quirks & Q3) ? f.delv_xi[clampi(nb - 1, E)] : f.delv_xi[clampi(nb, E)];
-    } else if (c == XI_P_SYMM) delvp = dvxi;
-    else if (c == XI_P_FREE) delvp = 0.0;
-    else { delvp = 0.0; bad = true; }
-    const double phixi = limit_phi(delvm, delvp, 1.0 / (dvxi + ptiny), mult, maxslope);
-    // eta
-    c = bc & ETA_M;
-    if (c == 0 || c == ETA_M_COMM) delvm = f.delv_eta[clampi(nb_etam(e, s), E)];
-    else if (c == ETA_M_SYMM) delvm = dveta;
-    else if (c == ETA_M_FREE) delvm = 0.0;
-    else { delvm = 0.0; bad = true; }
-    c = bc & ETA_P;
-    if (c == 0 || c == ETA_P_COMM) delvp = f.delv_eta[clampi(nb_etap(e, s, E), E)];
-    else if (c == ETA_P_SYMM) delvp = dveta;
-    else if (c == ETA_P_FREE) delvp = 0.0;
-    else { delvp = 0.0; bad = true; }
-    const double phieta = limit_phi(delvm, delvp, 1.0 / (dveta + ptiny), mult, maxslope);
-    // zeta
-    const int64_t s2 = (int64_t)s * s;
-    c = bc & ZETA_M;
-    if (c == 0 || c == ZETA_M_COMM) delvm = f.delv_zeta[clampi(nb_zetam(e, s2), E)];
-    else if (c == ZETA_M_SYMM) delvm = dvzeta;
-    else if (c == ZETA_M_FREE) delvm = 0.0;
-    else { delvm = 0.0; bad = true; }
-    c = bc & ZETA_P;
-    if (c == 0 || c == ZETA_P_COMM) delvp = f.delv_zeta[clampi(nb_zetap(e, s2, E), E)];
-    else if (c == ZETA_P_SYMM) delvp = dvzeta;
-    else if (c == ZETA_P_FREE) delvp = 0.0;
-    else { delvp = 0.0; bad = true; }
-    const double phizeta = limit_phi(delvm, delvp, 1.0 / (dvzeta + ptiny), mult, maxslope);
+    // what a face's bits select: the neighbour (interior or COMM), the
+    // element itself (SYMM), zero (FREE); anything else is the reference's
+    // "Error" path
+    auto side = [&](uint32_t mask, uint32_t symm, uint32_t free, uint32_t comm, double there, double self) {
+      const uint32_t c = bc & mask;
+      const bool read = c == 0 || c == comm;
+      bad = bad || !(read || c == symm || c == free);
+      return read ? there : c == symm ? self : 0.0;
+    };
+    const double phixi = limit_phi(side(XI_M, XI_M_SYMM, XI_M_FREE, XI_M_COMM, nxim, dvxi),
+                                   side(XI_P, XI_P_SYMM, XI_P_FREE, XI_P_COMM, nxip, dvxi),
+                                   1.0 / (dvxi + ptiny), mult, maxslope);
+    const double phieta = limit_phi(side(ETA_M, ETA_M_SYMM, ETA_M_FREE, ETA_M_COMM, netam, dveta),
+                                    side(ETA_P, ETA_P_SYMM, ETA_P_FREE, ETA_P_COMM, netap, dveta),
+                                    1.0 / (dveta + ptiny), mult, maxslope);
+    const double phizeta = limit_phi(side(ZETA_M, ZETA_M_SYMM, ZETA_M_FREE, ZETA_M_COMM, nzetam, dvzeta),
+                                     side(ZETA_P, ZETA_P_SYMM, ZETA_P_FREE, ZETA_P_COMM, nzetap, dvzeta),
+                                     1.0 / (dvzeta + ptiny), mult, maxslope);
     if (bad) raise(sc, ERR_BC);
 
-    const double vdov = ld_nt(&f.vdov[e]), volo = ld_nt(&f.volo[e]), vnew = ld_nt(&f.vnew[e]);
+    const double vdov = own(0, f.vdov), volo = own(1, f.volo), vnew = own(2, f.vnew);
     double qlin, qquad;
     if (vdov > 0.0) {
       qlin = 0.0;
       qquad = 0.0;
     } else {
-      double delvxxi = dvxi * ld_nt(&f.delx_xi[e]);
-      double delvxeta = dveta * ld_nt(&f.delx_eta[e]);
-      double delvxzeta = dvzeta * ld_nt(&f.delx_zeta[e]);
+      double delvxxi = dvxi * own(3, f.delx_xi);
+      double delvxeta = dveta * own(4, f.delx_eta);
+      double delvxzeta = dvzeta * own(5, f.delx_zeta);
       if (delvxxi > 0.0) delvxxi = 0.0;
       if (delvxeta > 0.0) delvxeta = 0.0;
       if (delvxzeta > 0.0) delvxzeta = 0.0;
-      const double rho = ld_nt(&f.elemMass[e]) / (volo * vnew);
+      const double rho = own(6, f.elemMass) / (volo * vnew);
       qlin = ((-sc->qlc_monoq) * rho) *
              (((delvxxi * (1.0 - phixi)) + (delvxeta * (1.0 - phieta))) + (delvxzeta * (1.0 - phizeta)));
       qquad = (sc->qqc_monoq * rho) *
@@ -1292,12 +1293,12 @@ __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
     }
 
     // QStop on the q of the previous cycle
-    double q_old = ld_nt(&f.q[e]);
+    double q_old = own(11, f.q);
     if (q_old > sc->qstop) raise(sc, ERR_QSTOP);
 
     // material properties
     const double eosvmin = sc->eosvmin, eosvmax = sc->eosvmax;
-    const double v_old = ld_nt(&f.v[e]);
+    const double v_old = own(7, f.v);
     double vc = v_old;
     if (eosvmin != 0.0 && vc < eosvmin) vc = eosvmin;
     if (eosvmax != 0.0 && vc > eosvmax) vc = eosvmax;
@@ -1308,7 +1309,7 @@ __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
 
     // delv as k_kin formed it from the same two values: 8 of 172 bytes per
     // element less to read (s=192 200 -> 190 us, batch 162 -> 151)
-    const double delvc_in = vnew - v_old, e_old_in = ld_nt(&f.e[e]), p_old_in = ld_nt(&f.p[e]);
+    const double delvc_in = vnew - v_old, e_old_in = own(9, f.e), p_old_in = own(10, f.p);
     const double TINY1 = 0.111111e-36, TINY3 = 0.333333e-18, SIXTH = 1.0 / 6.0;
     const double pmin = sc->pmin, p_cut = sc->p_cut, e_cut = sc->e_cut, q_cut = sc->q_cut;
     const double emin = sc->emin, rho0 = sc->refdens;
@@ -1397,7 +1398,7 @@ __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
     if (vdov != 0.0) {
       const double qqc = sc->qqc;
       const double qqc2 = (64.0 * qqc) * qqc;
-      const double arealg = ld_nt(&f.arealg[e]);
+      const double arealg = own(8, f.arealg);
       double dtf = ss * ss;
       if (vdov < 0.0) dtf = dtf + ((((qqc2 * arealg) * arealg) * vdov) * vdov);
       dtf = sqrt(dtf);
@@ -1587,9 +1588,11 @@ hipError_t launch_kernel(int id, hipStream_t st, const Batch &b) {
       break;
     case KID_QEOS:
       if (b.cost_mode)
-        hipLaunchKernelGGL(k_qeos<true>, dim3(b.qeos_launch), dim3(BLOCK), 0, st, b);
+        hipLaunchKernelGGL((k_qeos<true, false>), dim3(b.qeos_launch), dim3(BLOCK), 0, st, b);
+      else if (b.eblocks <= QEOS_EARLY)
+        hipLaunchKernelGGL((k_qeos<false, true>), dim3(b.qeos_launch), dim3(BLOCK), 0, st, b);
       else
-        hipLaunchKernelGGL(k_qeos<false>, dim3(b.qeos_launch), dim3(BLOCK), 0, st, b);
+        hipLaunchKernelGGL((k_qeos<false, false>), dim3(b.qeos_launch), dim3(BLOCK), 0, st, b);
       break;
     case KID_DT:
       hipLaunchKernelGGL(k_dt, dim3(b.n), dim3(1024), 0, st, b);
