@@ -49,7 +49,8 @@ struct lulesh_ctx {
   hipStream_t stream = nullptr;
   Batch b{};                      // device pointers + launch geometry
   DevScalars *hsc = nullptr;      // pinned host mirror [n]
-  bool partials_valid = false;
+  bool partials_valid = false;    // dtpart holds what the last lagrangeElements left
+  int partials = 0;               // ... in so many pairs (one domain)
   int cus = 256, nodal_per_cu = 2;  // compute units; k_nodal workgroups resident per CU
   int keep_aux = 0;
   // timing
@@ -128,6 +129,14 @@ Batch make_args(lulesh_ctx *c, int gated, int loop_mode, int64_t num_iters = 0) 
   a.keep_aux = c->keep_aux;
   a.num_iters = num_iters;
   a.flip = 1;
+  // (timing reports k_kin and k_qeos each by itself)
+  if (c->n == 1) {
+    const int ebn = c->inst[0].ebn;
+    const ElemsPlan p = elems_plan(c->inst[0].s, ebn, c->cus);
+    const bool apart = c->timing || c->b.cost_mode;
+    a.elems_form = apart ? ELEMS_APART : p.form;
+    a.parts = apart ? ebn : p.parts;
+  }
   return a;
 }
 
@@ -577,7 +586,9 @@ int create(int32_t n, const int32_t *nx, const double *einit_scale, const double
   for (double **p : nf)
     if (!rc) rc = dev_alloc(c, p, n0);
   if (!rc) rc = dev_alloc(c, &f.elemBC, e0);
-  if (!rc) rc = dev_alloc(c, &B.dtpart, 2 * (int64_t)eb);
+  int64_t parts = eb;
+  if (n == 1) parts = std::max<int64_t>(parts, elems_plan(c->inst[0].s, eb, c->cus).parts);
+  if (!rc) rc = dev_alloc(c, &B.dtpart, 2 * parts);
   if (!rc) rc = dev_alloc(c, &B.sc, n);
   InstDesc *dinst = nullptr;
   int *deb = nullptr, *dnb = nullptr;
@@ -1712,6 +1723,7 @@ int lulesh_lagrange_elements(lulesh_ctx *c) {
     if (rc) return rc;
     rc = finish(c, true);
     c->partials_valid = (rc == 0);
+    c->partials = a.parts;
     return rc;
   } catch (...) {
     return exception_status(c);
@@ -1722,7 +1734,8 @@ int lulesh_calc_time_constraints(lulesh_ctx *c) {
   try {
     if (!c) return LULESH_ERR_INVALID_ARG;
     HIP_TRY(c, hipSetDevice(c->device));
-    const Batch a = make_args(c, 0, 0);
+    Batch a = make_args(c, 0, 0);
+    a.parts = c->partials_valid ? c->partials : c->inst[0].ebn;
     int rc = 0;
     if (!c->partials_valid) rc = launch(c, KID_DTPART, a);
     if (!rc) rc = launch(c, KID_DT, a);

@@ -90,7 +90,9 @@ struct Batch {
   int qeos_launch;          // k_qeos workgroups launched
   DevScalars *sc;           // [n]
   DevFields f;
-  double *dtpart;           // 2 per element-kernel block
+  double *dtpart;           // 2 per element-kernel block (or k_elems workgroup)
+  int elems_form;           // ElemsForm; other than ELEMS_APART, KID_QEOS runs both and KID_KIN nothing
+  int parts;                // one domain: the pairs of dtpart its element kernel wrote
   int quirks;
   int gated;                // kernels skip instances whose active flag is 0
   int keep_aux;             // also write fx.., xdd.., dxx.., ql, qq

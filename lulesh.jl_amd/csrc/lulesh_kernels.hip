@@ -208,10 +208,10 @@ LDEV void gather_errs(DevScalars *sc) {
 struct DtFold {
   double courant, hydro;
 };
-LDEV DtFold dt_fold_load(const Batch &B, int ebn) {
+LDEV DtFold dt_fold_load(const Batch &B) {
   const double2 *__restrict__ p = (const double2 *)B.dtpart;
   double a = 1.0e+20, b = 1.0e+20;
-  for (int i = threadIdx.x; i < ebn; i += BLOCK) {
+  for (int i = threadIdx.x; i < B.parts; i += BLOCK) {
     const double2 v = p[i];
     a = v.x < a ? v.x : a;
     b = v.y < b ? v.y : b;
@@ -261,8 +261,8 @@ LDEV DtNow dt_now_of(const DevScalars &S, bool fold, const double (*m)[2]) {
 }
 // A nodal workgroup of a loop that has ended: the constraints are folded all
 // the same, and the last workgroup stores them.
-LDEV void dt_fold_end(DevScalars *sc, int last, double (*m)[2], const Batch &B, int ebn) {
-  dt_fold_wave(dt_fold_load(B, ebn), m);
+LDEV void dt_fold_end(DevScalars *sc, int last, double (*m)[2], const Batch &B) {
+  dt_fold_wave(dt_fold_load(B), m);
   __syncthreads();
   if (threadIdx.x == 0 && atomicAdd(&sc->nodal_done, 1) == last) {
     const DtFold d = dt_fold_take(*sc, m);
@@ -688,10 +688,10 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
     fold = S.dt_pending;
     if (fold) {
       if (!loop_goes_on(sc, previous_err(sc, par))) {
-        dt_fold_end(sc, I.gbn - 1, dt_shared().m, B, I.ebn);
+        dt_fold_end(sc, I.gbn - 1, dt_shared().m, B);
         return;
       }
-      dt_fold_wave(dt_fold_load(B, I.ebn), dt_shared().m);
+      dt_fold_wave(dt_fold_load(B), dt_shared().m);
     }
   }
 
@@ -932,10 +932,10 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
   DtFold mine{1.0e+20, 1.0e+20};
   if (fold) {
     if (!loop_goes_on(sc, previous_err(sc, par))) {
-      dt_fold_end(sc, last, dts.m, B, I.ebn);
+      dt_fold_end(sc, last, dts.m, B);
       return;
     }
-    mine = dt_fold_load(B, I.ebn);
+    mine = dt_fold_load(B);
   }
 
   // three node planes around k (those outside the domain repeat the edge)
@@ -1070,8 +1070,113 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
   }
 }
 
-// calcKinematicsForElems (src/domain.jl:2099-2147), the deviatoric loop
-// (2156-2171) and calcMonotonicQGradientsForElems (2175-2320)
+// the node values of the element at (col, row, plane) of a domain of s
+// elements per edge
+struct ElemNodes {
+  double X[8], Y[8], Z[8], XV[8], YV[8], ZV[8];
+};
+LDEV void load_nodes(const NodeSet &S, uint32_t col, uint32_t row, uint32_t plane, uint32_t s1, ElemNodes &n) {
+  uint32_t nid[4];
+  hex_pairs((plane * s1 + row) * s1 + col, s1, nid);
+  gather8p(S.x, nid, n.X); gather8p(S.y, nid, n.Y); gather8p(S.z, nid, n.Z);
+  gather8p(S.xd, nid, n.XV); gather8p(S.yd, nid, n.YV); gather8p(S.zd, nid, n.ZV);
+}
+
+// calcMonotonicQGradientsForElems (src/domain.jl:2175-2320) of one element
+// along one axis (0 xi, 1 eta, 2 zeta): the side's length delx and the
+// velocity gradient delv.
+//
+// Four times the reference's side differences d' = 4 d: powers of two
+// factor out exactly, so an area vector is a' = 16 a, sqrt(a.a + ptiny) =
+// sqrt(a'.a' + 256 ptiny) / 16, and a.dv norm = a'.dv' (norm / 64).
+#define LULESH_SIDE(v, a, b, c, d, e, f, g, h) (sum4(v[a], v[b], v[c], v[d]) - sum4(v[e], v[f], v[g], v[h]))
+#define LULESH_ETA(v) (-LULESH_SIDE(v, 0, 1, 5, 4, 3, 2, 6, 7))
+#define LULESH_XI(v) LULESH_SIDE(v, 1, 2, 6, 5, 0, 3, 7, 4)
+#define LULESH_ZETA(v) LULESH_SIDE(v, 4, 5, 6, 7, 0, 1, 2, 3)
+template <int AXIS>
+LDEV void monoq_gradient(const ElemNodes &n, double vol, double &delx, double &delv) {
+  const double norm = 1.0 / (vol + 1.e-36);
+  const double ptiny256 = 256.0 * 1.e-36, norm64 = norm * 0.015625, vol16 = vol * 16.0;
+  // zeta: i cross j, xi: j cross k, eta: k cross i
+  double u[3], w[3], dv[3];
+  if constexpr (AXIS == 0) {
+    u[0] = LULESH_ETA(n.X); u[1] = LULESH_ETA(n.Y); u[2] = LULESH_ETA(n.Z);
+    w[0] = LULESH_ZETA(n.X); w[1] = LULESH_ZETA(n.Y); w[2] = LULESH_ZETA(n.Z);
+    dv[0] = LULESH_XI(n.XV); dv[1] = LULESH_XI(n.YV); dv[2] = LULESH_XI(n.ZV);
+  } else if constexpr (AXIS == 1) {
+    u[0] = LULESH_ZETA(n.X); u[1] = LULESH_ZETA(n.Y); u[2] = LULESH_ZETA(n.Z);
+    w[0] = LULESH_XI(n.X); w[1] = LULESH_XI(n.Y); w[2] = LULESH_XI(n.Z);
+    dv[0] = LULESH_ETA(n.XV); dv[1] = LULESH_ETA(n.YV); dv[2] = LULESH_ETA(n.ZV);
+  } else {
+    u[0] = LULESH_XI(n.X); u[1] = LULESH_XI(n.Y); u[2] = LULESH_XI(n.Z);
+    w[0] = LULESH_ETA(n.X); w[1] = LULESH_ETA(n.Y); w[2] = LULESH_ETA(n.Z);
+    dv[0] = LULESH_ZETA(n.XV); dv[1] = LULESH_ZETA(n.YV); dv[2] = LULESH_ZETA(n.ZV);
+  }
+  const double ax = (u[1] * w[2]) - (u[2] * w[1]);
+  const double ay = (u[2] * w[0]) - (u[0] * w[2]);
+  const double az = (u[0] * w[1]) - (u[1] * w[0]);
+  delx = vol16 / sqrt((((ax * ax) + (ay * ay)) + (az * az)) + ptiny256);
+  delv = (((ax * norm64) * dv[0]) + ((ay * norm64) * dv[1])) + ((az * norm64) * dv[2]);
+}
+#undef LULESH_SIDE
+#undef LULESH_ETA
+#undef LULESH_XI
+#undef LULESH_ZETA
+
+// What calcKinematicsForElems (src/domain.jl:2099-2147) and the deviatoric
+// loop (2156-2171) leave of one element, each value handed to
+// put(field, value, index) where it is known; v_old() is the element's
+// relative volume before the cycle.  Returns the one after it.
+enum KinValue { KV_VDOV, KV_VNEW, KV_AREALG, KV_OTHER };
+template <class Put, class VOld>
+LDEV double kin_strain(const ElemNodes &n, const DevFields &f, DevScalars *sc, double volo, VOld v_old,
+                       int keep_aux, Put put) {
+  const double volume = elem_volume(n.X, n.Y, n.Z);
+  const double vnew = volume / volo;
+  if (vnew <= 0.0) raise(sc, ERR_KIN_VOLUME);
+  put(f.vnew, vnew, KV_VNEW);
+  put(f.delv, vnew - v_old(), KV_OTHER);
+  put(f.arealg, char_length(n.X, n.Y, n.Z, volume), KV_AREALG);
+  {
+    const double dt2 = 0.5 * sc->deltatime;
+    double XS[8], YS[8], ZS[8], b[4][3];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      XS[k] = n.X[k] - dt2 * n.XV[k];
+      YS[k] = n.Y[k] - dt2 * n.YV[k];
+      ZS[k] = n.Z[k] - dt2 * n.ZV[k];
+    }
+    // (64 x detJ and 64 x b: the factors cancel exactly)
+    const double detJ = shape_derivatives4_64(XS, YS, ZS, b);
+    const double inv_detJ = 1.0 / detJ;
+    const double d1 = inv_detJ * vgrad_term(b, 0, n.XV);
+    const double d2 = inv_detJ * vgrad_term(b, 1, n.YV);
+    const double d3 = inv_detJ * vgrad_term(b, 2, n.ZV);
+    const double vdov = (d1 + d2) + d3;
+    put(f.vdov, vdov, KV_VDOV);
+    if (keep_aux) {
+      const double vdovthird = vdov / 3.0;
+      put(f.dxx, d1 - vdovthird, KV_OTHER);
+      put(f.dyy, d2 - vdovthird, KV_OTHER);
+      put(f.dzz, d3 - vdovthird, KV_OTHER);
+    }
+    if (vnew <= 0.0) raise(sc, ERR_LAG_VOLUME);
+  }
+  return vnew;
+}
+// its side lengths and velocity gradients along all three axes, vol its volume
+template <class Put>
+LDEV void kin_gradients(const ElemNodes &n, const DevFields &f, double vol, Put put) {
+  double delx, delv;
+  monoq_gradient<2>(n, vol, delx, delv);
+  put(f.delx_zeta, f.delv_zeta, delx, delv, 2);
+  monoq_gradient<0>(n, vol, delx, delv);
+  put(f.delx_xi, f.delv_xi, delx, delv, 0);
+  monoq_gradient<1>(n, vol, delx, delv);
+  put(f.delx_eta, f.delv_eta, delx, delv, 1);
+}
+
+// kin_strain and kin_gradients of every element.
 //
 // Bound by its memory pattern (the same 24 gathers, 2 reads and 10 writes
 // alone take 240 us at s=192) and the vector instructions beside it.  Without
@@ -1095,80 +1200,19 @@ __global__ __launch_bounds__(KIN_CHUNK) void k_kin(Batch B) {
   const DevFields f = slice(B.f, I);
   if (e >= (int64_t)plane_end) return;
   const int keep_aux = B.keep_aux;
-  uint32_t nid[4];
-  {
-    const uint32_t ue = (uint32_t)e, us = (uint32_t)s, s1 = us + 1u;
-    const uint32_t col = ue % us, rest = ue / us;
-    hex_pairs(((rest / us) * s1 + rest % us) * s1 + col, s1, nid);
-  }
   const uint32_t eo = (uint32_t)e * 8u;
-  double X[8], Y[8], Z[8], XV[8], YV[8], ZV[8];
-  const NodeSet S = pick(f, sc->parity);
-  gather8p(S.x, nid, X); gather8p(S.y, nid, Y); gather8p(S.z, nid, Z);
-  gather8p(S.xd, nid, XV); gather8p(S.yd, nid, YV); gather8p(S.zd, nid, ZV);
-  const double volo = at(f.volo, eo);
-  const double volume = elem_volume(X, Y, Z);
-  const double vnew = volume / volo;
-  if (vnew <= 0.0) raise(sc, ERR_KIN_VOLUME);
-  st_nt(f.vnew, eo, vnew);
-  st_nt(f.delv, eo, vnew - at(f.v, eo));
-  st_nt(f.arealg, eo, char_length(X, Y, Z, volume));
+  ElemNodes n;
   {
-    const double dt2 = 0.5 * sc->deltatime;
-    double XS[8], YS[8], ZS[8], b[4][3];
-#pragma unroll
-    for (int n = 0; n < 8; ++n) {
-      XS[n] = X[n] - dt2 * XV[n];
-      YS[n] = Y[n] - dt2 * YV[n];
-      ZS[n] = Z[n] - dt2 * ZV[n];
-    }
-    // (64 x detJ and 64 x b: the factors cancel exactly)
-    const double detJ = shape_derivatives4_64(XS, YS, ZS, b);
-    const double inv_detJ = 1.0 / detJ;
-    const double d1 = inv_detJ * vgrad_term(b, 0, XV);
-    const double d2 = inv_detJ * vgrad_term(b, 1, YV);
-    const double d3 = inv_detJ * vgrad_term(b, 2, ZV);
-    const double vdov = (d1 + d2) + d3;
-    st_nt(f.vdov, eo, vdov);
-    if (keep_aux) {
-      const double vdovthird = vdov / 3.0;
-      st_nt(f.dxx, eo, d1 - vdovthird);
-      st_nt(f.dyy, eo, d2 - vdovthird);
-      st_nt(f.dzz, eo, d3 - vdovthird);
-    }
-    if (vnew <= 0.0) raise(sc, ERR_LAG_VOLUME);
+    const uint32_t ue = (uint32_t)e, us = (uint32_t)s, rest = ue / us;
+    load_nodes(pick(f, sc->parity), ue % us, rest % us, rest / us, us + 1u, n);
   }
-  // MonoQ gradients
-  const double ptiny = 1.e-36;
-  const double vol = volo * vnew;
-  const double norm = 1.0 / (vol + ptiny);
-  // Four times the reference's side differences d' = 4 d: powers of two
-  // factor out exactly, so an area vector is a' = 16 a, sqrt(a.a + ptiny) =
-  // sqrt(a'.a' + 256 ptiny) / 16, and a.dv norm = a'.dv' (norm / 64).
-  const double ptiny256 = 256.0 * 1.e-36, norm64 = norm * 0.015625, vol16 = vol * 16.0;
-#define LULESH_SIDE(v, a, b, c, d, e, f, g, h) (sum4(v[a], v[b], v[c], v[d]) - sum4(v[e], v[f], v[g], v[h]))
-#define LULESH_ETA(v) (-LULESH_SIDE(v, 0, 1, 5, 4, 3, 2, 6, 7))
-#define LULESH_XI(v) LULESH_SIDE(v, 1, 2, 6, 5, 0, 3, 7, 4)
-#define LULESH_ZETA(v) LULESH_SIDE(v, 4, 5, 6, 7, 0, 1, 2, 3)
-  const double dxj = LULESH_ETA(X), dyj = LULESH_ETA(Y), dzj = LULESH_ETA(Z);
-  const double dxi = LULESH_XI(X), dyi = LULESH_XI(Y), dzi = LULESH_XI(Z);
-  const double dxk = LULESH_ZETA(X), dyk = LULESH_ZETA(Y), dzk = LULESH_ZETA(Z);
-  auto gradient = [&](double ux, double uy, double uz, double wx, double wy, double wz, double dvx,
-                      double dvy, double dvz, double *delx, double *delv) {
-    const double ax = (uy * wz) - (uz * wy);
-    const double ay = (uz * wx) - (ux * wz);
-    const double az = (ux * wy) - (uy * wx);
-    st_nt(delx, eo, vol16 / sqrt((((ax * ax) + (ay * ay)) + (az * az)) + ptiny256));
-    st_nt(delv, eo, (((ax * norm64) * dvx) + ((ay * norm64) * dvy)) + ((az * norm64) * dvz));
-  };
-  // zeta: i cross j, xi: j cross k, eta: k cross i
-  gradient(dxi, dyi, dzi, dxj, dyj, dzj, LULESH_ZETA(XV), LULESH_ZETA(YV), LULESH_ZETA(ZV), f.delx_zeta, f.delv_zeta);
-  gradient(dxj, dyj, dzj, dxk, dyk, dzk, LULESH_XI(XV), LULESH_XI(YV), LULESH_XI(ZV), f.delx_xi, f.delv_xi);
-  gradient(dxk, dyk, dzk, dxi, dyi, dzi, LULESH_ETA(XV), LULESH_ETA(YV), LULESH_ETA(ZV), f.delx_eta, f.delv_eta);
-#undef LULESH_SIDE
-#undef LULESH_ETA
-#undef LULESH_XI
-#undef LULESH_ZETA
+  const double volo = at(f.volo, eo);
+  const double vnew = kin_strain(n, f, sc, volo, [&] { return at(f.v, eo); }, keep_aux,
+                                 [&](double *p, double v, int) { st_nt(p, eo, v); });
+  kin_gradients(n, f, volo * vnew, [&](double *px, double *pv, double delx, double delv, int) {
+    st_nt(px, eo, delx);
+    st_nt(pv, eo, delv);
+  });
 }
 
 // Neighbour ids as setupElementConnectivities stores them
@@ -1184,9 +1228,10 @@ LDEV uint32_t nb_minus(uint32_t e, uint32_t step) { return e < step ? e : e - st
 LDEV uint32_t nb_etap(uint32_t e, uint32_t s, uint32_t E) { return e < E - s ? e + s : e - (E - s); }
 LDEV uint32_t nb_zetap(uint32_t e, uint32_t s2, uint32_t E) { return e < E - s2 ? e + s2 : e; }
 
-// block-wide minimum of two values (64-wide wavefronts, BLOCK threads)
+// minimum of two values over a workgroup's first THREADS threads (64-wide
+// wavefronts), in thread 0; every thread calls it
+template <int THREADS = BLOCK>
 LDEV void block_min2(double &a, double &b) {
-  __shared__ double sa[BLOCK / 64], sb[BLOCK / 64];
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     const double oa = __shfl_xor(a, off, 64);
@@ -1194,11 +1239,13 @@ LDEV void block_min2(double &a, double &b) {
     a = oa < a ? oa : a;
     b = ob < b ? ob : b;
   }
+  if constexpr (THREADS == 64) return;
+  __shared__ double sa[THREADS / 64], sb[THREADS / 64];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  if (l == 0) { sa[w] = a; sb[w] = b; }
+  if (l == 0 && w < THREADS / 64) { sa[w] = a; sb[w] = b; }
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int i = 1; i < BLOCK / 64; ++i) {
+    for (int i = 1; i < THREADS / 64; ++i) {
       a = sa[i] < a ? sa[i] : a;
       b = sb[i] < b ? sb[i] : b;
     }
@@ -1212,6 +1259,179 @@ LDEV void block_min2(double &a, double &b) {
 // updateVolumesForElems (2912-2930) and the per-element terms of
 // calcCourantConstraintForElems / calcHydroConstraintForElems (2964-3054)
 //
+// own(field, index): the element's own value of a field; nb: the values of
+// delv_xi, delv_eta and delv_zeta at its six neighbours (xi -, +, eta -, +,
+// zeta -, +), whatever its boundary mask makes of them.
+enum QeosValue { QV_VDOV, QV_VOLO, QV_VNEW, QV_DELX, QV_MASS = QV_DELX + 3, QV_V, QV_AREALG, QV_E, QV_P, QV_Q, QV_COUNT };
+template <bool COST, class Own>
+LDEV void qeos_element(const DevFields &f, DevScalars *sc, uint32_t eo, uint32_t bc, double dvxi, double dveta,
+                       double dvzeta, const double (&nb)[6], Own own, int keep_aux, const int *elem_rep,
+                       double &cand_c, double &cand_h) {
+  const double ptiny = 1e-36;
+  const double mult = sc->monoq_limiter_mult, maxslope = sc->monoq_max_slope;
+  bool bad = false;
+  // what a face's bits select: the neighbour (interior or COMM), the
+  // element itself (SYMM), zero (FREE); anything else is the reference's
+  // "Error" path
+  auto side = [&](uint32_t mask, uint32_t symm, uint32_t free, uint32_t comm, double there, double self) {
+    const uint32_t c = bc & mask;
+    const bool read = c == 0 || c == comm;
+    bad = bad || !(read || c == symm || c == free);
+    return read ? there : c == symm ? self : 0.0;
+  };
+  const double phixi = limit_phi(side(XI_M, XI_M_SYMM, XI_M_FREE, XI_M_COMM, nb[0], dvxi),
+                                 side(XI_P, XI_P_SYMM, XI_P_FREE, XI_P_COMM, nb[1], dvxi),
+                                 1.0 / (dvxi + ptiny), mult, maxslope);
+  const double phieta = limit_phi(side(ETA_M, ETA_M_SYMM, ETA_M_FREE, ETA_M_COMM, nb[2], dveta),
+                                  side(ETA_P, ETA_P_SYMM, ETA_P_FREE, ETA_P_COMM, nb[3], dveta),
+                                  1.0 / (dveta + ptiny), mult, maxslope);
+  const double phizeta = limit_phi(side(ZETA_M, ZETA_M_SYMM, ZETA_M_FREE, ZETA_M_COMM, nb[4], dvzeta),
+                                   side(ZETA_P, ZETA_P_SYMM, ZETA_P_FREE, ZETA_P_COMM, nb[5], dvzeta),
+                                   1.0 / (dvzeta + ptiny), mult, maxslope);
+  if (bad) raise(sc, ERR_BC);
+
+  const double vdov = own(f.vdov, QV_VDOV), volo = own(f.volo, QV_VOLO), vnew = own(f.vnew, QV_VNEW);
+  double qlin, qquad;
+  if (vdov > 0.0) {
+    qlin = 0.0;
+    qquad = 0.0;
+  } else {
+    double delvxxi = dvxi * own(f.delx_xi, QV_DELX);
+    double delvxeta = dveta * own(f.delx_eta, QV_DELX + 1);
+    double delvxzeta = dvzeta * own(f.delx_zeta, QV_DELX + 2);
+    if (delvxxi > 0.0) delvxxi = 0.0;
+    if (delvxeta > 0.0) delvxeta = 0.0;
+    if (delvxzeta > 0.0) delvxzeta = 0.0;
+    const double rho = own(f.elemMass, QV_MASS) / (volo * vnew);
+    qlin = ((-sc->qlc_monoq) * rho) *
+           (((delvxxi * (1.0 - phixi)) + (delvxeta * (1.0 - phieta))) + (delvxzeta * (1.0 - phizeta)));
+    qquad = (sc->qqc_monoq * rho) *
+            ((((delvxxi * delvxxi) * (1.0 - (phixi * phixi))) +
+              ((delvxeta * delvxeta) * (1.0 - (phieta * phieta)))) +
+             ((delvxzeta * delvxzeta) * (1.0 - (phizeta * phizeta))));
+  }
+  if (keep_aux) {
+    st_nt(f.qq, eo, qquad);
+    st_nt(f.ql, eo, qlin);
+  }
+
+  // QStop on the q of the previous cycle
+  double q_old = own(f.q, QV_Q);
+  if (q_old > sc->qstop) raise(sc, ERR_QSTOP);
+
+  // material properties
+  const double eosvmin = sc->eosvmin, eosvmax = sc->eosvmax;
+  const double v_old = own(f.v, QV_V);
+  double vc = v_old;
+  if (eosvmin != 0.0 && vc < eosvmin) vc = eosvmin;
+  if (eosvmax != 0.0 && vc > eosvmax) vc = eosvmax;
+  if (vc <= 0.0) raise(sc, ERR_EOS_VOLUME);
+  double vnewc = vnew;
+  if (eosvmin != 0.0 && vnewc < eosvmin) vnewc = eosvmin;
+  if (eosvmax != 0.0 && vnewc > eosvmax) vnewc = eosvmax;
+
+  // delv as k_kin formed it from the same two values: 8 of 172 bytes per
+  // element less to read (s=192 200 -> 190 us, batch 162 -> 151)
+  const double delvc_in = vnew - v_old, e_old_in = own(f.e, QV_E), p_old_in = own(f.p, QV_P);
+  const double TINY1 = 0.111111e-36, TINY3 = 0.333333e-18, SIXTH = 1.0 / 6.0;
+  const double pmin = sc->pmin, p_cut = sc->p_cut, e_cut = sc->e_cut, q_cut = sc->q_cut;
+  const double emin = sc->emin, rho0 = sc->refdens;
+  // LULESH-2.0 cost mode: the energy update of an element is evaluated as
+  // many times as its region's regReps says (the same inputs each time, so
+  // the same result); the empty asm statements make every evaluation real
+  int rep = 1;
+  if constexpr (COST) rep = *elem_rep;
+  double p_new = 0.0, e_new = 0.0, q_new = 0.0, bvc = 0.0, pbvc = 0.0;
+  for (int rr = 0; rr < rep; ++rr) {
+  double delvc = delvc_in, e_old = e_old_in, p_old = p_old_in, q_o = q_old, vn = vnewc,
+         ql_r = qlin, qq_r = qquad;
+  if constexpr (COST) {
+    __asm__ volatile("" : "+v"(delvc), "+v"(e_old), "+v"(p_old), "+v"(q_o));
+    __asm__ volatile("" : "+v"(vn), "+v"(ql_r), "+v"(qq_r));
+  }
+  {
+  const double q_old = q_o, vnewc = vn, qlin = ql_r, qquad = qq_r;
+  double compression = 1.0 / vnewc - 1.0;
+  const double vchalf = vnewc - delvc * 0.5;
+  double compHalfStep = (1.0 / vchalf) - 1.0;
+  if (eosvmin != 0.0 && vnewc <= eosvmin) compHalfStep = compression;
+  if (eosvmax != 0.0 && vnewc >= eosvmax) {
+    p_old = 0.0;
+    compression = 0.0;
+    compHalfStep = 0.0;
+  }
+  const double work = 0.0;
+  e_new = (e_old - ((0.5 * delvc) * (p_old + q_old))) + (0.5 * work);
+  if (e_new < emin) e_new = emin;
+  const double pHalfStep = pressure(bvc, pbvc, e_new, compHalfStep, vnewc, pmin, p_cut, eosvmax);
+  const double vhalf = 1.0 / (1.0 + compHalfStep);
+  if (delvc > 0.0) {
+    q_new = 0.0;
+  } else {
+    double ssc = ((pbvc * e_new) + (((vhalf * vhalf) * bvc) * pHalfStep)) / rho0;
+    ssc = (ssc <= TINY1) ? TINY3 : sqrt(ssc);
+    q_new = (ssc * qlin) + qquad;
+  }
+  e_new = e_new + ((0.5 * delvc) * ((3.0 * (p_old + q_old)) - (4.0 * (pHalfStep + q_new))));
+  e_new = e_new + 0.5 * work;
+  if (fabs(e_new) < e_cut) e_new = 0.0;
+  if (e_new < emin) e_new = emin;
+  p_new = pressure(bvc, pbvc, e_new, compression, vnewc, pmin, p_cut, eosvmax);
+  double q_tilde;
+  if (delvc > 0.0) {
+    q_tilde = 0.0;
+  } else {
+    double ssc = ((pbvc * e_new) + (((vnewc * vnewc) * bvc) * p_new)) / rho0;
+    ssc = (ssc <= TINY1) ? TINY3 : sqrt(ssc);
+    q_tilde = (ssc * qlin) + qquad;
+  }
+  e_new = e_new - (((((7.0 * (p_old + q_old)) - (8.0 * (pHalfStep + q_new))) + (p_new + q_tilde)) *
+                    delvc) *
+                   SIXTH);
+  if (fabs(e_new) < e_cut) e_new = 0.0;
+  if (e_new < emin) e_new = emin;
+  p_new = pressure(bvc, pbvc, e_new, compression, vnewc, pmin, p_cut, eosvmax);
+  if (delvc <= 0.0) {
+    double ssc = ((pbvc * e_new) + (((vnewc * vnewc) * bvc) * p_new)) / rho0;
+    ssc = (ssc <= TINY1) ? TINY3 : sqrt(ssc);
+    q_new = (ssc * qlin) + qquad;
+    if (fabs(q_new) < q_cut) q_new = 0.0;
+  }
+  }
+  if constexpr (COST) {
+    __asm__ volatile("" ::"v"(p_new), "v"(e_new), "v"(q_new));
+    __asm__ volatile("" ::"v"(bvc), "v"(pbvc));
+  }
+  }
+  double ss = ((pbvc * e_new) + (((vnewc * vnewc) * bvc) * p_new)) / rho0;
+  ss = (ss <= TINY1) ? TINY3 : sqrt(ss);
+  st_nt(f.p, eo, p_new);
+  st_nt(f.e, eo, e_new);
+  st_nt(f.q, eo, q_new);
+  st_nt(f.ss, eo, ss);
+
+  // updateVolumesForElems
+  double tmpV = vnew;
+  if (fabs(tmpV - 1.0) < sc->v_cut) tmpV = 1.0;
+  st_nt(f.v, eo, tmpV);
+  if (tmpV <= 0.0) raise(sc, ERR_UPDATE_VOLUME);
+
+  // time-constraint terms; an element only counts where vdov != 0 and its
+  // value beats the 1e20 start value (strict <, as in the reference)
+  if (vdov != 0.0) {
+    const double qqc = sc->qqc;
+    const double qqc2 = (64.0 * qqc) * qqc;
+    const double arealg = own(f.arealg, QV_AREALG);
+    double dtf = ss * ss;
+    if (vdov < 0.0) dtf = dtf + ((((qqc2 * arealg) * arealg) * vdov) * vdov);
+    dtf = sqrt(dtf);
+    dtf = arealg / dtf;
+    if (dtf < cand_c) cand_c = dtf;
+    const double dtdvov = sc->dvovmax / (fabs(vdov) + 1.e-20);
+    if (dtdvov < cand_h) cand_h = dtdvov;
+  }
+}
+
 // EARLY: every value the element may need is read up front.  A small launch
 // lasts as long as its chain of waits and is shorter that way (s=16 9.1 ->
 // 8.7 us, s=48 10.8 -> 10.3); a large one streams, and the values held over
@@ -1222,12 +1442,10 @@ template <bool COST, bool EARLY>
 __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
   LULESH_ELEM_PREAMBLE_T(B, qeos_order)
   if (B.gated && !sc->active) return;  // uniform over the block
-  const int quirks = B.quirks, keep_aux = B.keep_aux;
+  const int quirks = B.quirks;
   double *__restrict__ dtpart = B.dtpart;
   double cand_c = 1.0e+20, cand_h = 1.0e+20;
   if (e < E) {
-    const double ptiny = 1e-36;
-    const double mult = sc->monoq_limiter_mult, maxslope = sc->monoq_max_slope;
     const uint32_t bc = ld_nt(&f.elemBC[e]);
     // The six neighbours' values are read before the boundary mask is known
     // (their ids are valid whatever it says), so nothing waits for it first:
@@ -1235,183 +1453,173 @@ __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
     const uint32_t ue = (uint32_t)e, uE = (uint32_t)E, us = (uint32_t)s, s2 = us * us;
     const uint32_t eo = ue * 8u;
     const double dvxi = at(f.delv_xi, eo), dveta = at(f.delv_eta, eo), dvzeta = at(f.delv_zeta, eo);
-    const double nxim = at(f.delv_xi, nb_xim(ue, uE) * 8u), nxip = at(f.delv_xi, nb_xip(ue, uE, quirks & Q3) * 8u);
-    const double netam = at(f.delv_eta, nb_minus(ue, us) * 8u), netap = at(f.delv_eta, nb_etap(ue, us, uE) * 8u);
-    const double nzetam = at(f.delv_zeta, nb_minus(ue, s2) * 8u), nzetap = at(f.delv_zeta, nb_zetap(ue, s2, uE) * 8u);
-    double early[12];
+    const double nb[6] = {
+        at(f.delv_xi, nb_xim(ue, uE) * 8u),         at(f.delv_xi, nb_xip(ue, uE, quirks & Q3) * 8u),
+        at(f.delv_eta, nb_minus(ue, us) * 8u),      at(f.delv_eta, nb_etap(ue, us, uE) * 8u),
+        at(f.delv_zeta, nb_minus(ue, s2) * 8u),     at(f.delv_zeta, nb_zetap(ue, s2, uE) * 8u)};
+    double early[QV_COUNT];
     if constexpr (EARLY) {
-      const double *src[12] = {f.vdov, f.volo, f.vnew, f.delx_xi, f.delx_eta, f.delx_zeta,
-                               f.elemMass, f.v, f.arealg, f.e, f.p, f.q};
+      const double *src[QV_COUNT] = {f.vdov, f.volo, f.vnew, f.delx_xi, f.delx_eta, f.delx_zeta,
+                                     f.elemMass, f.v, f.arealg, f.e, f.p, f.q};
 #pragma unroll
-      for (int k = 0; k < 12; ++k) early[k] = ld_nt(&src[k][e]);
+      for (int k = 0; k < QV_COUNT; ++k) early[k] = ld_nt(&src[k][e]);
     }
-    auto own = [&](int k, const double *p) { return EARLY ? early[k] : ld_nt(&p[e]); };
-    bool bad = false;
-    // what a face's bits select: the neighbour (interior or COMM), the
-    // element itself (SYMM), zero (FREE); anything else is the reference's
-    // "Error" path
-    auto side = [&](uint32_t mask, uint32_t symm, uint32_t free, uint32_t comm, double there, double self) {
-      const uint32_t c = bc & mask;
-      const bool read = c == 0 || c == comm;
-      bad = bad || !(read || c == symm || c == free);
-      return read ? there : c == symm ? self : 0.0;
-    };
-    const double phixi = limit_phi(side(XI_M, XI_M_SYMM, XI_M_FREE, XI_M_COMM, nxim, dvxi),
-                                   side(XI_P, XI_P_SYMM, XI_P_FREE, XI_P_COMM, nxip, dvxi),
-                                   1.0 / (dvxi + ptiny), mult, maxslope);
-    const double phieta = limit_phi(side(ETA_M, ETA_M_SYMM, ETA_M_FREE, ETA_M_COMM, netam, dveta),
-                                    side(ETA_P, ETA_P_SYMM, ETA_P_FREE, ETA_P_COMM, netap, dveta),
-                                    1.0 / (dveta + ptiny), mult, maxslope);
-    const double phizeta = limit_phi(side(ZETA_M, ZETA_M_SYMM, ZETA_M_FREE, ZETA_M_COMM, nzetam, dvzeta),
-                                     side(ZETA_P, ZETA_P_SYMM, ZETA_P_FREE, ZETA_P_COMM, nzetap, dvzeta),
-                                     1.0 / (dvzeta + ptiny), mult, maxslope);
-    if (bad) raise(sc, ERR_BC);
-
-    const double vdov = own(0, f.vdov), volo = own(1, f.volo), vnew = own(2, f.vnew);
-    double qlin, qquad;
-    if (vdov > 0.0) {
-      qlin = 0.0;
-      qquad = 0.0;
-    } else {
-      double delvxxi = dvxi * own(3, f.delx_xi);
-      double delvxeta = dveta * own(4, f.delx_eta);
-      double delvxzeta = dvzeta * own(5, f.delx_zeta);
-      if (delvxxi > 0.0) delvxxi = 0.0;
-      if (delvxeta > 0.0) delvxeta = 0.0;
-      if (delvxzeta > 0.0) delvxzeta = 0.0;
-      const double rho = own(6, f.elemMass) / (volo * vnew);
-      qlin = ((-sc->qlc_monoq) * rho) *
-             (((delvxxi * (1.0 - phixi)) + (delvxeta * (1.0 - phieta))) + (delvxzeta * (1.0 - phizeta)));
-      qquad = (sc->qqc_monoq * rho) *
-              ((((delvxxi * delvxxi) * (1.0 - (phixi * phixi))) +
-                ((delvxeta * delvxeta) * (1.0 - (phieta * phieta)))) +
-               ((delvxzeta * delvxzeta) * (1.0 - (phizeta * phizeta))));
-    }
-    if (keep_aux) {
-      st_nt(&f.qq[e], qquad);
-      st_nt(&f.ql[e], qlin);
-    }
-
-    // QStop on the q of the previous cycle
-    double q_old = own(11, f.q);
-    if (q_old > sc->qstop) raise(sc, ERR_QSTOP);
-
-    // material properties
-    const double eosvmin = sc->eosvmin, eosvmax = sc->eosvmax;
-    const double v_old = own(7, f.v);
-    double vc = v_old;
-    if (eosvmin != 0.0 && vc < eosvmin) vc = eosvmin;
-    if (eosvmax != 0.0 && vc > eosvmax) vc = eosvmax;
-    if (vc <= 0.0) raise(sc, ERR_EOS_VOLUME);
-    double vnewc = vnew;
-    if (eosvmin != 0.0 && vnewc < eosvmin) vnewc = eosvmin;
-    if (eosvmax != 0.0 && vnewc > eosvmax) vnewc = eosvmax;
-
-    // delv as k_kin formed it from the same two values: 8 of 172 bytes per
-    // element less to read (s=192 200 -> 190 us, batch 162 -> 151)
-    const double delvc_in = vnew - v_old, e_old_in = own(9, f.e), p_old_in = own(10, f.p);
-    const double TINY1 = 0.111111e-36, TINY3 = 0.333333e-18, SIXTH = 1.0 / 6.0;
-    const double pmin = sc->pmin, p_cut = sc->p_cut, e_cut = sc->e_cut, q_cut = sc->q_cut;
-    const double emin = sc->emin, rho0 = sc->refdens;
-    // LULESH-2.0 cost mode: the energy update of an element is evaluated as
-    // many times as its region's regReps says (the same inputs each time, so
-    // the same result); the empty asm statements make every evaluation real
-    int rep = 1;
-    if constexpr (COST) rep = B.elem_rep[I.e0 + e];
-    double p_new = 0.0, e_new = 0.0, q_new = 0.0, bvc = 0.0, pbvc = 0.0;
-    for (int rr = 0; rr < rep; ++rr) {
-    double delvc = delvc_in, e_old = e_old_in, p_old = p_old_in, q_o = q_old, vn = vnewc,
-           ql_r = qlin, qq_r = qquad;
-    if constexpr (COST) {
-      __asm__ volatile("" : "+v"(delvc), "+v"(e_old), "+v"(p_old), "+v"(q_o));
-      __asm__ volatile("" : "+v"(vn), "+v"(ql_r), "+v"(qq_r));
-    }
-    {
-    const double q_old = q_o, vnewc = vn, qlin = ql_r, qquad = qq_r;
-    double compression = 1.0 / vnewc - 1.0;
-    const double vchalf = vnewc - delvc * 0.5;
-    double compHalfStep = (1.0 / vchalf) - 1.0;
-    if (eosvmin != 0.0 && vnewc <= eosvmin) compHalfStep = compression;
-    if (eosvmax != 0.0 && vnewc >= eosvmax) {
-      p_old = 0.0;
-      compression = 0.0;
-      compHalfStep = 0.0;
-    }
-    const double work = 0.0;
-    e_new = (e_old - ((0.5 * delvc) * (p_old + q_old))) + (0.5 * work);
-    if (e_new < emin) e_new = emin;
-    const double pHalfStep = pressure(bvc, pbvc, e_new, compHalfStep, vnewc, pmin, p_cut, eosvmax);
-    const double vhalf = 1.0 / (1.0 + compHalfStep);
-    if (delvc > 0.0) {
-      q_new = 0.0;
-    } else {
-      double ssc = ((pbvc * e_new) + (((vhalf * vhalf) * bvc) * pHalfStep)) / rho0;
-      ssc = (ssc <= TINY1) ? TINY3 : sqrt(ssc);
-      q_new = (ssc * qlin) + qquad;
-    }
-    e_new = e_new + ((0.5 * delvc) * ((3.0 * (p_old + q_old)) - (4.0 * (pHalfStep + q_new))));
-    e_new = e_new + 0.5 * work;
-    if (fabs(e_new) < e_cut) e_new = 0.0;
-    if (e_new < emin) e_new = emin;
-    p_new = pressure(bvc, pbvc, e_new, compression, vnewc, pmin, p_cut, eosvmax);
-    double q_tilde;
-    if (delvc > 0.0) {
-      q_tilde = 0.0;
-    } else {
-      double ssc = ((pbvc * e_new) + (((vnewc * vnewc) * bvc) * p_new)) / rho0;
-      ssc = (ssc <= TINY1) ? TINY3 : sqrt(ssc);
-      q_tilde = (ssc * qlin) + qquad;
-    }
-    e_new = e_new - (((((7.0 * (p_old + q_old)) - (8.0 * (pHalfStep + q_new))) + (p_new + q_tilde)) *
-                      delvc) *
-                     SIXTH);
-    if (fabs(e_new) < e_cut) e_new = 0.0;
-    if (e_new < emin) e_new = emin;
-    p_new = pressure(bvc, pbvc, e_new, compression, vnewc, pmin, p_cut, eosvmax);
-    if (delvc <= 0.0) {
-      double ssc = ((pbvc * e_new) + (((vnewc * vnewc) * bvc) * p_new)) / rho0;
-      ssc = (ssc <= TINY1) ? TINY3 : sqrt(ssc);
-      q_new = (ssc * qlin) + qquad;
-      if (fabs(q_new) < q_cut) q_new = 0.0;
-    }
-    }
-    if constexpr (COST) {
-      __asm__ volatile("" ::"v"(p_new), "v"(e_new), "v"(q_new));
-      __asm__ volatile("" ::"v"(bvc), "v"(pbvc));
-    }
-    }
-    double ss = ((pbvc * e_new) + (((vnewc * vnewc) * bvc) * p_new)) / rho0;
-    ss = (ss <= TINY1) ? TINY3 : sqrt(ss);
-    st_nt(&f.p[e], p_new);
-    st_nt(&f.e[e], e_new);
-    st_nt(&f.q[e], q_new);
-    st_nt(&f.ss[e], ss);
-
-    // updateVolumesForElems
-    double tmpV = vnew;
-    if (fabs(tmpV - 1.0) < sc->v_cut) tmpV = 1.0;
-    st_nt(&f.v[e], tmpV);
-    if (tmpV <= 0.0) raise(sc, ERR_UPDATE_VOLUME);
-
-    // time-constraint terms; an element only counts where vdov != 0 and its
-    // value beats the 1e20 start value (strict <, as in the reference)
-    if (vdov != 0.0) {
-      const double qqc = sc->qqc;
-      const double qqc2 = (64.0 * qqc) * qqc;
-      const double arealg = own(8, f.arealg);
-      double dtf = ss * ss;
-      if (vdov < 0.0) dtf = dtf + ((((qqc2 * arealg) * arealg) * vdov) * vdov);
-      dtf = sqrt(dtf);
-      dtf = arealg / dtf;
-      if (dtf < cand_c) cand_c = dtf;
-      const double dtdvov = sc->dvovmax / (fabs(vdov) + 1.e-20);
-      if (dtdvov < cand_h) cand_h = dtdvov;
-    }
+    auto own = [&](const double *p, int k) { return EARLY ? early[k] : ld_nt(&p[e]); };
+    const int *rep = COST ? B.elem_rep + I.e0 + e : nullptr;
+    qeos_element<COST>(f, sc, eo, bc, dvxi, dveta, dvzeta, nb, own, B.keep_aux, rep, cand_c, cand_h);
   }
   block_min2(cand_c, cand_h);
   if (threadIdx.x == 0) {
     dtpart[2 * vb_] = cand_c;
     dtpart[2 * vb_ + 1] = cand_h;
+  }
+}
+
+// k_kin and k_qeos of one small domain in one launch (elems_form): a
+// workgroup runs its BX x BY x BZ block of elements and beside them the
+// velocity gradient of the elements behind each face along that face's axis;
+// after one barrier qeos_element finds its six neighbours in LDS.  Both
+// kernels last there as long as their launches and waits, so the elements
+// behind the faces, computed again by their own workgroups, cost nothing.
+// SPLIT: an element's kin_strain and kin_gradients run on two threads, a
+// third of the arithmetic off the longest chain; for launches that leave
+// SIMDs idle.  A cycle of the device loop loses 2.9 us of 24 at s=16 (2.3
+// unsplit), 3.1 of 27 at s=24, 1.4 of 30 at s=30; unsplit in blocks of 256
+// 3.3 of 35 at s=34, 0.9 of 39 at s=40.
+template <int BX, int BY, int BZ, bool SPLIT>
+struct ElemBlock {
+  static constexpr int CORE = BX * BY * BZ, FX = 2 * BY * BZ, FY = 2 * BX * BZ, FZ = 2 * BX * BY;
+  static constexpr int OWN = (SPLIT ? 2 : 1) * CORE;  // threads on the block's own elements
+  static constexpr int THREADS = (OWN + FX + FY + FZ + 63) / 64 * 64;
+  static_assert(CORE % 64 == 0, "the block's own elements fill whole waves");
+};
+template <int BX, int BY, int BZ, bool SPLIT>
+__global__ __launch_bounds__((ElemBlock<BX, BY, BZ, SPLIT>::THREADS)) void k_elems(Batch B) {
+  using EB = ElemBlock<BX, BY, BZ, SPLIT>;
+  __shared__ double lx[BZ][BY][BX + 2], ly[BZ][BY + 2][BX], lz[BZ + 2][BY][BX], ldelx[3][EB::CORE];
+  DevScalars *sc = B.sc;
+  if (B.gated && !sc->active) return;
+  const DevFields &f = B.f;
+  const int s = B.one.s, t = threadIdx.x;
+  // which element this thread runs, and what of it
+  enum { XI, ETA, ZETA, GRADIENTS, STRAIN, NONE };
+  int i, j, k, what;
+  if (t < EB::OWN) {
+    const int h = t % EB::CORE;
+    what = t < EB::CORE ? STRAIN : GRADIENTS;
+    i = h % BX; j = h / BX % BY; k = h / (BX * BY);
+  } else if (t < EB::OWN + EB::FZ) {
+    const int h = t - EB::OWN;
+    what = ZETA;
+    i = h % BX; j = h / BX % BY; k = h < EB::FZ / 2 ? -1 : BZ;
+  } else if (t < EB::OWN + EB::FZ + EB::FY) {
+    const int h = t - (EB::OWN + EB::FZ);
+    what = ETA;
+    i = h % BX; k = h / BX % BZ; j = h < EB::FY / 2 ? -1 : BY;
+  } else {
+    const int h = t - (EB::OWN + EB::FZ + EB::FY);
+    what = h < EB::FX ? XI : NONE;
+    j = h % BY; k = h / BY % BZ; i = h < EB::FX / 2 ? -1 : BX;
+  }
+  const int col = (int)blockIdx.x * BX + i, row = (int)blockIdx.y * BY + j, plane = (int)blockIdx.z * BZ + k;
+  const bool there = what != NONE && col >= 0 && col < s && row >= 0 && row < s && plane >= 0 && plane < s;
+  const uint32_t us = (uint32_t)s, ue = ((uint32_t)plane * us + (uint32_t)row) * us + (uint32_t)col, eo = ue * 8u;
+  const NodeSet S = pick(f, sc->parity);
+  double own[QV_COUNT];
+  uint32_t bc = 0;
+  if (there) {
+    ElemNodes n;
+    load_nodes(S, (uint32_t)col, (uint32_t)row, (uint32_t)plane, us + 1u, n);
+    const double volo = at(f.volo, eo);
+    double vnew;
+    if (what == STRAIN) {
+      own[QV_V] = at(f.v, eo); own[QV_MASS] = at(f.elemMass, eo);
+      own[QV_E] = at(f.e, eo); own[QV_P] = at(f.p, eo); own[QV_Q] = at(f.q, eo);
+      bc = f.elemBC[ue];
+      own[QV_VOLO] = volo;
+      vnew = kin_strain(n, f, sc, volo, [&] { return own[QV_V]; }, B.keep_aux, [&](double *p, double v, int kv) {
+        at(p, eo) = v;
+        if (kv == KV_VDOV) own[QV_VDOV] = v;
+        if (kv == KV_AREALG) own[QV_AREALG] = v;
+      });
+      own[QV_VNEW] = vnew;
+    } else {
+      vnew = elem_volume(n.X, n.Y, n.Z) / volo;
+    }
+    const double vol = volo * vnew;
+    double delx, delv;
+    if (what == GRADIENTS || (!SPLIT && what == STRAIN)) {
+      kin_gradients(n, f, vol, [&](double *px, double *pv, double dx, double dv, int axis) {
+        at(px, eo) = dx;
+        at(pv, eo) = dv;
+        ldelx[axis][t % EB::CORE] = dx;
+        if (axis == 0) lx[k][j][i + 1] = dv;
+        if (axis == 1) ly[k][j + 1][i] = dv;
+        if (axis == 2) lz[k + 1][j][i] = dv;
+      });
+    } else if (what == ZETA) {
+      monoq_gradient<2>(n, vol, delx, delv);
+      lz[k + 1][j][i] = delv;
+    } else if (what == ETA) {
+      monoq_gradient<1>(n, vol, delx, delv);
+      ly[k][j + 1][i] = delv;
+    } else if (what == XI) {
+      monoq_gradient<0>(n, vol, delx, delv);
+      lx[k][j][i + 1] = delv;
+    }
+  }
+  __syncthreads();
+  double cand_c = 1.0e+20, cand_h = 1.0e+20;
+  if (there && what == STRAIN) {
+    const double dv[3] = {lx[k][j][i + 1], ly[k][j + 1][i], lz[k + 1][j][i]};
+#pragma unroll
+    for (int a = 0; a < 3; ++a) own[QV_DELX + a] = ldelx[a][t];
+    // The neighbours the reference's lists name are those beside the element
+    // except at the domain's faces and, with quirk Q3, along +xi; there it is
+    // the element itself or one elsewhere (an uploaded mask that marks a
+    // boundary face interior), whose gradient is then formed here.
+    const uint32_t uE = us * us * us, s2 = us * us;
+    const uint32_t id[6] = {nb_xim(ue, uE), nb_xip(ue, uE, B.quirks & Q3), nb_minus(ue, us),
+                            nb_etap(ue, us, uE), nb_minus(ue, s2), nb_zetap(ue, s2, uE)};
+    const bool beside[6] = {col > 0, col < s - 1 && !(B.quirks & Q3), row > 0, row < s - 1, plane > 0, plane < s - 1};
+    constexpr uint32_t mask[6] = {XI_M, XI_P, ETA_M, ETA_P, ZETA_M, ZETA_P};
+    constexpr uint32_t comm[6] = {XI_M_COMM, XI_P_COMM, ETA_M_COMM, ETA_P_COMM, ZETA_M_COMM, ZETA_P_COMM};
+    double nb[6] = {lx[k][j][i], lx[k][j][i + 2], ly[k][j][i], ly[k][j + 2][i], lz[k][j][i], lz[k + 2][j][i]};
+    uint32_t far = 0;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      const uint32_t c = bc & mask[q];
+      if (!beside[q]) {
+        nb[q] = dv[q >> 1];
+        if ((c == 0 || c == comm[q]) && id[q] != ue) far |= 1u << q;
+      }
+    }
+    if (far) {
+#pragma unroll 1
+      for (int q = 0; q < 6; ++q) {
+        if (!((far >> q) & 1u)) continue;
+        uint32_t g = id[0];
+#pragma unroll
+        for (int r = 1; r < 6; ++r) g = q == r ? id[r] : g;
+        ElemNodes n;
+        load_nodes(S, g % us, g / us % us, g / s2, us + 1u, n);
+        const double volo = at(f.volo, g * 8u), vol = volo * (elem_volume(n.X, n.Y, n.Z) / volo);
+        double delx, d;
+        if (q < 2) monoq_gradient<0>(n, vol, delx, d);
+        else if (q < 4) monoq_gradient<1>(n, vol, delx, d);
+        else monoq_gradient<2>(n, vol, delx, d);
+#pragma unroll
+        for (int r = 0; r < 6; ++r) nb[r] = q == r ? d : nb[r];
+      }
+    }
+    qeos_element<false>(f, sc, eo, bc, dv[0], dv[1], dv[2], nb, [&](const double *, int v) { return own[v]; },
+                        B.keep_aux, nullptr, cand_c, cand_h);
+  }
+  block_min2<EB::CORE>(cand_c, cand_h);
+  if (t == 0) {
+    const int g = ((int)blockIdx.z * gridDim.y + (int)blockIdx.y) * gridDim.x + (int)blockIdx.x;
+    B.dtpart[2 * g] = cand_c;
+    B.dtpart[2 * g + 1] = cand_h;
   }
 }
 
@@ -1456,7 +1664,7 @@ __global__ __launch_bounds__(1024) void k_dt(Batch B) {
   // (courant, hydro) pairs, 16-byte aligned; four independent loads in
   // flight per thread (a minimum does not depend on the order it is taken in)
   const double2 *__restrict__ dtpart = (const double2 *)(B.dtpart + 2 * (int64_t)I.eb0);
-  const int64_t nb = I.ebn, bd = blockDim.x;
+  const int64_t nb = B.n == 1 ? B.parts : I.ebn, bd = blockDim.x;
   double a = 1.0e+20, b = 1.0e+20, a1 = 1.0e+20, b1 = 1.0e+20;
   int64_t i = threadIdx.x;
   for (; i + 3 * bd < nb; i += 4 * bd) {
@@ -1563,6 +1771,13 @@ static void launch_nodal(hipStream_t st, const Batch &b) {
   }
 }
 
+template <bool SPLIT, int BX, int BY, int BZ>
+static void launch_elems(hipStream_t st, const Batch &b) {
+  const int s = b.one.s;
+  hipLaunchKernelGGL((k_elems<BX, BY, BZ, SPLIT>), dim3((s + BX - 1) / BX, (s + BY - 1) / BY, (s + BZ - 1) / BZ),
+                     dim3(ElemBlock<BX, BY, BZ, SPLIT>::THREADS), 0, st, b);
+}
+
 hipError_t launch_kernel(int id, hipStream_t st, const Batch &b) {
   switch (id) {
     case KID_NODAL:
@@ -1584,10 +1799,15 @@ hipError_t launch_kernel(int id, hipStream_t st, const Batch &b) {
       }
       break;
     case KID_KIN:
+      if (b.elems_form) break;  // part of KID_QEOS' launch
       hipLaunchKernelGGL(k_kin, dim3(b.kin_launch), dim3(KIN_CHUNK), 0, st, b);
       break;
     case KID_QEOS:
-      if (b.cost_mode)
+      if (b.elems_form == ELEMS_SMALL)
+        launch_elems<true, ELEMS_SMALL_BLOCK>(st, b);
+      else if (b.elems_form == ELEMS_MID)
+        launch_elems<false, ELEMS_MID_BLOCK>(st, b);
+      else if (b.cost_mode)
         hipLaunchKernelGGL((k_qeos<true, false>), dim3(b.qeos_launch), dim3(BLOCK), 0, st, b);
       else if (b.eblocks <= QEOS_EARLY)
         hipLaunchKernelGGL((k_qeos<false, true>), dim3(b.qeos_launch), dim3(BLOCK), 0, st, b);

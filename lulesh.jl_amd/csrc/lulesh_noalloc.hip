@@ -64,6 +64,7 @@ struct Carve {
   int eb, gb, glaunch, kin_launch, qeos_launch;
   NodalTile tile;
   NodalCut cut;
+  ElemsPlan elems;
   size_t off_nodes, off_temps, off_dtpart, off_sc, off_inst, off_eblk, off_gblk, off_gord,
       off_kin, off_qeos, bytes;
 };
@@ -93,10 +94,12 @@ Carve carve(int nx, const DeviceScratch &d) {
   }
   c.kin_launch = 8 * nx * widest;
   c.qeos_launch = qeos_launch(c.eb);
+  c.elems = elems_plan(nx, c.eb, d.cus);
+  const int parts = c.elems.parts > c.eb ? c.elems.parts : c.eb;
   size_t o = 0;
   c.off_nodes = o;  o += round_up(6 * (size_t)c.N * sizeof(double));
   c.off_temps = o;  o += round_up(7 * (size_t)c.E * sizeof(double));
-  c.off_dtpart = o; o += round_up(2 * (size_t)c.eb * sizeof(double));
+  c.off_dtpart = o; o += round_up(2 * (size_t)parts * sizeof(double));
   c.off_sc = o;     o += round_up(sizeof(DevScalars));
   c.off_inst = o;   o += round_up(sizeof(InstDesc));
   c.off_eblk = o;   o += round_up((size_t)c.eb * sizeof(int));
@@ -246,6 +249,8 @@ int run(const lulesh_device_domain *dom, double *scalars, hipStream_t st, int de
   B.one = I;
   B.ptile = plane_tile(nx);
   B.nodal_planes = nodal_planes_fit(nx, (int64_t)d.cus * d.nodal_per_cu);
+  B.elems_form = c.elems.form;
+  B.parts = c.elems.parts;
   B.nodal_wide = nodal_patch_wide(c.tile) ? 1 : 0;
   B.nodal_lead = d.cus / 8 > 1 ? d.cus / 8 : 1;
   B.sc = (DevScalars *)(base + c.off_sc);

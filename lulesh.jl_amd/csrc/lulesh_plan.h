@@ -344,6 +344,30 @@ inline std::vector<KinWork> kin_table(const std::vector<int> &s, const std::vect
   return table;
 }
 
+// How one domain runs its two element kernels: apart, or as one k_elems
+// launch of blocks of elements.  The line lies where the blocks still all
+// run at once: two workgroups of the small form, four waves each, or one of
+// the other, eight waves, are what 235 VGPRs let a CU hold.  At 256 CUs the
+// small form ends at s=32 and the other at s=40; further out the elements
+// that are computed twice cost more than the launch saved (s=34 small 29.2
+// us a cycle, mid 27.1, apart 30.4; s=48 52.4, 46.6, 43.2).
+enum ElemsForm { ELEMS_APART, ELEMS_SMALL, ELEMS_MID };
+#define ELEMS_SMALL_BLOCK 8, 4, 2
+#define ELEMS_MID_BLOCK 8, 8, 4
+inline int64_t elems_blocks(int64_t s, int bx, int by, int bz) {
+  return ((s + bx - 1) / bx) * ((s + by - 1) / by) * ((s + bz - 1) / bz);
+}
+struct ElemsPlan {
+  int form;
+  int parts;  // workgroups of the cycle's last element kernel, a (courant, hydro) pair each
+};
+inline ElemsPlan elems_plan(int s, int eblocks, int cus) {
+  const int64_t small = elems_blocks(s, ELEMS_SMALL_BLOCK), mid = elems_blocks(s, ELEMS_MID_BLOCK);
+  if (small <= 2 * (int64_t)cus) return ElemsPlan{ELEMS_SMALL, (int)small};
+  if (mid <= cus) return ElemsPlan{ELEMS_MID, (int)mid};
+  return ElemsPlan{ELEMS_APART, eblocks};
+}
+
 // k_qeos runs 256-element blocks (each writes one pair of dt partial
 // minima); XCD x takes runs of QEOS_GROUP consecutive blocks, the runs
 // dealt round-robin, so the eight XCDs sweep neighbouring addresses
