@@ -8,7 +8,7 @@ HBM; warm-up cycles run on the same context, which is then reset to the
 initial state before the timed region.
 
 Prints ONE JSON line: zone-cycles/s over the timed cycles (the production
-path: the captured one-cycle hipGraph replayed), the roofline of the
+path: captured cycles replayed as hipGraphs), the roofline of the
 dominant kernel (algorithmic bytes per launch / mean launch time from HIP
 events recorded on the context's stream over a second timed run of the
 same cycles, launched one by one) and the CPU baseline (the oracle, one
@@ -265,8 +265,8 @@ def main():
     E, N = dom.numElem, dom.numNode
     if args.warmup > 0:
         run(dom, args.warmup)
-    # timed region 1: the production path (the captured one-cycle hipGraph
-    # replayed, loop test on the device) -> value
+    # timed region 1: the production path (captured cycles replayed as
+    # hipGraphs, loop test on the device) -> value
     dom.reset()
     t0 = time.perf_counter()
     ncyc = run(dom, args.steps)

@@ -120,7 +120,7 @@ int lulesh_lagrange_elements(lulesh_ctx *ctx);
 int lulesh_calc_time_constraints(lulesh_ctx *ctx);
 /* The driver loop of examples/benchmark.jl:82-98:
  *   while time < stoptime: timeIncrement!; lagrangeLeapFrog; break if cycle >= num_iters
- * run on the device (cycles replayed from a captured hipGraph, the loop
+ * run on the device (captured cycles replayed as hipGraphs, the loop
  * condition evaluated on the device).  *cycles_run = cycles executed. */
 int lulesh_run(lulesh_ctx *ctx, int64_t num_iters, int64_t *cycles_run);
 /* verifyAndWriteFinalOutput's numbers (src/utils.jl:124-152):

@@ -63,8 +63,8 @@ struct lulesh_ctx {
   std::vector<hipEvent_t> event_pool;
   double ktime[LULESH_K_COUNT] = {0};
   int64_t kcount[LULESH_K_COUNT] = {0};
-  // driver-loop graph (one cycle of every instance)
-  hipGraphExec_t graph = nullptr;
+  // driver-loop graphs: one cycle of every instance, and kGraphCycles
+  hipGraphExec_t graph[2] = {nullptr, nullptr};
   int graph_keep_aux = -1;
   std::string last_error;
   std::vector<void *> allocations;
@@ -259,8 +259,15 @@ int dev_alloc(lulesh_ctx *c, T **p, int64_t n) {
   return 0;
 }
 
+void drop_graphs(lulesh_ctx *c) {
+  for (hipGraphExec_t &g : c->graph) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
+  }
+}
+
 void release(lulesh_ctx *c) {
-  if (c->graph) (void)hipGraphExecDestroy(c->graph);
+  drop_graphs(c);
   for (auto &p : c->pending) {
     (void)hipEventDestroy(p.a);
     (void)hipEventDestroy(p.b);
@@ -284,38 +291,46 @@ bool defer_dt(const lulesh_ctx *c) {
   return c->n == 1 && c->inst[0].ebn <= kDeferBlocks && !c->b.nodal_wide;
 }
 
-int build_graph(lulesh_ctx *c) {
+// Cycles in the longer of the driver loop's two graphs.  A graph launch
+// leaves the GPU idle for about 5 us before its first kernel; with eight
+// cycles behind one a cycle at s=16 takes 17.2 us instead of 21.7, s=30 25.0
+// instead of 29.0, s=64 62.7 instead of 67.5 (16 or 32 cycles: 0.1 us less
+// again, and their capture is paid for by every context).
+constexpr int kGraphCycles = 8;
+
+// the graph of `cycles` (1 or kGraphCycles) driver-loop cycles
+int build_graph(lulesh_ctx *c, int cycles) {
   if (!c->nodal_ready)
     return fail(c, LULESH_ERR_HIP, "k_nodal tables unavailable (a device allocation failed)");
-  if (c->graph && c->graph_keep_aux == c->keep_aux && c->graph_cost_mode == c->b.cost_mode)
-    return 0;
-  if (c->graph) {
-    (void)hipGraphExecDestroy(c->graph);
-    c->graph = nullptr;
+  if (c->graph_keep_aux != c->keep_aux || c->graph_cost_mode != c->b.cost_mode) {
+    drop_graphs(c);
+    c->graph_keep_aux = c->keep_aux;
+    c->graph_cost_mode = c->b.cost_mode;
   }
+  hipGraphExec_t &graph = c->graph[cycles > 1];
+  if (graph) return 0;
   Batch a = make_args(c, 1, 1);
   a.defer_dt = defer_dt(c);
   hipGraph_t g = nullptr;
   HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
-  for (int id : ids) {
-    if (id == KID_DT && a.defer_dt) break;
-    hipError_t e = launch_kernel(id, c->stream, a);
-    if (e != hipSuccess) {
-      (void)hipStreamEndCapture(c->stream, &g);
-      if (g) (void)hipGraphDestroy(g);
-      return hip_fail(c, e, "graph capture");
+  for (int k = 0; k < cycles; ++k)
+    for (int id : ids) {
+      if (id == KID_DT && a.defer_dt) break;
+      hipError_t e = launch_kernel(id, c->stream, a);
+      if (e != hipSuccess) {
+        (void)hipStreamEndCapture(c->stream, &g);
+        if (g) (void)hipGraphDestroy(g);
+        return hip_fail(c, e, "graph capture");
+      }
     }
-  }
   HIP_TRY(c, hipStreamEndCapture(c->stream, &g));
-  hipError_t e = hipGraphInstantiate(&c->graph, g, nullptr, nullptr, 0);
+  hipError_t e = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e != hipSuccess) {
-    c->graph = nullptr;
+    graph = nullptr;
     return hip_fail(c, e, "hipGraphInstantiate");
   }
-  c->graph_keep_aux = c->keep_aux;
-  c->graph_cost_mode = c->b.cost_mode;
   return 0;
 }
 
@@ -359,7 +374,7 @@ int order_nodal(lulesh_ctx *c, const std::vector<char> *live) {
   if ((int64_t)order.size() > c->gorder_cap) {
     // only a new plan grows the table (a live subset keeps glaunch), and a
     // new plan has already dropped the graph that holds the old pointer
-    if (c->graph) return fail(c, LULESH_ERR_HIP, "k_nodal order table would move under the graph");
+    if (c->graph[0] || c->graph[1]) return fail(c, LULESH_ERR_HIP, "k_nodal order table would move under the graph");
     c->b.gblock_order = nullptr;
     if (c->gorder) HIP_TRY(c, hipFree(c->gorder));
     c->gorder = nullptr;
@@ -398,10 +413,7 @@ int plan_nodal(lulesh_ctx *c, int cz) {
   // until the new tables are on the device, k_nodal must not run, and the
   // captured graph (which holds the old ones) is gone
   c->nodal_ready = false;
-  if (c->graph) {
-    (void)hipGraphExecDestroy(c->graph);
-    c->graph = nullptr;
-  }
+  drop_graphs(c);
   c->b.nodal_wide = 0;
   for (InstDesc &I : c->inst) {
     const NodalTile t = nodal_tile(I.s, c->tile_lo, c->tile_hi);
@@ -651,23 +663,26 @@ int run_cycles_body(lulesh_ctx *c, int64_t num_iters, int64_t *cycles_run) {
   rc = launch(c, KID_RUN_BEGIN, a);
   if (rc) return rc;
   // with timing on, kernels are launched one by one so each can carry its
-  // events; otherwise one captured cycle (all instances) is replayed
+  // events; otherwise captured cycles (all instances) are replayed
   const bool use_graph = !c->timing;
-  if (use_graph) {
-    rc = build_graph(c);
-    if (rc) return rc;
-  }
   // replay exactly the cycles num_iters still allows the least advanced
   // active instance (its first cycle always runs); only stop-time exits and
-  // unequal instances leave gated no-op replays behind
-  int64_t cap = 8;
+  // unequal instances leave gated no-op replays behind.  The first batch is
+  // of 32 cycles, as each wait for the device between batches costs about 10
+  // us (s=16, 10 cycles 246 -> 207 us against a first batch of 8), and a
+  // cycle that no longer runs costs about 6
+  int64_t cap = 32;
   long long next_cycle = min_cycle0 + 1;
   for (;;) {
     const long long left = (long long)num_iters - next_cycle + 1;
     const int64_t batch = left < 1 ? 1 : (left < cap ? left : cap);
-    for (int64_t i = 0; i < batch; ++i) {
+    for (int64_t i = 0; i < batch;) {
+      const int cycles = use_graph && batch - i >= kGraphCycles ? kGraphCycles : 1;
+      i += cycles;
       if (use_graph) {
-        HIP_TRY(c, hipGraphLaunch(c->graph, c->stream));
+        rc = build_graph(c, cycles);
+        if (rc) return rc;
+        HIP_TRY(c, hipGraphLaunch(c->graph[cycles > 1], c->stream));
       } else {
         const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
         for (int id : ids) {
