@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "lulesh_adjoint.h"
+#include "lulesh_hostcopy.h"
 #include "lulesh_kernels.h"
 #include "lulesh_regions.h"
 
@@ -49,6 +50,11 @@ struct lulesh_ctx {
   hipStream_t stream = nullptr;
   Batch b{};                      // device pointers + launch geometry
   DevScalars *hsc = nullptr;      // pinned host mirror [n]
+  HostCopy host;                  // field downloads
+  // hsc holds what the device does: set by finish() when nothing has been
+  // launched since pull_scalars, dropped by touch().  Reading a scalar then
+  // takes no copy (13 us), nor does the node-set parity of a download.
+  bool pulled = false, known = false;
   bool partials_valid = false;    // dtpart holds what the last lagrangeElements left
   int partials = 0;               // ... in so many pairs (one domain)
   int cus = 256, nodal_per_cu = 2;  // compute units; k_nodal workgroups resident per CU
@@ -151,8 +157,12 @@ hipEvent_t get_event(lulesh_ctx *c) {
   return e;
 }
 
+// before anything that may change the scalars on the device
+void touch(lulesh_ctx *c) { c->pulled = c->known = false; }
+
 // one launch on the context stream, bracketed by events when timing is on
 int launch(lulesh_ctx *c, int id, const Batch &a) {
+  touch(c);
   if (id == KID_NODAL && !c->nodal_ready)
     return fail(c, LULESH_ERR_HIP, "k_nodal tables unavailable (a device allocation failed)");
   hipEvent_t ea = nullptr, eb = nullptr;
@@ -175,6 +185,7 @@ int launch(lulesh_ctx *c, int id, const Batch &a) {
 int pull_scalars(lulesh_ctx *c) {
   HIP_TRY(c, hipMemcpyAsync(c->hsc, c->b.sc, sizeof(DevScalars) * c->n, hipMemcpyDeviceToHost,
                             c->stream));
+  c->pulled = true;
   return 0;
 }
 
@@ -186,6 +197,7 @@ int finish(lulesh_ctx *c, bool check_err) {
     if (rc) return rc;
   }
   HIP_TRY(c, hipStreamSynchronize(c->stream));
+  c->known = c->known || c->pulled;
   for (auto &p : c->pending) {
     float ms = 0.f;
     HIP_TRY(c, hipEventElapsedTime(&ms, p.a, p.b));
@@ -205,7 +217,18 @@ int finish(lulesh_ctx *c, bool check_err) {
   return 0;
 }
 
-int clear_err(lulesh_ctx *c) { return launch(c, KID_CLEAR_ERR, make_args(c, 0, 0)); }
+// the scalars in hsc, fetched only if they are not there
+int know_scalars(lulesh_ctx *c) {
+  if (c->known) return 0;
+  int rc = pull_scalars(c);
+  return rc ? rc : finish(c, false);
+}
+
+int clear_err(lulesh_ctx *c) {
+  bool clean = c->known;
+  for (int i = 0; i < c->n && clean; ++i) clean = c->hsc[i].err == ERR_NONE;
+  return clean ? 0 : launch(c, KID_CLEAR_ERR, make_args(c, 0, 0));
+}
 
 struct FieldRef {
   double *ptr;
@@ -641,17 +664,19 @@ int create(int32_t n, const int32_t *nx, const double *einit_scale, const double
 // Fetch the instance's scalars (synchronous).
 int get_inst_scalars(lulesh_ctx *c, int32_t inst, DevScalars *out) {
   HIP_TRY(c, hipSetDevice(c->device));
-  HIP_TRY(c, hipMemcpyAsync(c->hsc + inst, c->b.sc + inst, sizeof(DevScalars),
-                            hipMemcpyDeviceToHost, c->stream));
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
+  if (!c->known) {
+    HIP_TRY(c, hipMemcpyAsync(c->hsc + inst, c->b.sc + inst, sizeof(DevScalars),
+                              hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, hipStreamSynchronize(c->stream));
+    c->known = c->n == 1;
+  }
   *out = c->hsc[inst];
   return 0;
 }
 
 int run_cycles_body(lulesh_ctx *c, int64_t num_iters, int64_t *cycles_run) {
   HIP_TRY(c, hipSetDevice(c->device));
-  int rc = pull_scalars(c);
-  if (!rc) rc = finish(c, false);
+  int rc = know_scalars(c);
   if (rc) return rc;
   std::vector<long long> cycle0(c->n);
   long long min_cycle0 = 0;
@@ -682,6 +707,7 @@ int run_cycles_body(lulesh_ctx *c, int64_t num_iters, int64_t *cycles_run) {
       if (use_graph) {
         rc = build_graph(c, cycles);
         if (rc) return rc;
+        touch(c);
         HIP_TRY(c, hipGraphLaunch(c->graph[cycles > 1], c->stream));
       } else {
         const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
@@ -862,6 +888,7 @@ int adj_setup(lulesh_ctx *c, int64_t ncycles, int64_t every) {
 }
 
 int state_copy(lulesh_ctx *c, double *buf, int to_buf) {
+  touch(c);
   hipError_t e = launch_state_copy(c->stream, c->b.sc, c->b.f, c->inst[0].E, c->inst[0].N, buf,
                                    to_buf);
   return e == hipSuccess ? 0 : hip_fail(c, e, "state copy");
@@ -871,6 +898,7 @@ int state_copy(lulesh_ctx *c, double *buf, int to_buf) {
 // `state` and the next cycle's scheduled dt (each step optional; one launch)
 int slot_step(lulesh_ctx *c, double *temps, double *state, const double *dt, int64_t base) {
   const int64_t E = c->inst[0].E, N = c->inst[0].N;
+  touch(c);
   hipError_t e = launch_slot_step(c->stream, c->b.sc, c->b.f, E, N, temps, state, dt, base);
   return e == hipSuccess ? 0 : hip_fail(c, e, "slot step");
 }
@@ -940,6 +968,36 @@ int adjoint_cycle(lulesh_ctx *c, const AdjArgs &aa, bool last) {
   return 0;
 }
 
+// sum_e e * elemMass, in element order (the products formed on the host too)
+int energy_loss(lulesh_ctx *c, double *loss) {
+  const int64_t E = c->inst[0].E;
+  std::vector<double> e(E);
+  HIP_TRY(c, c->host.fetch(c->stream, e.data(), c->b.f.e, sizeof(double) * E));
+  double L = 0.0;
+  const double *pe = e.data();
+  HIP_TRY(c, c->host.stream(c->stream, c->b.f.elemMass, 1, E, [&](const double *v, int64_t, int64_t m) {
+    for (int64_t i = 0; i < m; ++i) L += pe[i] * v[i];
+    pe += m;
+  }));
+  if (loss) *loss = L;
+  return 0;
+}
+
+// the parameter gradients: each the sum of its elements' shares in element order
+int param_sums(lulesh_ctx *c, double (&sum)[3]) {
+  double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+  HIP_TRY(c, c->host.stream(c->stream, c->adj.a.pacc, 3, c->inst[0].E,
+                            [&](const double *v, int64_t stride, int64_t m) {
+    for (int64_t i = 0; i < m; ++i) {
+      a0 += v[i];
+      a1 += v[i + stride];
+      a2 += v[i + 2 * stride];
+    }
+  }));
+  sum[0] = a0; sum[1] = a1; sum[2] = a2;
+  return 0;
+}
+
 // The gradient run's forward pass: `ncycles` cycles of the driver loop from
 // the current state with timeIncrement! recording each dt; the start state
 // of cycle k is saved into save(k) when that is not null, and from cycle
@@ -982,15 +1040,9 @@ int grad_forward(lulesh_ctx *c, int64_t ncycles, long long cycle0, Save save, in
   if (!rc && slot_from < ncycles) rc = slot_step(c, nullptr, seg_slot(c, ncycles - slot_from), nullptr, 0);
   if (!rc) rc = finish(c, true);
   if (rc) return rc;
-  if (dt_out) HIP_TRY(c, hipMemcpy(dt_out, B.dt, sizeof(double) * ncycles, hipMemcpyDeviceToHost));
-  {
-    std::vector<double> ev(E), mv(E);
-    HIP_TRY(c, hipMemcpy(ev.data(), c->b.f.e, sizeof(double) * E, hipMemcpyDeviceToHost));
-    HIP_TRY(c, hipMemcpy(mv.data(), c->b.f.elemMass, sizeof(double) * E, hipMemcpyDeviceToHost));
-    double L = 0.0;
-    for (int64_t i = 0; i < E; ++i) L += ev[i] * mv[i];
-    if (loss) *loss = L;
-  }
+  if (dt_out) HIP_TRY(c, c->host.fetch(c->stream, dt_out, B.dt, sizeof(double) * ncycles));
+  rc = energy_loss(c, loss);
+  if (rc) return rc;
   rc = state_copy(c, B.final_state, 1);
   if (rc) return rc;
   HIP_TRY(c, hipMemcpyAsync(B.final_sc, c->b.sc, sizeof(DevScalars), hipMemcpyDeviceToDevice, c->stream));
@@ -1003,17 +1055,14 @@ int grad_forward(lulesh_ctx *c, int64_t ncycles, long long cycle0, Save save, in
 int grad_results(lulesh_ctx *c, double *grad_e, double grad_params[3]) {
   AdjBuffers &B = c->adj;
   const int64_t E = c->inst[0].E;
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
-  if (grad_e) HIP_TRY(c, hipMemcpy(grad_e, B.a.le, sizeof(double) * E, hipMemcpyDeviceToHost));
+  if (grad_e) HIP_TRY(c, c->host.fetch(c->stream, grad_e, B.a.le, sizeof(double) * E));
   if (grad_params) {
-    std::vector<double> pa(3 * E);
-    HIP_TRY(c, hipMemcpy(pa.data(), B.a.pacc, sizeof(double) * 3 * E, hipMemcpyDeviceToHost));
-    for (int k = 0; k < 3; ++k) {
-      double sum = 0.0;
-      for (int64_t i = 0; i < E; ++i) sum += pa[k * E + i];
-      grad_params[k] = sum;
-    }
+    double sum[3];
+    int r = param_sums(c, sum);
+    if (r) return r;
+    for (int k = 0; k < 3; ++k) grad_params[k] = sum[k];
   }
+  touch(c);
   HIP_TRY(c, hipMemcpyAsync(c->b.sc, B.final_sc, sizeof(DevScalars), hipMemcpyDeviceToDevice, c->stream));
   int rc = state_copy(c, B.final_state, 0);
   if (!rc) rc = finish(c, false);
@@ -1030,8 +1079,7 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
   if (rc) return rc;
   AdjBuffers &B = c->adj;
   const int64_t E = c->inst[0].E, N = c->inst[0].N, state = 6 * N + 5 * E;
-  rc = pull_scalars(c);
-  if (!rc) rc = finish(c, false);
+  rc = know_scalars(c);
   if (rc) return rc;
   const long long cycle0 = c->hsc[0].cycle;
   // 1. forward pass: checkpoints every `every` cycles, dt schedule recorded,
@@ -1046,13 +1094,14 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
   // replay it storing each cycle's start state and temporaries, then run
   // the adjoint kernels of its cycles backwards against the stored slots
   std::vector<double> hdt(ncycles);
-  HIP_TRY(c, hipMemcpy(hdt.data(), B.dt, sizeof(double) * ncycles, hipMemcpyDeviceToHost));
+  HIP_TRY(c, c->host.fetch(c->stream, hdt.data(), B.dt, sizeof(double) * ncycles));
   for (int64_t sg = nseg - 1; sg >= 0 && !rc; --sg) {
     const int64_t k0 = sg * every, k1 = (k0 + every < ncycles) ? k0 + every : ncycles;
     const int64_t L = k1 - k0;
     if (sg < nseg - 1) {
       rc = state_copy(c, B.ckpt + sg * state, 0);
       if (!rc) {
+        touch(c);
         hipError_t e = launch_set_cycle(c->stream, c->b.sc, cycle0 + k0);
         if (e != hipSuccess) rc = hip_fail(c, e, "set cycle");
       }
@@ -1107,6 +1156,7 @@ struct Revolve {
     if (i < 0) return fail(c, LULESH_ERR_HIP, "revolve: missing saved state");
     int rc = state_copy(c, buf(i), 0);
     if (rc) return rc;
+    touch(c);
     hipError_t e = launch_set_cycle(c->stream, c->b.sc, cycle0 + k);
     if (e != hipSuccess) return hip_fail(c, e, "set cycle");
     cur = k;
@@ -1146,20 +1196,15 @@ struct Revolve {
   // the forward pass has reached the end: errors, loss, end state, dt record
   int end_of_forward() {
     AdjBuffers &B = c->adj;
-    const int64_t E = c->inst[0].E;
     int rc = finish(c, true);
     if (rc) return rc;
-    std::vector<double> ev(E), mv(E);
-    HIP_TRY(c, hipMemcpy(ev.data(), c->b.f.e, sizeof(double) * E, hipMemcpyDeviceToHost));
-    HIP_TRY(c, hipMemcpy(mv.data(), c->b.f.elemMass, sizeof(double) * E, hipMemcpyDeviceToHost));
-    double L = 0.0;
-    for (int64_t i = 0; i < E; ++i) L += ev[i] * mv[i];
-    if (loss) *loss = L;
+    rc = energy_loss(c, loss);
+    if (rc) return rc;
     rc = state_copy(c, B.final_state, 1);
     if (rc) return rc;
     HIP_TRY(c, hipMemcpyAsync(B.final_sc, c->b.sc, sizeof(DevScalars), hipMemcpyDeviceToDevice,
                               c->stream));
-    HIP_TRY(c, hipMemcpy(hdt.data(), B.dt, sizeof(double) * n, hipMemcpyDeviceToHost));
+    HIP_TRY(c, c->host.fetch(c->stream, hdt.data(), B.dt, sizeof(double) * n));
     return 0;
   }
   // cycle k forward with its start state and temporaries kept, then its
@@ -1192,8 +1237,7 @@ int grad_run_revolve(lulesh_ctx *c, int64_t ncycles, int64_t snapshots, double *
   HIP_TRY(c, hipSetDevice(c->device));
   int rc = adj_setup_n(c, ncycles, snapshots, 1);
   if (rc) return rc;
-  rc = pull_scalars(c);
-  if (!rc) rc = finish(c, false);
+  rc = know_scalars(c);
   if (rc) return rc;
   Revolve R;
   R.c = c;
@@ -1246,17 +1290,13 @@ int vjp_cycle(lulesh_ctx *c, double grad_params[3]) {
   rc = adjoint_cycle(c, stored_args(c, seg_slot(c, 0), seg_slot(c, 1), c->hsc[0].deltatime, 0),
                      true);
   if (rc) return rc;
-  HIP_TRY(c, hipStreamSynchronize(c->stream));
   if (grad_params) {
-    std::vector<double> pa(3 * E);
-    HIP_TRY(c, hipMemcpy(pa.data(), B.a.pacc, sizeof(double) * 3 * E, hipMemcpyDeviceToHost));
-    for (int k = 0; k < 3; ++k) {
-      double sum = 0.0;
-      for (int64_t i = 0; i < E; ++i) sum += pa[k * E + i];
-      grad_params[k] += sum;
-    }
+    double sum[3];
+    rc = param_sums(c, sum);
+    if (rc) return rc;
+    for (int k = 0; k < 3; ++k) grad_params[k] += sum[k];
   }
-  return 0;
+  return finish(c, false);
 }
 
 // shadow buffer of one state field, or nullptr
@@ -1290,8 +1330,8 @@ int shadow_move(lulesh_ctx *c, const char *field, double *host, int64_t n, bool 
   double *p = shadow_field(c, field, &len);
   if (!p) return fail(c, LULESH_ERR_INVALID_ARG, std::string("no shadow for field ") + (field ? field : "(null)"));
   if (n != len) return fail(c, LULESH_ERR_INVALID_ARG, "shadow field length mismatch");
-  if (up) HIP_TRY(c, hipMemcpy(p, host, sizeof(double) * n, hipMemcpyHostToDevice));
-  else HIP_TRY(c, hipMemcpy(host, p, sizeof(double) * n, hipMemcpyDeviceToHost));
+  if (up) HIP_TRY(c, c->host.send(c->stream, p, host, sizeof(double) * n));
+  else HIP_TRY(c, c->host.fetch(c->stream, host, p, sizeof(double) * n));
   return 0;
 }
 
@@ -1380,8 +1420,7 @@ int lulesh_replay(lulesh_ctx *c, const double *dt, int64_t ncycles) {
     int rc = adj_setup(c, ncycles > 0 ? ncycles : 1, 0);
     if (rc) return rc;
     HIP_TRY(c, hipMemcpy(c->adj.dt, dt, sizeof(double) * ncycles, hipMemcpyHostToDevice));
-    rc = pull_scalars(c);
-    if (!rc) rc = finish(c, false);
+    rc = know_scalars(c);
     if (rc) return rc;
     const long long cycle0 = c->hsc[0].cycle;
     rc = clear_err(c);
@@ -1447,10 +1486,12 @@ int lulesh_reset(lulesh_ctx *c) {
   try {
     if (!c) return LULESH_ERR_INVALID_ARG;
     HIP_TRY(c, hipSetDevice(c->device));
+    touch(c);
     hipError_t e = launch_init(c->stream, c->b);
     if (e != hipSuccess) return hip_fail(c, e, "init kernels");
     c->partials_valid = false;
-    return finish(c, false);
+    int rc = pull_scalars(c);
+    return rc ? rc : finish(c, false);
   } catch (...) {
     return exception_status(c);
   }
@@ -1477,7 +1518,7 @@ int lulesh_batch_download(lulesh_ctx *c, int32_t inst, const char *field, double
     FieldRef r = find_field(c, inst, field, s.parity);
     if (!r.ptr) return fail(c, LULESH_ERR_INVALID_ARG, std::string("unknown field ") + (field ? field : "(null)"));
     if (n != r.n) return fail(c, LULESH_ERR_INVALID_ARG, "field length mismatch");
-    HIP_TRY(c, hipMemcpyAsync(dst, r.ptr, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, c->host.fetch(c->stream, dst, r.ptr, (size_t)n * sizeof(double)));
     return finish(c, false);
   } catch (...) {
     return exception_status(c);
@@ -1495,7 +1536,7 @@ int lulesh_batch_upload(lulesh_ctx *c, int32_t inst, const char *field, const do
     FieldRef r = find_field(c, inst, field, s.parity);
     if (!r.ptr) return fail(c, LULESH_ERR_INVALID_ARG, std::string("unknown field ") + (field ? field : "(null)"));
     if (n != r.n) return fail(c, LULESH_ERR_INVALID_ARG, "field length mismatch");
-    HIP_TRY(c, hipMemcpyAsync(r.ptr, src, (size_t)n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, c->host.send(c->stream, r.ptr, src, (size_t)n * sizeof(double)));
     c->partials_valid = false;
     return finish(c, false);
   } catch (...) {
@@ -1524,8 +1565,7 @@ int lulesh_batch_download_elem_bc(lulesh_ctx *c, int32_t inst, uint32_t *dst, in
     if (rc) return rc;
     if (!dst || n != c->inst[inst].E) return fail(c, LULESH_ERR_INVALID_ARG, "elemBC length mismatch");
     HIP_TRY(c, hipSetDevice(c->device));
-    HIP_TRY(c, hipMemcpyAsync(dst, c->b.f.elemBC + c->inst[inst].e0, (size_t)n * 4,
-                              hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, c->host.fetch(c->stream, dst, c->b.f.elemBC + c->inst[inst].e0, (size_t)n * 4));
     return finish(c, false);
   } catch (...) {
     return exception_status(c);
@@ -1538,8 +1578,7 @@ int lulesh_batch_upload_elem_bc(lulesh_ctx *c, int32_t inst, const uint32_t *src
     if (rc) return rc;
     if (!src || n != c->inst[inst].E) return fail(c, LULESH_ERR_INVALID_ARG, "elemBC length mismatch");
     HIP_TRY(c, hipSetDevice(c->device));
-    HIP_TRY(c, hipMemcpyAsync(c->b.f.elemBC + c->inst[inst].e0, src, (size_t)n * 4,
-                              hipMemcpyHostToDevice, c->stream));
+    HIP_TRY(c, c->host.send(c->stream, c->b.f.elemBC + c->inst[inst].e0, src, (size_t)n * 4));
     return finish(c, false);
   } catch (...) {
     return exception_status(c);
@@ -1601,11 +1640,15 @@ int lulesh_batch_set_scalar(lulesh_ctx *c, int32_t inst, const char *name, doubl
       if (!slot) return fail(c, LULESH_ERR_INVALID_ARG, "unknown scalar " + nm);
       *slot = value;
     }
+    const bool known = c->known;
+    touch(c);
     c->hsc[inst] = s;
     HIP_TRY(c, hipMemcpyAsync(c->b.sc + inst, c->hsc + inst, sizeof(DevScalars),
                               hipMemcpyHostToDevice, c->stream));
     c->partials_valid = false;
-    return finish(c, false);
+    rc = finish(c, false);
+    c->known = known && !rc;
+    return rc;
   } catch (...) {
     return exception_status(c);
   }
@@ -1705,6 +1748,7 @@ int lulesh_time_increment(lulesh_ctx *c) {
     if (!c) return LULESH_ERR_INVALID_ARG;
     HIP_TRY(c, hipSetDevice(c->device));
     int rc = launch(c, KID_TIME_INCREMENT, make_args(c, 0, 0));
+    if (!rc) rc = pull_scalars(c);  // the caller's loop test reads them
     if (rc) return rc;
     return finish(c, false);
   } catch (...) {
@@ -1814,8 +1858,7 @@ int lulesh_batch_verify(lulesh_ctx *c, int32_t inst, double out[4]) {
     const int64_t nx = c->inst[inst].s;
     std::vector<double> e(nx * nx);
     HIP_TRY(c, hipSetDevice(c->device));
-    HIP_TRY(c, hipMemcpyAsync(e.data(), c->b.f.e + c->inst[inst].e0, e.size() * sizeof(double),
-                              hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(c, c->host.fetch(c->stream, e.data(), c->b.f.e + c->inst[inst].e0, e.size() * sizeof(double)));
     rc = finish(c, false);
     if (rc) return rc;
     // src/utils.jl:134-152
@@ -1946,10 +1989,10 @@ int lulesh_autotune(lulesh_ctx *c, int32_t *chosen, double *best_ms) {
     // the tuning launches may raise an error code the live state would
     // raise on its next cycle; the scalars are put back as they were, so
     // an error already on the device survives and a new one does not appear
-    int rc = pull_scalars(c);
-    if (!rc) rc = finish(c, false);
+    int rc = know_scalars(c);
     if (rc) return rc;
     const std::vector<DevScalars> saved(c->hsc, c->hsc + c->n);
+    touch(c);
     int best_f = -1, best_cz = -1;
     float best_t = 0.f;
     hipEvent_t ea = get_event(c), eb = get_event(c);
