@@ -33,15 +33,6 @@ enum AdjKernel { AK_QEOS = 0, AK_KIN, AK_NODE1, AK_FORCE, AK_NODE2, AK_SEED };
 hipError_t launch_adjoint(int which, hipStream_t st, const AdjArgs &a);
 hipError_t launch_state_copy(hipStream_t st, DevScalars *sc, const DevFields &f, int64_t E,
                              int64_t N, double *buf, int to_buf);
-// Between two cycles of a segment replay, in one launch: the temporaries of
-// the cycle just run (vnew delv vdov delx_xi delx_eta delx_zeta delv_xi
-// delv_eta delv_zeta, 9E) into `temps` (if non-null), the current state
-// (x y z xd yd zd of the current node set, 6N, then e p q v ss, 5E) into
-// `state` (if non-null), and, with `dt` non-null, the next cycle's time step
-// dt[cycle - base] with timeIncrement!'s time/cycle bookkeeping.
-hipError_t launch_slot_step(hipStream_t st, DevScalars *sc, const DevFields &f, int64_t E,
-                            int64_t N, double *temps, double *state, const double *dt,
-                            int64_t base);
 hipError_t launch_set_cycle(hipStream_t st, DevScalars *sc, long long cycle);
 
 }  // namespace lulesh

@@ -1,7 +1,7 @@
 // Adjoint kernels of one LULESH cycle on gfx950 (reverse of k_nodal ->
 // k_kin -> k_qeos with the cycle's dt held fixed).
 //
-// The kernels read cycle c from a stored slot (AdjArgs): its start state
+// The kernels read cycle c from where it ran (AdjArgs): its start state
 // S_c = (x y z xd yd zd, e p q v ss), the node set after it (x', xd') and its
 // temporaries (vnew delv vdov delx_* delv_*), all kept when the forward
 // cycle ran.  On entry the adjoint buffers hold the adjoint of S_{c+1}; on
@@ -431,36 +431,6 @@ __global__ __launch_bounds__(BLOCK) void a_state_copy(DevScalars *sc, DevFields 
     }
 }
 
-__global__ __launch_bounds__(BLOCK) void a_slot_step(DevScalars *sc, DevFields f, int64_t E,
-                                                     int64_t N, double *temps, double *state,
-                                                     const double *dt, int64_t base) {
-  const int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-  const int par = sc->parity;
-  if (temps && i < E) {
-    const double *el[9] = {f.vnew, f.delv, f.vdov, f.delx_xi, f.delx_eta, f.delx_zeta,
-                           f.delv_xi, f.delv_eta, f.delv_zeta};
-    for (int k = 0; k < 9; ++k) temps[k * E + i] = el[k][i];
-  }
-  if (state) {
-    if (i < N) {
-      const double *nd[6] = {par ? f.ns[1].x : f.ns[0].x, par ? f.ns[1].y : f.ns[0].y,
-                             par ? f.ns[1].z : f.ns[0].z, par ? f.ns[1].xd : f.ns[0].xd,
-                             par ? f.ns[1].yd : f.ns[0].yd, par ? f.ns[1].zd : f.ns[0].zd};
-      for (int k = 0; k < 6; ++k) state[k * N + i] = nd[k][i];
-    }
-    if (i < E) {
-      const double *el[5] = {f.e, f.p, f.q, f.v, f.ss};
-      for (int k = 0; k < 5; ++k) state[6 * N + k * E + i] = el[k][i];
-    }
-  }
-  if (dt && i == 0) {
-    const double d = dt[sc->cycle - base];
-    sc->deltatime = d;
-    sc->time = sc->time + d;
-    sc->cycle = sc->cycle + 1;
-  }
-}
-
 __global__ void a_set_cycle(DevScalars *sc, long long cycle) {
   if (threadIdx.x == 0 && blockIdx.x == 0) sc->cycle = cycle;
 }
@@ -504,14 +474,6 @@ hipError_t launch_state_copy(hipStream_t st, DevScalars *sc, const DevFields &f,
                              int64_t N, double *buf, int to_buf) {
   hipLaunchKernelGGL(a_state_copy, dim3(nblk_a(N > E ? N : E)), dim3(BLOCK), 0, st, sc, f, E, N,
                      buf, to_buf);
-  return hipGetLastError();
-}
-
-hipError_t launch_slot_step(hipStream_t st, DevScalars *sc, const DevFields &f, int64_t E,
-                            int64_t N, double *temps, double *state, const double *dt,
-                            int64_t base) {
-  hipLaunchKernelGGL(a_slot_step, dim3(nblk_a(N > E ? N : E)), dim3(BLOCK), 0, st, sc, f, E, N,
-                     temps, state, dt, base);
   return hipGetLastError();
 }
 

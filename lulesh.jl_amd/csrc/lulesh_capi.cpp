@@ -621,6 +621,7 @@ int create(int32_t n, const int32_t *nx, const double *einit_scale, const double
   for (double **p : nf)
     if (!rc) rc = dev_alloc(c, p, n0);
   if (!rc) rc = dev_alloc(c, &f.elemBC, e0);
+  B.out = ElemState{f.e, f.p, f.q, f.v, f.ss};
   int64_t parts = eb;
   if (n == 1) parts = std::max<int64_t>(parts, elems_plan(c->inst[0].s, eb, c->cus).parts);
   if (!rc) rc = dev_alloc(c, &B.dtpart, 2 * parts);
@@ -894,34 +895,59 @@ int state_copy(lulesh_ctx *c, double *buf, int to_buf) {
   return e == hipSuccess ? 0 : hip_fail(c, e, "state copy");
 }
 
-// temporaries of the cycle just run into `temps`, the current state into
-// `state` and the next cycle's scheduled dt (each step optional; one launch)
-int slot_step(lulesh_ctx *c, double *temps, double *state, const double *dt, int64_t base) {
-  const int64_t E = c->inst[0].E, N = c->inst[0].N;
-  touch(c);
-  hipError_t e = launch_slot_step(c->stream, c->b.sc, c->b.f, E, N, temps, state, dt, base);
-  return e == hipSuccess ? 0 : hip_fail(c, e, "slot step");
-}
-
 // slot j of the segment buffer; its temporaries follow the 6N + 5E state
 double *seg_slot(lulesh_ctx *c, int64_t j) { return c->adj.seg + j * cycle_slot(c); }
 double *slot_temps(lulesh_ctx *c, double *slot) {
   return slot + 6 * c->inst[0].N + 5 * c->inst[0].E;
 }
 
-// cycle arguments whose temporaries (vnew delv vdov delx_* delv_*) are
-// written straight into a slot, in the slot's order, instead of being
-// copied there after the cycle
-Batch into_slot(lulesh_ctx *c, Batch a, double *slot) {
+// the state before or after a cycle, wherever it lies: in the context's own
+// arrays (its current node set), or in a slot of the segment buffer
+struct StateRef {
+  NodeSet n;
+  ElemState el;
+};
+StateRef slot_state(lulesh_ctx *c, double *slot) {
+  const int64_t E = c->inst[0].E, N = c->inst[0].N;
+  double *p = slot, *el = slot + 6 * N;
+  return StateRef{NodeSet{p, p + N, p + 2 * N, p + 3 * N, p + 4 * N, p + 5 * N},
+                  ElemState{el, el + E, el + 2 * E, el + 3 * E, el + 4 * E}};
+}
+StateRef own_state(lulesh_ctx *c, int parity) { return StateRef{c->b.f.ns[parity & 1], c->b.out}; }
+
+// where the cycle leaves vnew delv vdov delx_* delv_* (null: where f says)
+void set_temps(lulesh_ctx *c, DevFields &f, double *t) {
+  if (!t) return;
   const int64_t E = c->inst[0].E;
-  double *t = slot_temps(c, slot);
-  a.f.vnew = t; a.f.delv = t + E; a.f.vdov = t + 2 * E;
-  a.f.delx_xi = t + 3 * E; a.f.delx_eta = t + 4 * E; a.f.delx_zeta = t + 5 * E;
-  a.f.delv_xi = t + 6 * E; a.f.delv_eta = t + 7 * E; a.f.delv_zeta = t + 8 * E;
+  f.vnew = t; f.delv = t + E; f.vdov = t + 2 * E;
+  f.delx_xi = t + 3 * E; f.delx_eta = t + 4 * E; f.delx_zeta = t + 5 * E;
+  f.delv_xi = t + 6 * E; f.delv_eta = t + 7 * E; f.delv_zeta = t + 8 * E;
+}
+
+// The cycle `a` from the state at `from` to the one at `to`, its temporaries
+// in `temps`: a cycle whose start state is to be kept writes the next state
+// beside it, and nothing is copied (the copies were a launch of 7 us and a
+// gap of 4 before each cycle of 44 at s=48).  parity: sc->parity at its start.
+Batch between(lulesh_ctx *c, Batch a, const StateRef &from, const StateRef &to, double *temps, int parity) {
+  a.f.ns[parity & 1] = from.n;
+  a.f.ns[(parity & 1) ^ 1] = to.n;
+  a.f.e = from.el.e; a.f.p = from.el.p; a.f.q = from.el.q; a.f.v = from.el.v; a.f.ss = from.el.ss;
+  a.out = to.el;
+  set_temps(c, a.f, temps);
+  return a;
+}
+// ... from slot j of the segment to slot j + 1
+Batch between_slots(lulesh_ctx *c, const Batch &a, int64_t j, int parity) {
+  return between(c, a, slot_state(c, seg_slot(c, j)), slot_state(c, seg_slot(c, j + 1)),
+                 slot_temps(c, seg_slot(c, j)), parity);
+}
+// ... with the recorded time step (timeIncrement! replaced)
+Batch scheduled(Batch a, double dt) {
+  a.scheduled = 1;
+  a.dt = dt;
   return a;
 }
 
-// the cycle after the scheduled dt was set (timeIncrement! replaced)
 int cycle_body(lulesh_ctx *c, bool constraints, const Batch &a) {
   const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
   for (int id : ids) {
@@ -931,28 +957,23 @@ int cycle_body(lulesh_ctx *c, bool constraints, const Batch &a) {
   }
   return 0;
 }
-int cycle_body(lulesh_ctx *c, bool constraints) {
-  return cycle_body(c, constraints, make_args(c, 0, 0));
-}
 
-// adjoint kernel arguments reading cycle k from its stored slot (start
-// state + temporaries) and the next slot (node set after the cycle)
-AdjArgs stored_args(lulesh_ctx *c, double *slot, double *next, double dt, int force_pending) {
-  const int64_t E = c->inst[0].E, N = c->inst[0].N;
+// adjoint kernel arguments of the cycle that ran from `from` (start state and
+// temporaries) to the node set `after`
+AdjArgs stored_args(lulesh_ctx *c, const StateRef &from, double *temps, const NodeSet &after, double dt,
+                    int force_pending) {
   AdjArgs a = c->adj.a;
-  double *p = slot;
-  a.old = NodeSet{p, p + N, p + 2 * N, p + 3 * N, p + 4 * N, p + 5 * N};
-  double *el = p + 6 * N;
-  a.f.e = el; a.f.p = el + E; a.f.q = el + 2 * E; a.f.v = el + 3 * E; a.f.ss = el + 4 * E;
-  double *t = el + 5 * E;
-  a.f.vnew = t; a.f.delv = t + E; a.f.vdov = t + 2 * E;
-  a.f.delx_xi = t + 3 * E; a.f.delx_eta = t + 4 * E; a.f.delx_zeta = t + 5 * E;
-  a.f.delv_xi = t + 6 * E; a.f.delv_eta = t + 7 * E; a.f.delv_zeta = t + 8 * E;
-  double *nw = next;
-  a.cur = NodeSet{nw, nw + N, nw + 2 * N, nw + 3 * N, nw + 4 * N, nw + 5 * N};
+  a.old = from.n;
+  a.f.e = from.el.e; a.f.p = from.el.p; a.f.q = from.el.q; a.f.v = from.el.v; a.f.ss = from.el.ss;
+  set_temps(c, a.f, temps);
+  a.cur = after;
   a.dt = dt;
   a.force_pending = force_pending;
   return a;
+}
+AdjArgs stored_slots(lulesh_ctx *c, int64_t j, double dt, int force_pending) {
+  return stored_args(c, slot_state(c, seg_slot(c, j)), slot_temps(c, seg_slot(c, j)),
+                     slot_state(c, seg_slot(c, j + 1)).n, dt, force_pending);
 }
 
 // one cycle's adjoint kernels; a_node1 first folds in the force corners
@@ -1011,6 +1032,7 @@ int grad_forward(lulesh_ctx *c, int64_t ncycles, long long cycle0, Save save, in
                  double *loss, double *dt_out) {
   AdjBuffers &B = c->adj;
   const int64_t E = c->inst[0].E;
+  const int parity0 = c->hsc[0].parity;
   const Batch a = make_args(c, 0, 0);
   Batch ta = a;  // timeIncrement! that also records the dt it takes
   ta.dt_record = B.dt;
@@ -1025,19 +1047,16 @@ int grad_forward(lulesh_ctx *c, int64_t ncycles, long long cycle0, Save save, in
   for (int64_t k = 0; k < ncycles && !rc; ++k) {
     double *buf = save(k);
     if (buf) rc = state_copy(c, buf, 1);
-    Batch ak = a, dk = k + 1 < ncycles ? da : a;
-    if (!rc && k >= slot_from) {
-      double *slot = seg_slot(c, k - slot_from);
-      rc = slot_step(c, nullptr, slot, nullptr, 0);
-      ak = into_slot(c, ak, slot);
-      dk = into_slot(c, dk, slot);
-    }
+    const Batch &dk = k + 1 < ncycles ? da : a;
+    Batch ak = a;
+    if (!rc && k == slot_from) rc = state_copy(c, seg_slot(c, 0), 1);
+    if (k >= slot_from) ak = between_slots(c, a, k - slot_from, parity0 + (int)(k & 1));
     const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS};
     for (int id : ids)
       if (!rc) rc = launch(c, id, ak);
     if (!rc) rc = launch(c, KID_DT, dk);
   }
-  if (!rc && slot_from < ncycles) rc = slot_step(c, nullptr, seg_slot(c, ncycles - slot_from), nullptr, 0);
+  if (!rc && slot_from < ncycles) rc = state_copy(c, seg_slot(c, ncycles - slot_from), 0);
   if (!rc) rc = finish(c, true);
   if (rc) return rc;
   if (dt_out) HIP_TRY(c, c->host.fetch(c->stream, dt_out, B.dt, sizeof(double) * ncycles));
@@ -1082,6 +1101,7 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
   rc = know_scalars(c);
   if (rc) return rc;
   const long long cycle0 = c->hsc[0].cycle;
+  int parity = c->hsc[0].parity + (int)(ncycles & 1);  // after the forward pass
   // 1. forward pass: checkpoints every `every` cycles, dt schedule recorded,
   // the last segment's slots filled on the way
   const int64_t nseg = (ncycles + every - 1) / every;
@@ -1091,33 +1111,23 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
       (nseg - 1) * every, loss, dt_out);
   if (rc) return rc;
   // 2. reverse sweep, segment by segment: restore the segment's checkpoint,
-  // replay it storing each cycle's start state and temporaries, then run
-  // the adjoint kernels of its cycles backwards against the stored slots
+  // replay it from slot to slot, then run the adjoint kernels of its cycles
+  // backwards against the stored slots
   std::vector<double> hdt(ncycles);
   HIP_TRY(c, c->host.fetch(c->stream, hdt.data(), B.dt, sizeof(double) * ncycles));
   for (int64_t sg = nseg - 1; sg >= 0 && !rc; --sg) {
     const int64_t k0 = sg * every, k1 = (k0 + every < ncycles) ? k0 + every : ncycles;
     const int64_t L = k1 - k0;
     if (sg < nseg - 1) {
-      rc = state_copy(c, B.ckpt + sg * state, 0);
-      if (!rc) {
-        touch(c);
-        hipError_t e = launch_set_cycle(c->stream, c->b.sc, cycle0 + k0);
-        if (e != hipSuccess) rc = hip_fail(c, e, "set cycle");
-      }
-      // slot j <- S_{k0+j}, dt, cycle; the cycle writes its temporaries there
+      HIP_TRY(c, hipMemcpyAsync(seg_slot(c, 0), B.ckpt + sg * state, sizeof(double) * state,
+                                hipMemcpyDeviceToDevice, c->stream));
       const Batch a = make_args(c, 0, 0);
-      for (int64_t j = 0; j < L && !rc; ++j) {
-        rc = slot_step(c, nullptr, seg_slot(c, j), B.dt, cycle0);
-        if (!rc) rc = cycle_body(c, false, into_slot(c, a, seg_slot(c, j)));
-      }
-      if (!rc) rc = slot_step(c, nullptr, seg_slot(c, L), nullptr, 0);
+      for (int64_t j = 0; j < L && !rc; ++j, ++parity)
+        rc = cycle_body(c, false, scheduled(between_slots(c, a, j, parity), hdt[k0 + j]));
     }
     for (int64_t j = L - 1; j >= 0 && !rc; --j) {
       const int64_t k = k0 + j;
-      rc = adjoint_cycle(
-          c, stored_args(c, seg_slot(c, j), seg_slot(c, j + 1), hdt[k], k == ncycles - 1 ? 0 : 1),
-          k == 0);
+      rc = adjoint_cycle(c, stored_slots(c, j, hdt[k], k == ncycles - 1 ? 0 : 1), k == 0);
     }
   }
   if (rc) return rc;
@@ -1140,6 +1150,7 @@ struct Revolve {
   int64_t frontier = 0;      // first cycle not run yet (its dt not recorded)
   int64_t cur = -1;          // cycle whose start state the context holds (-1: other)
   int64_t forward = 0;       // cycles run
+  int parity = 0;            // sc->parity, which every cycle flips
   double *loss = nullptr;
   double *buf(int i) {
     const int64_t E = c->inst[0].E, N = c->inst[0].N;
@@ -1162,28 +1173,24 @@ struct Revolve {
     cur = k;
     return 0;
   }
-  // one cycle from the current state: the first time with timeIncrement!
-  // recording its dt and the time constraints, after that at the recorded
-  // dt (state_slot: where to keep the start state, or null)
-  int step(int64_t k, double *state_slot) {
+  // cycle k as `b` places it: the first time with timeIncrement! recording
+  // its dt and the time constraints, after that at the recorded dt
+  int step(int64_t k, const Batch &b) {
     int rc = 0;
     if (k == frontier) {
-      if (state_slot) rc = slot_step(c, nullptr, state_slot, nullptr, 0);
-      if (!rc) rc = launch(c, KID_TIME_INCREMENT, ta);
-      const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
-      for (int id : ids)
-        if (!rc) rc = launch(c, id, a);
+      rc = launch(c, KID_TIME_INCREMENT, ta);
+      if (!rc) rc = cycle_body(c, true, b);
       ++frontier;
     } else {
-      rc = slot_step(c, nullptr, state_slot, c->adj.dt, cycle0);
-      if (!rc) rc = cycle_body(c, false);
+      rc = cycle_body(c, false, scheduled(b, hdt[k]));
     }
     ++forward;
+    ++parity;
     return rc;
   }
   int advance(int64_t from, int64_t to) {
     int rc = restore(from);
-    for (int64_t k = from; k < to && !rc; ++k) rc = step(k, nullptr);
+    for (int64_t k = from; k < to && !rc; ++k) rc = step(k, a);
     cur = to;
     return rc;
   }
@@ -1193,30 +1200,34 @@ struct Revolve {
     pos[i] = k;
     return state_copy(c, buf(i), 1);
   }
-  // the forward pass has reached the end: errors, loss, end state, dt record
+  // the forward pass has reached the end: errors, dt record, and with the
+  // context's own arrays holding the end state its loss and a copy of it
   int end_of_forward() {
     AdjBuffers &B = c->adj;
-    int rc = finish(c, true);
+    int rc = state_copy(c, seg_slot(c, 1), 0);
+    if (!rc) rc = finish(c, true);
+    if (!rc) rc = energy_loss(c, loss);
     if (rc) return rc;
-    rc = energy_loss(c, loss);
-    if (rc) return rc;
-    rc = state_copy(c, B.final_state, 1);
-    if (rc) return rc;
+    const size_t state = (size_t)(6 * c->inst[0].N + 5 * c->inst[0].E);
+    HIP_TRY(c, hipMemcpyAsync(B.final_state, seg_slot(c, 1), sizeof(double) * state, hipMemcpyDeviceToDevice,
+                              c->stream));
     HIP_TRY(c, hipMemcpyAsync(B.final_sc, c->b.sc, sizeof(DevScalars), hipMemcpyDeviceToDevice,
                               c->stream));
     HIP_TRY(c, c->host.fetch(c->stream, hdt.data(), B.dt, sizeof(double) * n));
     return 0;
   }
-  // cycle k forward with its start state and temporaries kept, then its
-  // adjoint kernels
+  // cycle k forward into slot 1, with its temporaries in slot 0, then its
+  // adjoint kernels.  Its start state stays where it is, in the context's own
+  // arrays, but for the forward pass's last cycle, which ends there.
   int youturn(int64_t k) {
     int rc = restore(k);
-    double *sa = seg_slot(c, 0), *sb = seg_slot(c, 1);
-    const bool last = k == frontier;  // the forward pass's last cycle
-    if (!rc) rc = step(k, sa);
-    if (!rc) rc = slot_step(c, slot_temps(c, sa), sb, nullptr, 0);
+    const bool last = k == frontier;
+    double *s0 = seg_slot(c, 0), *s1 = seg_slot(c, 1);
+    if (!rc && last) rc = state_copy(c, s0, 1);
+    const StateRef from = last ? slot_state(c, s0) : own_state(c, parity), to = slot_state(c, s1);
+    if (!rc) rc = step(k, between(c, a, from, to, slot_temps(c, s0), parity));
     if (!rc && last) rc = end_of_forward();
-    if (!rc) rc = adjoint_cycle(c, stored_args(c, sa, sb, hdt[k], k == n - 1 ? 0 : 1), k == 0);
+    if (!rc) rc = adjoint_cycle(c, stored_args(c, from, slot_temps(c, s0), to.n, hdt[k], k == n - 1 ? 0 : 1), k == 0);
     cur = -1;
     return rc;
   }
@@ -1243,6 +1254,7 @@ int grad_run_revolve(lulesh_ctx *c, int64_t ncycles, int64_t snapshots, double *
   R.c = c;
   R.n = ncycles;
   R.cycle0 = c->hsc[0].cycle;
+  R.parity = c->hsc[0].parity;
   R.a = make_args(c, 0, 0);
   R.ta = R.a;
   R.ta.dt_record = c->adj.dt;
@@ -1273,22 +1285,26 @@ int vjp_cycle(lulesh_ctx *c, double grad_params[3]) {
   if (rc) return rc;
   AdjBuffers &B = c->adj;
   const int64_t E = c->inst[0].E;
-  const Batch a = make_args(c, 0, 0);
-  // the forward cycle exactly as lulesh_lagrange_leapfrog runs it, with its
-  // start state and temporaries kept in slot 0 and the state after it in
-  // slot 1
-  rc = slot_step(c, nullptr, seg_slot(c, 0), nullptr, 0);
-  if (!rc) rc = clear_err(c);
-  const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
-  for (int id : ids)
-    if (!rc) rc = launch(c, id, a);
-  if (!rc) rc = slot_step(c, slot_temps(c, seg_slot(c, 0)), seg_slot(c, 1), nullptr, 0);
+  rc = know_scalars(c);
+  if (rc) return rc;
+  const int parity = c->hsc[0].parity;
+  // the forward cycle exactly as lulesh_lagrange_leapfrog runs it, reading its
+  // start state's element fields from a copy in slot 0 (the node set it
+  // started from and its temporaries are there afterwards anyway)
+  StateRef from = own_state(c, parity);
+  const StateRef to = own_state(c, parity ^ 1);
+  from.el = slot_state(c, seg_slot(c, 0)).el;
+  rc = clear_err(c);
+  if (!rc) {
+    hipError_t e = launch_state_copy(c->stream, c->b.sc, c->b.f, E, 0, from.el.e, 1);
+    if (e != hipSuccess) rc = hip_fail(c, e, "state copy");
+  }
+  if (!rc) rc = cycle_body(c, true, between(c, make_args(c, 0, 0), from, to, nullptr, parity));
   if (!rc) rc = finish(c, true);
   if (rc) return rc;
   c->partials_valid = false;
   HIP_TRY(c, hipMemsetAsync(B.a.pacc, 0, sizeof(double) * 3 * E, c->stream));
-  rc = adjoint_cycle(c, stored_args(c, seg_slot(c, 0), seg_slot(c, 1), c->hsc[0].deltatime, 0),
-                     true);
+  rc = adjoint_cycle(c, stored_args(c, from, nullptr, to.n, c->hsc[0].deltatime, 0), true);
   if (rc) return rc;
   if (grad_params) {
     double sum[3];
@@ -1417,17 +1433,9 @@ int lulesh_replay(lulesh_ctx *c, const double *dt, int64_t ncycles) {
     if (!c || !dt || ncycles < 0) return LULESH_ERR_INVALID_ARG;
     if (c->n != 1) return fail(c, LULESH_ERR_UNSUPPORTED, "replay needs a one-domain context");
     HIP_TRY(c, hipSetDevice(c->device));
-    int rc = adj_setup(c, ncycles > 0 ? ncycles : 1, 0);
-    if (rc) return rc;
-    HIP_TRY(c, hipMemcpy(c->adj.dt, dt, sizeof(double) * ncycles, hipMemcpyHostToDevice));
-    rc = know_scalars(c);
-    if (rc) return rc;
-    const long long cycle0 = c->hsc[0].cycle;
-    rc = clear_err(c);
-    for (int64_t k = 0; k < ncycles && !rc; ++k) {
-      rc = slot_step(c, nullptr, nullptr, c->adj.dt, cycle0);
-      if (!rc) rc = cycle_body(c, true);
-    }
+    const Batch a = make_args(c, 0, 0);
+    int rc = clear_err(c);
+    for (int64_t k = 0; k < ncycles && !rc; ++k) rc = cycle_body(c, true, scheduled(a, dt[k]));
     if (rc) return rc;
     c->partials_valid = false;
     return finish(c, true);

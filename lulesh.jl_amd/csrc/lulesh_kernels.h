@@ -53,6 +53,12 @@ struct DevFields {
   double *xdd, *ydd, *zdd, *fx, *fy, *fz, *nodalMass;
 };
 
+// the element state a cycle leaves; DevFields' own arrays, or others where the
+// state before the cycle is to be kept
+struct ElemState {
+  double *e, *p, *q, *v, *ss;
+};
+
 // one instance of a (ragged) batch
 struct InstDesc {
   int s;                 // elements per edge
@@ -90,6 +96,9 @@ struct Batch {
   int qeos_launch;          // k_qeos workgroups launched
   DevScalars *sc;           // [n]
   DevFields f;
+  ElemState out;            // where k_qeos (k_elems) writes e p q v ss
+  int scheduled;            // the cycle's time step is `dt`: k_nodal takes it instead of
+  double dt;                // sc->deltatime and does timeIncrement!'s bookkeeping with it
   double *dtpart;           // 2 per element-kernel block (or k_elems workgroup)
   int elems_form;           // ElemsForm; other than ELEMS_APART, KID_QEOS runs both and KID_KIN nothing
   int parts;                // one domain: the pairs of dtpart its element kernel wrote

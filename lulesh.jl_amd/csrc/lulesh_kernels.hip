@@ -88,6 +88,10 @@ LDEV DevFields slice(const DevFields &f, const InstDesc &I) {
   return g;
 }
 
+LDEV ElemState slice(const ElemState &s, const InstDesc &I) {
+  return ElemState{s.e + I.e0, s.p + I.e0, s.q + I.e0, s.v + I.e0, s.ss + I.e0};
+}
+
 // NodeSet k of a sliced field view, chosen without indexing a local array
 // by a run-time value (that would put the struct in scratch memory)
 LDEV NodeSet pick(const DevFields &f, int k) {
@@ -614,6 +618,11 @@ LDEV void nodal_finish(const Batch &B, DevScalars *sc, int par, const DtNow *now
     store(sc, now->ts);
     sc->dt_pending = 1;
   }
+  if (B.scheduled) {
+    sc->deltatime = B.dt;
+    sc->time = sc->time + B.dt;
+    sc->cycle = sc->cycle + 1;
+  }
   sc->nodal_done = 0;
   sc->parity = par ^ 1;
 }
@@ -679,7 +688,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal(Batch B) {
   const double hourg = sc->hgcoef;
   const bool hg_on = hourg > 0.0;
   const double u_cut = sc->u_cut;
-  const double dt = sc->deltatime;
+  const double dt = B.scheduled ? B.dt : sc->deltatime;
   int *const err = DEFER ? &sc->err_nodal[par] : &sc->err;
   [[maybe_unused]] DevScalars S;
   [[maybe_unused]] bool fold = false;
@@ -1058,7 +1067,7 @@ __global__ __launch_bounds__(BLOCK) void k_nodal_planes(Batch B) {
     node_update(out, f, no, ni, nj, k, cs0, cs1, cs2,
                 NodeOld{mass, patch[1][0][po], patch[1][1][po], patch[1][2][po], patch[1][3][po],
                         patch[1][4][po], patch[1][5][po]},
-                B.defer_dt ? dts.now.ts.deltatime : S.deltatime, u_cut, B.keep_aux);
+                B.defer_dt ? dts.now.ts.deltatime : B.scheduled ? B.dt : S.deltatime, u_cut, B.keep_aux);
   }
   // as in k_nodal: the last workgroup to finish makes the set just written
   // current
@@ -1264,7 +1273,7 @@ LDEV void block_min2(double &a, double &b) {
 // zeta -, +), whatever its boundary mask makes of them.
 enum QeosValue { QV_VDOV, QV_VOLO, QV_VNEW, QV_DELX, QV_MASS = QV_DELX + 3, QV_V, QV_AREALG, QV_E, QV_P, QV_Q, QV_COUNT };
 template <bool COST, class Own>
-LDEV void qeos_element(const DevFields &f, DevScalars *sc, uint32_t eo, uint32_t bc, double dvxi, double dveta,
+LDEV void qeos_element(const DevFields &f, const ElemState &out, DevScalars *sc, uint32_t eo, uint32_t bc, double dvxi, double dveta,
                        double dvzeta, const double (&nb)[6], Own own, int keep_aux, const int *elem_rep,
                        double &cand_c, double &cand_h) {
   const double ptiny = 1e-36;
@@ -1405,15 +1414,15 @@ LDEV void qeos_element(const DevFields &f, DevScalars *sc, uint32_t eo, uint32_t
   }
   double ss = ((pbvc * e_new) + (((vnewc * vnewc) * bvc) * p_new)) / rho0;
   ss = (ss <= TINY1) ? TINY3 : sqrt(ss);
-  st_nt(f.p, eo, p_new);
-  st_nt(f.e, eo, e_new);
-  st_nt(f.q, eo, q_new);
-  st_nt(f.ss, eo, ss);
+  st_nt(out.p, eo, p_new);
+  st_nt(out.e, eo, e_new);
+  st_nt(out.q, eo, q_new);
+  st_nt(out.ss, eo, ss);
 
   // updateVolumesForElems
   double tmpV = vnew;
   if (fabs(tmpV - 1.0) < sc->v_cut) tmpV = 1.0;
-  st_nt(f.v, eo, tmpV);
+  st_nt(out.v, eo, tmpV);
   if (tmpV <= 0.0) raise(sc, ERR_UPDATE_VOLUME);
 
   // time-constraint terms; an element only counts where vdov != 0 and its
@@ -1466,7 +1475,7 @@ __global__ __launch_bounds__(BLOCK) void k_qeos(Batch B) {
     }
     auto own = [&](const double *p, int k) { return EARLY ? early[k] : ld_nt(&p[e]); };
     const int *rep = COST ? B.elem_rep + I.e0 + e : nullptr;
-    qeos_element<COST>(f, sc, eo, bc, dvxi, dveta, dvzeta, nb, own, B.keep_aux, rep, cand_c, cand_h);
+    qeos_element<COST>(f, slice(B.out, I), sc, eo, bc, dvxi, dveta, dvzeta, nb, own, B.keep_aux, rep, cand_c, cand_h);
   }
   block_min2(cand_c, cand_h);
   if (threadIdx.x == 0) {
@@ -1612,7 +1621,7 @@ __global__ __launch_bounds__((ElemBlock<BX, BY, BZ, SPLIT>::THREADS)) void k_ele
         for (int r = 0; r < 6; ++r) nb[r] = q == r ? d : nb[r];
       }
     }
-    qeos_element<false>(f, sc, eo, bc, dv[0], dv[1], dv[2], nb, [&](const double *, int v) { return own[v]; },
+    qeos_element<false>(f, B.out, sc, eo, bc, dv[0], dv[1], dv[2], nb, [&](const double *, int v) { return own[v]; },
                         B.keep_aux, nullptr, cand_c, cand_h);
   }
   block_min2<EB::CORE>(cand_c, cand_h);

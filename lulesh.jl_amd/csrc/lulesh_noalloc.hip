@@ -272,6 +272,8 @@ int run(const lulesh_device_domain *dom, double *scalars, hipStream_t st, int de
   double *ns = (double *)(base + c.off_nodes);
   f.ns[0] = NodeSet{ns, ns + N, ns + 2 * N, ns + 3 * N, ns + 4 * N, ns + 5 * N};
   f.ns[1] = NodeSet{dom->x, dom->y, dom->z, dom->xd, dom->yd, dom->zd};
+  B.out = ElemState{f.e, f.p, f.q, f.v, f.ss};
+  B.scheduled = 0;
   B.dtpart = (double *)(base + c.off_dtpart);
   B.quirks = dom->quirks;
   B.gated = 0;
