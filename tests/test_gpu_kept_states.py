@@ -86,3 +86,25 @@ def test_a_forward_pass_that_raises_leaves_its_end_state(s):
         d.close()
     same(ends[0], ends[1])
     same(ends[0], ends[2])
+
+
+@pytest.mark.gpu
+def test_gradients_with_every_share_of_cycles_kept():
+    """From its second gradient on a context keeps as many segments as a
+    thirty-second of the card's memory holds instead of replaying them: all
+    of them, some, and only the last give the same bits and end state."""
+    from lulesh_amd import grad_run
+    print("[kept] shares", flush=True)
+    for s, n, every in ((20, 11, 3), (150, 23, 4)):  # 150: about 16 slots in 9 GB
+        got = []
+        d = started(s, 1)
+        begin = {f: d.get(f) for f in STATE + SCALARS}
+        for k in range(3):
+            for f, v in begin.items():
+                d.set(f, v)
+            r = grad_run(d, n, every)
+            got.append(([r["grad_e"].view(np.uint64), r["dt"].view(np.uint64)] + held(d)[0],
+                        [r["loss"], r["grad_hgcoef"], r["grad_qlc_monoq"], r["grad_qqc_monoq"]] + held(d)[1]))
+        d.close()
+        same(got[0], got[1])
+        same(got[0], got[2])
