@@ -26,6 +26,8 @@ struct AdjArgs {
   int force_pending;                       // corner_f holds the later cycle's a_force
                                            // output, which a_node1 gathers first
   double *pacc;                            // [3][E] hgcoef, qlc_monoq, qqc_monoq partials
+  int pacc_set;                            // they start here: stored, not added to
+  int gated;                               // nothing is done if the cycle raised an error
 };
 
 enum AdjKernel { AK_QEOS = 0, AK_KIN, AK_NODE1, AK_FORCE, AK_NODE2, AK_SEED };
@@ -33,6 +35,5 @@ enum AdjKernel { AK_QEOS = 0, AK_KIN, AK_NODE1, AK_FORCE, AK_NODE2, AK_SEED };
 hipError_t launch_adjoint(int which, hipStream_t st, const AdjArgs &a);
 hipError_t launch_state_copy(hipStream_t st, DevScalars *sc, const DevFields &f, int64_t E,
                              int64_t N, double *buf, int to_buf);
-hipError_t launch_set_cycle(hipStream_t st, DevScalars *sc, long long cycle);
 
 }  // namespace lulesh

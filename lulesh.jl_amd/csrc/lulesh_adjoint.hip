@@ -80,6 +80,7 @@ LDEV int bc_source(uint32_t bc, int d, int sd) {
 __global__ __launch_bounds__(BLOCK) void a_qeos(AdjArgs A) {
   const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (e >= A.E) return;
+  if (A.gated && A.sc->err != ERR_NONE) return;
   const DevScalars *sc = A.sc;
   const DevFields &f = A.f;
   const double *dvs[3] = {f.delv_xi, f.delv_eta, f.delv_zeta};
@@ -157,14 +158,19 @@ __global__ __launch_bounds__(BLOCK) void a_qeos(AdjArgs A) {
   A.lv[e] = -li[1];
   A.lss[e] = 0.0;
   A.lvnew_delv[e] = li[1];
-  A.pacc[(int64_t)1 * A.E + e] += lqlc;
-  A.pacc[(int64_t)2 * A.E + e] += lqqc;
+  if (!A.pacc_set) {
+    lqlc = A.pacc[(int64_t)1 * A.E + e] + lqlc;
+    lqqc = A.pacc[(int64_t)2 * A.E + e] + lqqc;
+  }
+  A.pacc[(int64_t)1 * A.E + e] = lqlc;
+  A.pacc[(int64_t)2 * A.E + e] = lqqc;
 }
 
 // ---- reverse of k_kin (MonoQ gradients + relative volume) -------------------
 __global__ __launch_bounds__(BLOCK) void a_kin(AdjArgs A) {
   const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (e >= A.E) return;
+  if (A.gated && A.sc->err != ERR_NONE) return;
   const DevFields &f = A.f;
   const NodeSet S = A.cur;
   // Own delv adjoint plus what the elements that read this delv sent back:
@@ -264,6 +270,7 @@ LDEV void gather_corners(const AdjArgs &A, const double *corner, const NodeElems
 __global__ __launch_bounds__(BLOCK) void a_node1(AdjArgs A) {
   const int64_t n = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (n >= A.N) return;
+  if (A.gated && A.sc->err != ERR_NONE) return;
   const int s1 = A.s + 1, un = (int)n;
   const int i = un % s1, j = (un / s1) % s1, k = un / (s1 * s1);
   const NodeElems ne(i, j, k, A.s);
@@ -340,6 +347,7 @@ template <bool Q1, bool Q2>
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void a_force(AdjArgs A) {
   const int64_t e = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (e >= A.E) return;
+  if (A.gated && A.sc->err != ERR_NONE) return;
   const DevFields &f = A.f;
   const NodeSet S = A.old;
   int64_t nid[8];
@@ -364,8 +372,9 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void
                                                                 mass, hourg, c13, lX, lY, lZ);
     A.lv[e] += r.ldeterm * volo;
     A.lss[e] += r.lss;
-    A.pacc[e] += r.lhgcoef;
+    A.pacc[e] = A.pacc_set ? r.lhgcoef : A.pacc[e] + r.lhgcoef;
   } else {
+    if (A.pacc_set) A.pacc[e] = 0.0;
     for (int c = 0; c < 3; ++c)
       for (int n = 0; n < 8; ++n) sink.lv(c, n, 0.0);
   }
@@ -383,6 +392,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2))) void
 __global__ __launch_bounds__(BLOCK) void a_node2(AdjArgs A) {
   const int64_t n = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
   if (n >= A.N) return;
+  if (A.gated && A.sc->err != ERR_NONE) return;
   const int s1 = A.s + 1, un = (int)n;
   const NodeElems ne(un % s1, (un / s1) % s1, un / (s1 * s1), A.s);
   double g[6];
@@ -431,10 +441,6 @@ __global__ __launch_bounds__(BLOCK) void a_state_copy(DevScalars *sc, DevFields 
     }
 }
 
-__global__ void a_set_cycle(DevScalars *sc, long long cycle) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) sc->cycle = cycle;
-}
-
 static inline unsigned nblk_a(int64_t n) { return (unsigned)((n + BLOCK - 1) / BLOCK); }
 
 hipError_t launch_adjoint(int which, hipStream_t st, const AdjArgs &a) {
@@ -474,11 +480,6 @@ hipError_t launch_state_copy(hipStream_t st, DevScalars *sc, const DevFields &f,
                              int64_t N, double *buf, int to_buf) {
   hipLaunchKernelGGL(a_state_copy, dim3(nblk_a(N > E ? N : E)), dim3(BLOCK), 0, st, sc, f, E, N,
                      buf, to_buf);
-  return hipGetLastError();
-}
-
-hipError_t launch_set_cycle(hipStream_t st, DevScalars *sc, long long cycle) {
-  hipLaunchKernelGGL(a_set_cycle, dim3(1), dim3(64), 0, st, sc, cycle);
   return hipGetLastError();
 }
 

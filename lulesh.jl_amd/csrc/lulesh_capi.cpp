@@ -193,7 +193,7 @@ int pull_scalars(lulesh_ctx *c) {
 // synchronise, fold pending event pairs into the timing totals, then report
 // the lowest physics error raised on the device (if any, over all instances)
 int finish(lulesh_ctx *c, bool check_err) {
-  if (check_err) {
+  if (check_err && !c->pulled) {
     int rc = pull_scalars(c);
     if (rc) return rc;
   }
@@ -1176,8 +1176,7 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
 struct Revolve {
   lulesh_ctx *c;
   int64_t n;
-  long long cycle0;
-  Batch a, ta;               // the cycle; timeIncrement! recording its dt
+  Batch a, ta, da;           // the cycle; timeIncrement! recording its dt; k_dt with it
   std::vector<int64_t> pos;  // cycle whose start state each buffer holds (-1: free)
   std::vector<double> hdt;
   int64_t frontier = 0;      // first cycle not run yet (its dt not recorded)
@@ -1194,16 +1193,16 @@ struct Revolve {
       if (pos[i] == k) return (int)i;
     return -1;
   }
-  int restore(int64_t k) {
-    if (cur == k) return 0;
+  // where the start state of cycle k is: the context's own arrays, or the
+  // buffer it was saved in
+  int start_of(int64_t k, StateRef &from) {
+    if (cur == k) {
+      from = own_state(c, parity);
+      return 0;
+    }
     const int i = find(k);
     if (i < 0) return fail(c, LULESH_ERR_HIP, "revolve: missing saved state");
-    int rc = state_copy(c, buf(i), 0);
-    if (rc) return rc;
-    touch(c);
-    hipError_t e = launch_set_cycle(c->stream, c->b.sc, cycle0 + k);
-    if (e != hipSuccess) return hip_fail(c, e, "set cycle");
-    cur = k;
+    from = slot_state(c, buf(i));
     return 0;
   }
   // cycle k as `b` places it: the first time with timeIncrement! recording
@@ -1211,8 +1210,11 @@ struct Revolve {
   int step(int64_t k, const Batch &b) {
     int rc = 0;
     if (k == frontier) {
-      rc = launch(c, KID_TIME_INCREMENT, ta);
-      if (!rc) rc = cycle_body(c, true, b);
+      // (the first pass runs the cycles in order, and a k_dt takes the next
+      // one's timeIncrement! along, as in grad_forward)
+      if (k == 0) rc = launch(c, KID_TIME_INCREMENT, ta);
+      if (!rc) rc = cycle_body(c, false, b);
+      if (!rc) rc = launch(c, KID_DT, k + 1 < n ? da : a);
       ++frontier;
     } else {
       rc = cycle_body(c, false, scheduled(b, hdt[k]));
@@ -1222,10 +1224,14 @@ struct Revolve {
     return rc;
   }
   int advance(int64_t from, int64_t to) {
-    int rc = restore(from);
-    for (int64_t k = from; k < to && !rc; ++k) rc = step(k, a);
-    cur = to;
-    return rc;
+    for (int64_t k = from; k < to; ++k) {
+      StateRef start;
+      int rc = start_of(k, start);
+      if (!rc) rc = step(k, between(c, a, start, own_state(c, parity ^ 1), nullptr, parity));
+      if (rc) return rc;
+      cur = k + 1;
+    }
+    return 0;
   }
   int save(int64_t k) {
     const int i = find(-1);
@@ -1250,14 +1256,18 @@ struct Revolve {
     return 0;
   }
   // cycle k forward into slot 1, with its temporaries in slot 0, then its
-  // adjoint kernels.  Its start state stays where it is, in the context's own
-  // arrays, but for the forward pass's last cycle, which ends there.
+  // adjoint kernels.  Its start state is read where it is, but the forward
+  // pass's last cycle ends in the context's own arrays and starts from a copy.
   int youturn(int64_t k) {
-    int rc = restore(k);
+    StateRef from;
+    int rc = start_of(k, from);
     const bool last = k == frontier;
     double *s0 = seg_slot(c, 0), *s1 = seg_slot(c, 1);
-    if (!rc && last) rc = state_copy(c, s0, 1);
-    const StateRef from = last ? slot_state(c, s0) : own_state(c, parity), to = slot_state(c, s1);
+    if (!rc && last) {
+      rc = state_copy(c, s0, 1);
+      from = slot_state(c, s0);
+    }
+    const StateRef to = slot_state(c, s1);
     if (!rc) rc = step(k, between(c, a, from, to, slot_temps(c, s0), parity));
     if (!rc && last) rc = end_of_forward();
     if (!rc) rc = adjoint_cycle(c, stored_args(c, from, slot_temps(c, s0), to.n, hdt[k], k == n - 1 ? 0 : 1), k == 0);
@@ -1286,12 +1296,13 @@ int grad_run_revolve(lulesh_ctx *c, int64_t ncycles, int64_t snapshots, double *
   Revolve R;
   R.c = c;
   R.n = ncycles;
-  R.cycle0 = c->hsc[0].cycle;
   R.parity = c->hsc[0].parity;
   R.a = make_args(c, 0, 0);
   R.ta = R.a;
   R.ta.dt_record = c->adj.dt;
-  R.ta.dt_base = R.cycle0;
+  R.ta.dt_base = c->hsc[0].cycle;
+  R.da = R.ta;
+  R.da.loop_mode = 2;
   R.pos.assign((size_t)snapshots, -1);
   R.hdt.resize(ncycles);
   R.loss = loss;
@@ -1333,19 +1344,19 @@ int vjp_cycle(lulesh_ctx *c, double grad_params[3]) {
     if (e != hipSuccess) rc = hip_fail(c, e, "state copy");
   }
   if (!rc) rc = cycle_body(c, true, between(c, make_args(c, 0, 0), from, to, nullptr, parity));
+  // the adjoint follows without a wait for the cycle's error code: its kernels
+  // look at it themselves, and leave the shadow alone if there is one
+  AdjArgs aa = stored_args(c, from, nullptr, to.n, c->hsc[0].deltatime, 0);
+  aa.pacc_set = aa.gated = 1;
+  if (!rc) rc = adjoint_cycle(c, aa, true);
+  if (!rc) rc = pull_scalars(c);
+  double sum[3] = {0.0, 0.0, 0.0};
+  if (!rc && grad_params) rc = param_sums(c, sum);
   if (!rc) rc = finish(c, true);
   if (rc) return rc;
   c->partials_valid = false;
-  HIP_TRY(c, hipMemsetAsync(B.a.pacc, 0, sizeof(double) * 3 * E, c->stream));
-  rc = adjoint_cycle(c, stored_args(c, from, nullptr, to.n, c->hsc[0].deltatime, 0), true);
-  if (rc) return rc;
-  if (grad_params) {
-    double sum[3];
-    rc = param_sums(c, sum);
-    if (rc) return rc;
-    for (int k = 0; k < 3; ++k) grad_params[k] += sum[k];
-  }
-  return finish(c, false);
+  for (int k = 0; k < 3 && grad_params; ++k) grad_params[k] += sum[k];
+  return 0;
 }
 
 // shadow buffer of one state field, or nullptr

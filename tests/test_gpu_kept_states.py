@@ -108,3 +108,28 @@ def test_gradients_with_every_share_of_cycles_kept():
         d.close()
         same(got[0], got[1])
         same(got[0], got[2])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("raise_by", ["qstop", "volume"])
+def test_a_reversed_cycle_that_raises_leaves_the_shadow(raise_by):
+    """vjp_cycle launches its adjoint before it knows whether the cycle raised
+    an error; the shadow and the parameter sums then stay as they were."""
+    from lulesh_amd import LuleshError, vjp_cycle
+    from lulesh_amd.domain import get_shadow
+    d = started(9, 3)
+    g = np.random.default_rng(5)
+    shadow = {f: g.standard_normal(d.get(f).size) for f in STATE}
+    if raise_by == "qstop":
+        d.qstop = 1.0e-3
+    else:
+        v = d.get("v")
+        v[40] = -1.0
+        d.set("v", v)
+    params = np.array([1.0, 2.0, 3.0])
+    with pytest.raises(LuleshError):
+        vjp_cycle(d, shadow, params)
+    assert list(params) == [1.0, 2.0, 3.0]
+    for f in STATE:
+        assert np.array_equal(get_shadow(d, f).view(np.uint64), shadow[f].view(np.uint64)), f
+    d.close()
