@@ -1,7 +1,7 @@
 """Fields come to the host through pinned staging memory, in one copy up to a
 chunk of 1 MiB and moved on by threads in pieces of 128 KiB beyond that, and
 scalars are read from the host's copy while it is current: what was uploaded
-comes back at the edges of pieces, chunks and the sixteen chunks in flight,
+comes back at the edges of pieces, of chunks and of the chunks in flight,
 from several threads at once, and the scalars are the device's after every
 kind of call."""
 import threading
