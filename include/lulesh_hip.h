@@ -294,14 +294,21 @@ int lulesh_shadow_download(lulesh_ctx *ctx, const char *field, double *dst, int6
 #define LULESH_K_QEOS 2  /* MonoQ limiter, EOS, volume update, dt partial minima */
 #define LULESH_K_DT 3    /* dt minima + next timeIncrement! */
 #define LULESH_K_COUNT 4
+/* With timing on, every kernel is a launch of its own, one cycle at a time;
+ * otherwise the driver loop runs a small domain's kinematics and MonoQ/EOS as
+ * one launch, takes the dt minima inside the next nodal one, and replays
+ * several cycles to a graph launch.  The results are the same bits. */
 int lulesh_set_timing(lulesh_ctx *ctx, int32_t on);
 /* k_nodal geometry (no reference counterpart): each workgroup marches
  * `depth` node planes of its node column (16x14 nodes for large domains);
  * in a single-domain context the first chunk takes one plane more, so
  * that every chunk but the last marches depth + 1 element planes.
- * 0 restores the default: per instance, node planes split into equal
- * chunks whose depth minimises (launch rounds x planes per workgroup), a
- * round being CUs x the workgroups one CU holds.  Tile shape: per
+  * 0 restores the default: one domain whose tiles x node planes all fit on
+ * the device at once (nx <= 34) is not marched at all, a workgroup computing
+ * the two element planes around its node plane; larger ones take the chunk
+ * count whose modelled time, start plus planes marched per round of CUs x the
+ * workgroups one CU holds, is least; a batch, per instance, equal chunks of
+ * the depth that minimises (launch rounds x planes per workgroup).  Tile shape: per
  * instance the etx x (256/etx) element tile, etx in [lo, hi], that covers
  * the node columns with the fewest tiles (lulesh_set_nodal_tiles; 0, 0
  * restores the default 16..32; 2 <= lo <= hi <= 128); lulesh_nodal_tile

@@ -1,6 +1,7 @@
 // MI355X (gfx950) kernels of one LULESH Lagrange leap-frog cycle, FP64.
 //
-// One cycle = four launches on the context stream:
+// One cycle = four launches on the context stream (a small domain's has
+// other forms of the first three, k_nodal_planes and k_elems, below):
 //   k_nodal  stress corner forces (integrateStressForElems), Flanagan-
 //            Belytschko hourglass corner forces (calcHourglassControlForElems
 //            + calcFBHourglassForceForElems), their fixed-order sums at the
@@ -14,6 +15,7 @@
 //            reduced to one minimum per block
 //   k_dt     one block: the final minima (calcTimeConstraintsForElems) and,
 //            in driver-loop mode, the loop test and the next timeIncrement!
+//            (one domain of few minima: the next nodal launch does that)
 // No atomics touch field data: a node sums its corners in the reference's
 // order, so the FP64 result is deterministic run to run.
 #include "lulesh_elem.h"
