@@ -45,6 +45,7 @@ class HostCopy {
 
   // dst[0, bytes) = device src; on return the copy is done and `st` idle.
   hipError_t fetch(hipStream_t st, void *dst, const void *src, size_t bytes) {
+    std::lock_guard<std::mutex> l(one_);
     if (bytes > kChunk) return fetch_chunks(st, (char *)dst, (const char *)src, bytes);
     hipError_t e = ready(bytes, 0);
     if (e == hipSuccess && bytes) e = hipMemcpyAsync(pin_, src, bytes, hipMemcpyDeviceToHost, st);
@@ -57,6 +58,7 @@ class HostCopy {
   // (Beyond a chunk the runtime's own copy does; below, it takes 60 us where
   // this takes 15.)
   hipError_t send(hipStream_t st, void *dst, const void *src, size_t bytes) {
+    std::lock_guard<std::mutex> l(one_);
     const bool staged = bytes <= kChunk;
     hipError_t e = staged ? ready(bytes, 0) : hipSuccess;
     if (e == hipSuccess && staged && bytes) memcpy(pin_, src, bytes);
@@ -70,6 +72,7 @@ class HostCopy {
   // v + k * stride holds array k's.  Nothing but staging memory is written.
   template <class F>
   hipError_t stream(hipStream_t st, const double *src, int arrays, int64_t n, F f) {
+    std::lock_guard<std::mutex> l(one_);
     const int64_t m = (int64_t)(kChunk / sizeof(double)), chunks = (n + m - 1) / m;
     if (arrays * n <= m) {
       hipError_t e = ready((size_t)(arrays * n) * sizeof(double), 0);
@@ -110,6 +113,7 @@ class HostCopy {
     size_t bytes;
     int slot;
   };
+  std::mutex one_;  // threads that read one context's fields take turns
   char *pin_ = nullptr;
   size_t pinned_ = 0;  // bytes at pin_
   hipEvent_t ev_[kSlots] = {};

@@ -56,6 +56,30 @@ def test_threads_with_a_domain_each():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("s", [20, 70])
+def test_threads_reading_one_domain(s):
+    d = domain(s)
+    g = np.random.default_rng(s)
+    want = {f: g.standard_normal(s ** 3) for f in ("e", "p", "q", "v")}
+    for f, a in want.items():
+        d.set(f, a)
+    wrong = []
+
+    def work(f):
+        for _ in range(10):
+            if not np.array_equal(d.get(f), want[f]):
+                wrong.append(f)
+
+    threads = [threading.Thread(target=work, args=(f,)) for f in want]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    d.close()
+
+
+@pytest.mark.gpu
 def test_scalars_after_every_kind_of_call():
     import lulesh_amd as L
     s, n = 9, 12
