@@ -70,8 +70,8 @@ struct lulesh_ctx {
   std::vector<hipEvent_t> event_pool;
   double ktime[LULESH_K_COUNT] = {0};
   int64_t kcount[LULESH_K_COUNT] = {0};
-  // driver-loop graphs: one cycle of every instance, and kGraphCycles
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  // driver-loop graph: kGraphCycles cycles of every instance
+  hipGraphExec_t graph = nullptr;
   int graph_keep_aux = -1;
   std::string last_error;
   std::vector<void *> allocations;
@@ -283,15 +283,13 @@ int dev_alloc(lulesh_ctx *c, T **p, int64_t n) {
   return 0;
 }
 
-void drop_graphs(lulesh_ctx *c) {
-  for (hipGraphExec_t &g : c->graph) {
-    if (g) (void)hipGraphExecDestroy(g);
-    g = nullptr;
-  }
+void drop_graph(lulesh_ctx *c) {
+  if (c->graph) (void)hipGraphExecDestroy(c->graph);
+  c->graph = nullptr;
 }
 
 void release(lulesh_ctx *c) {
-  drop_graphs(c);
+  drop_graph(c);
   for (auto &p : c->pending) {
     (void)hipEventDestroy(p.a);
     (void)hipEventDestroy(p.b);
@@ -315,30 +313,33 @@ bool defer_dt(const lulesh_ctx *c) {
   return c->n == 1 && c->inst[0].ebn <= kDeferBlocks && !c->b.nodal_wide;
 }
 
-// Cycles in the longer of the driver loop's two graphs.  A graph launch
-// leaves the GPU idle for about 5 us before its first kernel; with eight
-// cycles behind one a cycle at s=16 takes 17.2 us instead of 21.7, s=30 25.0
-// instead of 29.0, s=64 62.7 instead of 67.5 (16 or 32 cycles: 0.1 us less
-// again, and their capture is paid for by every context).
+// Cycles in the driver loop's graph.  A graph launch leaves the GPU idle for
+// about 5 us before its first kernel; with eight cycles behind one a cycle at
+// s=16 takes 17.2 us instead of 21.7, s=30 25.0 instead of 29.0, s=64 62.7
+// instead of 67.5 (16 or 32 cycles: 0.1 us less again, and their capture is
+// paid for by every context).
 constexpr int kGraphCycles = 8;
+// Launched kernel by kernel a cycle takes hardly longer where the host keeps
+// ahead of the device (s=16 17.5 us), so only a call of this many cycles
+// captures a graph, which takes about 100 us: a context's first 10 cycles at
+// s=16 570 -> 190 us, and 20 cycles 438 -> 362.
+constexpr int kGraphFrom = 64;
 
-// the graph of `cycles` (1 or kGraphCycles) driver-loop cycles
-int build_graph(lulesh_ctx *c, int cycles) {
+int build_graph(lulesh_ctx *c) {
   if (!c->nodal_ready)
     return fail(c, LULESH_ERR_HIP, "k_nodal tables unavailable (a device allocation failed)");
   if (c->graph_keep_aux != c->keep_aux || c->graph_cost_mode != c->b.cost_mode) {
-    drop_graphs(c);
+    drop_graph(c);
     c->graph_keep_aux = c->keep_aux;
     c->graph_cost_mode = c->b.cost_mode;
   }
-  hipGraphExec_t &graph = c->graph[cycles > 1];
-  if (graph) return 0;
+  if (c->graph) return 0;
   Batch a = make_args(c, 1, 1);
   a.defer_dt = defer_dt(c);
   hipGraph_t g = nullptr;
   HIP_TRY(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
   const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
-  for (int k = 0; k < cycles; ++k)
+  for (int k = 0; k < kGraphCycles; ++k)
     for (int id : ids) {
       if (id == KID_DT && a.defer_dt) break;
       hipError_t e = launch_kernel(id, c->stream, a);
@@ -349,10 +350,10 @@ int build_graph(lulesh_ctx *c, int cycles) {
       }
     }
   HIP_TRY(c, hipStreamEndCapture(c->stream, &g));
-  hipError_t e = hipGraphInstantiate(&graph, g, nullptr, nullptr, 0);
+  hipError_t e = hipGraphInstantiate(&c->graph, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e != hipSuccess) {
-    graph = nullptr;
+    c->graph = nullptr;
     return hip_fail(c, e, "hipGraphInstantiate");
   }
   return 0;
@@ -398,7 +399,7 @@ int order_nodal(lulesh_ctx *c, const std::vector<char> *live) {
   if ((int64_t)order.size() > c->gorder_cap) {
     // only a new plan grows the table (a live subset keeps glaunch), and a
     // new plan has already dropped the graph that holds the old pointer
-    if (c->graph[0] || c->graph[1]) return fail(c, LULESH_ERR_HIP, "k_nodal order table would move under the graph");
+    if (c->graph) return fail(c, LULESH_ERR_HIP, "k_nodal order table would move under the graph");
     c->b.gblock_order = nullptr;
     if (c->gorder) HIP_TRY(c, hipFree(c->gorder));
     c->gorder = nullptr;
@@ -437,7 +438,7 @@ int plan_nodal(lulesh_ctx *c, int cz) {
   // until the new tables are on the device, k_nodal must not run, and the
   // captured graph (which holds the old ones) is gone
   c->nodal_ready = false;
-  drop_graphs(c);
+  drop_graph(c);
   c->b.nodal_wide = 0;
   for (InstDesc &I : c->inst) {
     const NodalTile t = nodal_tile(I.s, c->tile_lo, c->tile_hi);
@@ -676,6 +677,17 @@ int get_inst_scalars(lulesh_ctx *c, int32_t inst, DevScalars *out) {
   return 0;
 }
 
+// one cycle, launched kernel by kernel
+int cycle_body(lulesh_ctx *c, bool constraints, const Batch &a) {
+  const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
+  for (int id : ids) {
+    if (id == KID_DT && !constraints) break;
+    int rc = launch(c, id, a);
+    if (rc) return rc;
+  }
+  return 0;
+}
+
 int run_cycles_body(lulesh_ctx *c, int64_t num_iters, int64_t *cycles_run) {
   HIP_TRY(c, hipSetDevice(c->device));
   int rc = know_scalars(c);
@@ -686,12 +698,14 @@ int run_cycles_body(lulesh_ctx *c, int64_t num_iters, int64_t *cycles_run) {
     cycle0[i] = c->hsc[i].cycle;
     min_cycle0 = (i == 0 || cycle0[i] < min_cycle0) ? cycle0[i] : min_cycle0;
   }
-  const Batch a = make_args(c, 1, 1, num_iters);
+  // with timing on, kernels are launched one by one so each can carry its
+  // events; otherwise captured cycles (all instances) are replayed while a
+  // graph's worth of them is left
+  const bool use_graph = !c->timing;
+  Batch a = make_args(c, 1, 1, num_iters);
+  a.defer_dt = use_graph && defer_dt(c);
   rc = launch(c, KID_RUN_BEGIN, a);
   if (rc) return rc;
-  // with timing on, kernels are launched one by one so each can carry its
-  // events; otherwise captured cycles (all instances) are replayed
-  const bool use_graph = !c->timing;
   // replay exactly the cycles num_iters still allows the least advanced
   // active instance (its first cycle always runs); only stop-time exits and
   // unequal instances leave gated no-op replays behind.  The first batch is
@@ -704,25 +718,20 @@ int run_cycles_body(lulesh_ctx *c, int64_t num_iters, int64_t *cycles_run) {
     const long long left = (long long)num_iters - next_cycle + 1;
     const int64_t batch = left < 1 ? 1 : (left < cap ? left : cap);
     for (int64_t i = 0; i < batch;) {
-      const int cycles = use_graph && batch - i >= kGraphCycles ? kGraphCycles : 1;
-      i += cycles;
-      if (use_graph) {
-        rc = build_graph(c, cycles);
+      if (use_graph && batch - i >= kGraphCycles && (c->graph || left >= kGraphFrom)) {
+        rc = build_graph(c);
         if (rc) return rc;
         touch(c);
-        HIP_TRY(c, hipGraphLaunch(c->graph[cycles > 1], c->stream));
+        HIP_TRY(c, hipGraphLaunch(c->graph, c->stream));
+        i += kGraphCycles;
       } else {
-        const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
-        for (int id : ids) {
-          rc = launch(c, id, a);
-          if (rc) return rc;
-        }
+        rc = cycle_body(c, !a.defer_dt, a);
+        if (rc) return rc;
+        ++i;
       }
     }
-    if (use_graph && defer_dt(c)) {
-      Batch d = a;
-      d.defer_dt = 1;
-      rc = launch(c, KID_DT, d);
+    if (a.defer_dt) {  // the last cycle's end
+      rc = launch(c, KID_DT, a);
       if (rc) return rc;
     }
     rc = pull_scalars(c);
@@ -947,16 +956,6 @@ Batch scheduled(Batch a, double dt) {
   a.scheduled = 1;
   a.dt = dt;
   return a;
-}
-
-int cycle_body(lulesh_ctx *c, bool constraints, const Batch &a) {
-  const int ids[] = {KID_NODAL, KID_KIN, KID_QEOS, KID_DT};
-  for (int id : ids) {
-    if (id == KID_DT && !constraints) break;
-    int rc = launch(c, id, a);
-    if (rc) return rc;
-  }
-  return 0;
 }
 
 // adjoint kernel arguments of the cycle that ran from `from` (start state and
