@@ -871,11 +871,13 @@ int adj_setup_n(lulesh_ctx *c, int64_t ncycles, int64_t nstates, int64_t seg) {
       B.mem.push_back(B.final_sc);
     }
     if (rc) return rc;
-    // the shadow of lulesh_vjp_cycle starts at zero
+    // the shadow of lulesh_vjp_cycle starts at zero, on the stream that its
+    // uploads and kernels follow on (a hipMemset goes to the null stream,
+    // which this one does not wait for, and may return before it is done)
     double *zero[] = {a.lx, a.ly, a.lz, a.lxd, a.lyd, a.lzd};
-    for (double *p : zero) HIP_TRY(c, hipMemset(p, 0, sizeof(double) * N));
+    for (double *p : zero) HIP_TRY(c, hipMemsetAsync(p, 0, sizeof(double) * N, c->stream));
     double *zeroe[] = {a.le, a.lp, a.lq, a.lv, a.lss};
-    for (double *p : zeroe) HIP_TRY(c, hipMemset(p, 0, sizeof(double) * E));
+    for (double *p : zeroe) HIP_TRY(c, hipMemsetAsync(p, 0, sizeof(double) * E, c->stream));
     B.ready = true;
   }
   if (nstates > B.ckpt_cap) {
