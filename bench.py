@@ -73,20 +73,10 @@ def bench_adjoint(nx=48, cycles=200, every=20, snapshots=10):
     forward run of the same cycles, both from the initial state.  Beside it
     the memory-bounded binomial schedule with `snapshots` saved states and
     the store-everything end (one segment: every cycle's slot kept from the
-    forward pass), same gradient bit for bit, with each scheme's memory.  A
-    context's first gradient replays its segments in `checkpoint_MB`; the
-    timed one, its second, keeps `kept_MB` more of slots instead."""
-    import ctypes
+    forward pass), same gradient bit for bit, with each scheme's memory.  The
+    context's first gradient, which also allocates all this, is given too."""
     import numpy as np
     from lulesh_amd import Domain, LuleshProblem, grad_run, grad_run_revolve, run
-    hip = ctypes.CDLL("libamdhip64.so", mode=ctypes.RTLD_GLOBAL)
-
-    def free_bytes():
-        avail, total = ctypes.c_size_t(), ctypes.c_size_t()
-        if hip.hipMemGetInfo(ctypes.byref(avail), ctypes.byref(total)) != 0:
-            raise RuntimeError("hipMemGetInfo failed")
-        return avail.value
-
     d = Domain(LuleshProblem(cycles, True, nx, 11, 1, 1))
     # warm-up: the forward graph is captured and the gradient's checkpoint and
     # segment buffers are allocated (first use) outside the timed runs
@@ -95,10 +85,6 @@ def bench_adjoint(nx=48, cycles=200, every=20, snapshots=10):
     t0 = time.perf_counter()
     grad_run(d, cycles, every)
     first = time.perf_counter() - t0
-    before = free_bytes()
-    d.reset()
-    grad_run(d, cycles, every)
-    kept = before - free_bytes()
     d.reset()
     t0 = time.perf_counter()
     run(d, cycles)
@@ -127,7 +113,7 @@ def bench_adjoint(nx=48, cycles=200, every=20, snapshots=10):
             "forward_ms": round(fwd * 1e3, 3), "gradient_ms": round(grad * 1e3, 3),
             "ratio": round(grad / fwd, 3), "loss": g["loss"],
             "first_gradient_ms": round(first * 1e3, 3),
-            "checkpoint_MB": round(mem_two / 1e6, 1), "kept_MB": round(kept / 1e6, 1),
+            "checkpoint_MB": round(mem_two / 1e6, 1),
             "revolve": {"snapshots": snapshots, "gradient_ms": round(grad_rv * 1e3, 3),
                         "ratio": round(grad_rv / fwd, 3), "cycles_run": gr["forward_cycles"],
                         "checkpoint_MB": round(mem_rv / 1e6, 1),

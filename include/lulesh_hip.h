@@ -232,9 +232,9 @@ int lulesh_batch_verify(lulesh_ctx *ctx, int32_t inst, double out[4]);
  * (examples/benchmark.jl:48-51,85-86) with hand-written adjoint kernels.
  * lulesh_grad_run runs `ncycles` cycles of the driver loop from the current
  * state (checkpointing it every `checkpoint_every` cycles), then sweeps back
- * through them, recomputing each segment from its checkpoint (from the
- * context's second gradient on, only the segments that a thirty-second of
- * the device's memory does not hold), and returns
+ * through them, recomputing each segment but the last from its checkpoint
+ * (what it may keep on the device is the caller's choice: the checkpoints
+ * and the cycles of one segment, no more), and returns
  *   *loss        = sum_e e[e] * elemMass[e] at the end (total internal energy),
  *   grad_e[E]    = d loss / d e at the start,
  *   grad_params  = d loss / d {hgcoef, qlc_monoq, qqc_monoq},

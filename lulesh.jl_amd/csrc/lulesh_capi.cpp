@@ -36,7 +36,6 @@ struct AdjBuffers {
   int64_t ckpt_cap = 0;        // states
   double *seg = nullptr;       // states of the segment being reversed
   int64_t seg_cap = 0;
-  int64_t gradients = 0;       // grad_run calls that ran to their end
   double *final_state = nullptr;
   DevScalars *final_sc = nullptr;
   std::vector<void *> mem;
@@ -1033,7 +1032,6 @@ template <typename Save>
 int grad_forward(lulesh_ctx *c, int64_t ncycles, long long cycle0, Save save, int64_t slot_from,
                  double *loss, double *dt_out) {
   AdjBuffers &B = c->adj;
-  const int64_t E = c->inst[0].E;
   const int parity0 = c->hsc[0].parity;
   const Batch a = make_args(c, 0, 0);
   Batch ta = a;  // timeIncrement! that also records the dt it takes
@@ -1091,51 +1089,24 @@ int grad_results(lulesh_ctx *c, double *grad_e, double grad_params[3]) {
   return rc;
 }
 
-// Cycle slots a gradient may keep beyond the segment it was asked for: from
-// the context's second gradient on, a thirty-second of the card's memory (9
-// GB of 288) and no more than a quarter of what is free now.  A kept cycle
-// is not replayed: 200 cycles at s=48 in segments of 20 take 23.5 ms instead
-// of 30.6.  But a GB costs 2.5 ms to allocate and as long to free, twice what
-// its replays take once, so a context's first gradient does without.
-int64_t kept_slots(lulesh_ctx *c, int64_t ncycles) {
-  const int64_t have = c->adj.seg_cap;
-  if (have >= ncycles || !c->adj.gradients) return have;
-  size_t avail = 0, total = 0;
-  if (hipMemGetInfo(&avail, &total) != hipSuccess) {
-    (void)hipGetLastError();
-    return have;
-  }
-  return std::max(have, (int64_t)(std::min(avail / 4, total / 32) / sizeof(double)) / cycle_slot(c) - 1);
-}
-
 int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, double grad_params[3],
              double *loss, double *dt_out) {
   if (c->n != 1) return fail(c, LULESH_ERR_UNSUPPORTED, "the adjoint needs a one-domain context");
   if (ncycles < 1 || every < 1) return fail(c, LULESH_ERR_INVALID_ARG, "ncycles and checkpoint interval must be >= 1");
   HIP_TRY(c, hipSetDevice(c->device));
-  // 1. which of the segments of `every` cycles the forward pass keeps whole
-  const int64_t nseg = (ncycles + every - 1) / every;
-  int64_t kept = kept_segments(ncycles, every, kept_slots(c, ncycles));
-  auto setup = [&] {
-    const int64_t whole = ncycles - (nseg - kept) * every;
-    return adj_setup_n(c, ncycles, nseg - kept, kept < nseg ? std::max(whole, every) : whole);
-  };
-  int rc = setup();
-  if (rc && kept > 1) {  // no room for that: the last segment alone
-    (void)hipGetLastError();
-    kept = 1;
-    rc = setup();
-  }
+  // a checkpoint for each segment of `every` cycles but the last, whose
+  // cycles the forward pass leaves in the slots
+  every = std::min(every, ncycles);
+  const int64_t nseg = (ncycles + every - 1) / every, slot_from = (nseg - 1) * every;
+  int rc = adj_setup_n(c, ncycles, nseg - 1, every);
   if (rc) return rc;
   AdjBuffers &B = c->adj;
-  const int64_t E = c->inst[0].E, N = c->inst[0].N, state = 6 * N + 5 * E;
-  const int64_t slot_from = (nseg - kept) * every;
+  const int64_t state = 6 * c->inst[0].N + 5 * c->inst[0].E;
   rc = know_scalars(c);
   if (rc) return rc;
   const long long cycle0 = c->hsc[0].cycle;
   int parity = c->hsc[0].parity + (int)(ncycles & 1);  // after the forward pass
-  // 2. forward pass: a checkpoint at the start of every other segment, dt
-  // schedule recorded, the kept segments' slots filled on the way
+  // 1. forward pass: dt schedule recorded, checkpoints and slots filled
   rc = grad_forward(
       c, ncycles, cycle0,
       [&](int64_t k) -> double * {
@@ -1143,15 +1114,15 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
       },
       slot_from, loss, dt_out);
   if (rc) return rc;
-  // 3. reverse sweep, segment by segment: where it is not kept, replay it from
-  // its checkpoint from slot to slot; then run the adjoint kernels of its
-  // cycles backwards against the slots
+  // 2. reverse sweep, segment by segment: every one but the last is replayed
+  // from its checkpoint, from slot to slot; then the adjoint kernels of its
+  // cycles run backwards against the slots
   std::vector<double> hdt(ncycles);
   HIP_TRY(c, c->host.fetch(c->stream, hdt.data(), B.dt, sizeof(double) * ncycles));
   for (int64_t sg = nseg - 1; sg >= 0 && !rc; --sg) {
     const int64_t k0 = sg * every, k1 = (k0 + every < ncycles) ? k0 + every : ncycles;
-    const int64_t L = k1 - k0, s0 = k0 >= slot_from ? k0 - slot_from : 0;
-    if (k0 < slot_from) {
+    const int64_t L = k1 - k0;
+    if (sg < nseg - 1) {
       HIP_TRY(c, hipMemcpyAsync(seg_slot(c, 0), B.ckpt + sg * state, sizeof(double) * state,
                                 hipMemcpyDeviceToDevice, c->stream));
       const Batch a = make_args(c, 0, 0);
@@ -1160,12 +1131,11 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
     }
     for (int64_t j = L - 1; j >= 0 && !rc; --j) {
       const int64_t k = k0 + j;
-      rc = adjoint_cycle(c, stored_slots(c, s0 + j, hdt[k], k == ncycles - 1 ? 0 : 1), k == 0);
+      rc = adjoint_cycle(c, stored_slots(c, j, hdt[k], k == ncycles - 1 ? 0 : 1), k == 0);
     }
   }
   if (rc) return rc;
-  ++B.gradients;
-  // 4. results, then the state the forward pass ended in
+  // 3. results, then the state the forward pass ended in
   return grad_results(c, grad_e, grad_params);
 }
 

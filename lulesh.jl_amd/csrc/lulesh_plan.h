@@ -368,15 +368,6 @@ inline ElemsPlan elems_plan(int s, int eblocks, int cus) {
   return ElemsPlan{ELEMS_APART, eblocks};
 }
 
-// A gradient over `ncycles` cycles in segments of `every`: how many of the
-// last segments are kept whole if their cycles may take `slots` slots (at
-// least the last one, which the reverse sweep starts with).
-inline int64_t kept_segments(int64_t ncycles, int64_t every, int64_t slots) {
-  const int64_t nseg = (ncycles + every - 1) / every, last = ncycles - (nseg - 1) * every;
-  const int64_t more = slots > last ? (slots - last) / every : 0;
-  return more < nseg - 1 ? more + 1 : nseg;
-}
-
 // k_qeos runs 256-element blocks (each writes one pair of dt partial
 // minima); XCD x takes runs of QEOS_GROUP consecutive blocks, the runs
 // dealt round-robin, so the eight XCDs sweep neighbouring addresses
