@@ -4,9 +4,9 @@
 // A copy straight into pageable memory costs the runtime a pass of its own
 // over the destination, page by page and on one thread: a fresh array's pages
 // are not there yet, and 7 MB take 1.1 ms where the bus needs 0.15.  Here the
-// device copies into pinned chunks and a few threads move them on, each
-// meeting its own share of the page faults; a field of less than a chunk
-// takes one copy and one wait.  The eleven state fields into fresh arrays, with
+// device copies into pinned chunks and the process's few threads for that
+// (lulesh_copypool.h) move them on, each meeting its own share of the page
+// faults; a field of less than a chunk takes one copy and one wait.  The eleven state fields into fresh arrays, with
 // the scalars the caller reads known on the host: s=16 500 -> 165 us, s=30 470
 // -> 260, s=63 4.7 -> 2.4 ms, s=96 11.0 -> 4.7, s=192 63.6 -> 21.6.
 #pragma once
@@ -18,11 +18,11 @@
 
 #include <algorithm>
 #include <atomic>
-#include <condition_variable>
+#include <memory>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
+
+#include "lulesh_copypool.h"
 
 namespace lulesh {
 
@@ -32,12 +32,6 @@ class HostCopy {
   HostCopy(const HostCopy &) = delete;
   HostCopy &operator=(const HostCopy &) = delete;
   ~HostCopy() {
-    {
-      std::lock_guard<std::mutex> l(m_);
-      stop_ = true;
-    }
-    cv_.notify_all();
-    for (std::thread &w : workers_) w.join();
     for (hipEvent_t e : ev_)
       if (e) (void)hipEventDestroy(e);
     if (pin_) (void)hipHostFree(pin_);
@@ -106,24 +100,15 @@ class HostCopy {
   // MB with 4, 6, 16 chunks in flight 2.17, 1.95, 1.92 ms; six are pinned in
   // the time of one download of 7 MB).
   static constexpr size_t kChunk = 1 << 20, kPiece = 1 << 17;
-  static constexpr int kSlots = 6, kWorkers = 7, kJobs = kSlots * (int)(kChunk / kPiece);
-  struct Job {
-    char *dst;
-    const char *src;
-    size_t bytes;
-    int slot;
-  };
+  static constexpr int kSlots = 6;
+  static_assert(kSlots * (int)(kChunk / kPiece) <= CopyPool::kPieces, "a queue holds what is in flight");
   std::mutex one_;  // threads that read one context's fields take turns
   char *pin_ = nullptr;
   size_t pinned_ = 0;  // bytes at pin_
   hipEvent_t ev_[kSlots] = {};
-  std::atomic<int> busy_[kSlots] = {};  // jobs that still read the slot
-  std::mutex m_;
-  std::condition_variable cv_;
-  Job jobs_[kJobs];  // ring of landed pieces
-  int head_ = 0, count_ = 0;
-  bool stop_ = false;
-  std::vector<std::thread> workers_;
+  std::atomic<int> busy_[kSlots] = {};  // pieces that still read the slot
+  std::shared_ptr<CopyPool> pool_;      // from the first large field on
+  CopyPool::Queue queue_;
 
   char *slot(int i) { return pin_ + (size_t)i * kChunk; }
 
@@ -145,53 +130,11 @@ class HostCopy {
     return e;
   }
 
-  bool take(Job &j) {
-    if (!count_) return false;
-    j = jobs_[head_];
-    head_ = (head_ + 1) % kJobs;
-    --count_;
-    return true;
-  }
-  void move(const Job &j) {
-    memcpy(j.dst, j.src, j.bytes);
-    busy_[j.slot].fetch_sub(1, std::memory_order_release);
-  }
-  bool help() {
-    Job j;
-    {
-      std::lock_guard<std::mutex> l(m_);
-      if (!take(j)) return false;
-    }
-    move(j);
-    return true;
-  }
-  void work() {
-    std::unique_lock<std::mutex> l(m_);
-    for (;;) {
-      Job j;
-      if (take(j)) {
-        l.unlock();
-        move(j);
-        l.lock();
-      } else if (stop_) {
-        return;
-      } else {
-        cv_.wait(l);
-      }
-    }
-  }
-
   hipError_t fetch_chunks(hipStream_t st, char *dst, const char *src, size_t bytes) {
     hipError_t e = ready(kSlots * kChunk, kSlots);
     if (e != hipSuccess) return e;
-    if (workers_.empty()) {
-      const int n = std::min<int>(kWorkers, (int)std::thread::hardware_concurrency() - 1);
-      try {
-        for (int i = 0; i < n; ++i) workers_.emplace_back([this] { work(); });
-      } catch (const std::system_error &) {
-        // fewer threads: this one moves what they do not
-      }
-    }
+    if (!pool_) pool_ = CopyPool::get();
+    pool_->attach(queue_);
     const int64_t chunks = (int64_t)((bytes + kChunk - 1) / kChunk);
     auto size = [&](int64_t k) { return std::min(kChunk, bytes - (size_t)k * kChunk); };
     int64_t asked = 0, landed = 0;
@@ -208,25 +151,18 @@ class HostCopy {
         const int s = (int)(landed % kSlots);
         e = hipEventSynchronize(ev_[s]);
         if (e != hipSuccess) break;
-        const size_t all = size(landed);
-        busy_[s].store((int)((all + kPiece - 1) / kPiece), std::memory_order_relaxed);
-        {
-          std::lock_guard<std::mutex> l(m_);
-          for (size_t o = 0; o < all; o += kPiece, ++count_)
-            jobs_[(head_ + count_) % kJobs] =
-                Job{dst + (size_t)landed * kChunk + o, slot(s) + o, std::min(kPiece, all - o), s};
-        }
-        cv_.notify_all();
+        pool_->push(queue_, dst + (size_t)landed * kChunk, slot(s), size(landed), kPiece, &busy_[s]);
         ++landed;
-      } else if (!help()) {
+      } else if (!pool_->help(queue_)) {
         std::this_thread::yield();
       }
     }
     // no thread writes dst and no copy is under way once this returns
-    while (help()) {
+    while (pool_->help(queue_)) {
     }
     for (std::atomic<int> &b : busy_)
       while (b.load(std::memory_order_acquire)) std::this_thread::yield();
+    pool_->detach(queue_);
     const hipError_t e2 = hipStreamSynchronize(st);
     return e != hipSuccess ? e : e2;
   }
