@@ -706,16 +706,24 @@ int run_cycles_body(lulesh_ctx *c, int64_t num_iters, int64_t *cycles_run) {
   rc = launch(c, KID_RUN_BEGIN, a);
   if (rc) return rc;
   // replay exactly the cycles num_iters still allows the least advanced
-  // active instance (its first cycle always runs); only stop-time exits and
-  // unequal instances leave gated no-op replays behind.  The first batch is
-  // of 32 cycles, as each wait for the device between batches costs about 10
-  // us (s=16, 10 cycles 246 -> 207 us against a first batch of 8), and a
-  // cycle that no longer runs costs about 6
-  int64_t cap = 32;
+  // active instance (its first cycle always runs); only stop-time exits,
+  // errors and unequal instances leave gated no-op replays behind, one where
+  // every instance has reached its stop time already.
+  // The first batch is of 8 cycles: a no-op cycle still starts all its
+  // workgroups, 6 us at s=48, 8 at s=96, 35 at s=192.  Where the element
+  // kernels are one launch (s <= 40) it is 4 and a cycle 17 to 34, so that the
+  // 10 us of each wait for the device between batches count for more: 32 (s=16,
+  // 10 cycles 246 -> 207 us), unless the stop time is nearer than that many
+  // of the last time step.
+  bool go = false;
+  for (int i = 0; i < c->n; ++i) go = go || c->hsc[i].time < c->hsc[i].stoptime;
+  const DevScalars &S0 = c->hsc[0];
+  const bool small = a.elems_form != ELEMS_APART && S0.stoptime - S0.time >= 32 * S0.deltatime;
+  int64_t cap = small ? 32 : 8;
   long long next_cycle = min_cycle0 + 1;
   for (;;) {
     const long long left = (long long)num_iters - next_cycle + 1;
-    const int64_t batch = left < 1 ? 1 : (left < cap ? left : cap);
+    const int64_t batch = !go || left < 1 ? 1 : (left < cap ? left : cap);
     for (int64_t i = 0; i < batch;) {
       if (use_graph && batch - i >= kGraphCycles && (c->graph || left >= kGraphFrom)) {
         rc = build_graph(c);
