@@ -828,12 +828,10 @@ int64_t cycle_slot(const lulesh_ctx *c) {
   return 6 * N + 14 * E;
 }
 
-// dt schedule of `ncycles`; with `every` > 0 also the adjoint fields, the
-// checkpoints and one segment of `every` cycle slots
-// Adjoint buffers for `ncycles` recorded time steps, `nstates` saved
-// states (6N + 5E doubles each) and a segment of `seg` cycle slots plus one
-// (seg <= 0: the time-step record only).
-int adj_setup_n(lulesh_ctx *c, int64_t ncycles, int64_t nstates, int64_t seg) {
+// The adjoint fields, and room for `ncycles` recorded time steps, `nstates`
+// saved states (6N + 5E doubles each) and, if `seg` > 0, a segment of so many
+// cycle slots plus one.
+int adj_setup(lulesh_ctx *c, int64_t ncycles, int64_t nstates, int64_t seg) {
   AdjBuffers &B = c->adj;
   const int64_t E = c->inst[0].E, N = c->inst[0].N;
   const int64_t state = 6 * N + 5 * E;
@@ -844,7 +842,6 @@ int adj_setup_n(lulesh_ctx *c, int64_t ncycles, int64_t nstates, int64_t seg) {
     if (rc) return rc;
     B.dt_cap = ncycles;
   }
-  if (seg <= 0) return 0;
   if (!B.ready) {
     // a_force addresses node and element values by 32-bit byte offsets
     if (8 * N > (int64_t)UINT32_MAX || 8 * E > (int64_t)UINT32_MAX)
@@ -900,11 +897,6 @@ int adj_setup_n(lulesh_ctx *c, int64_t ncycles, int64_t nstates, int64_t seg) {
     B.seg_cap = seg;
   }
   return 0;
-}
-
-// checkpoints every `every` cycles and a segment of `every` slots
-int adj_setup(lulesh_ctx *c, int64_t ncycles, int64_t every) {
-  return adj_setup_n(c, ncycles, every > 0 ? (ncycles + every - 1) / every : 0, every);
 }
 
 int state_copy(lulesh_ctx *c, double *buf, int to_buf) {
@@ -1106,7 +1098,7 @@ int grad_run(lulesh_ctx *c, int64_t ncycles, int64_t every, double *grad_e, doub
   // cycles the forward pass leaves in the slots
   every = std::min(every, ncycles);
   const int64_t nseg = (ncycles + every - 1) / every, slot_from = (nseg - 1) * every;
-  int rc = adj_setup_n(c, ncycles, nseg - 1, every);
+  int rc = adj_setup(c, ncycles, nseg - 1, every);
   if (rc) return rc;
   AdjBuffers &B = c->adj;
   const int64_t state = 6 * c->inst[0].N + 5 * c->inst[0].E;
@@ -1268,7 +1260,7 @@ int grad_run_revolve(lulesh_ctx *c, int64_t ncycles, int64_t snapshots, double *
     return fail(c, LULESH_ERR_INVALID_ARG, "ncycles and snapshots must be >= 1");
   if (snapshots > ncycles) snapshots = ncycles;
   HIP_TRY(c, hipSetDevice(c->device));
-  int rc = adj_setup_n(c, ncycles, snapshots, 1);
+  int rc = adj_setup(c, ncycles, snapshots, 1);
   if (rc) return rc;
   rc = know_scalars(c);
   if (rc) return rc;
@@ -1304,19 +1296,18 @@ int grad_run_revolve(lulesh_ctx *c, int64_t ncycles, int64_t snapshots, double *
 int vjp_cycle(lulesh_ctx *c, double grad_params[3]) {
   if (c->n != 1) return fail(c, LULESH_ERR_UNSUPPORTED, "the adjoint needs a one-domain context");
   HIP_TRY(c, hipSetDevice(c->device));
-  int rc = adj_setup(c, 1, 1);
+  int rc = adj_setup(c, 0, 0, 0);
   if (rc) return rc;
-  AdjBuffers &B = c->adj;
   const int64_t E = c->inst[0].E;
   rc = know_scalars(c);
   if (rc) return rc;
   const int parity = c->hsc[0].parity;
   // the forward cycle exactly as lulesh_lagrange_leapfrog runs it, reading its
-  // start state's element fields from a copy in slot 0 (the node set it
-  // started from and its temporaries are there afterwards anyway)
+  // start state's element fields from a copy in the gradients' end state (the
+  // node set it started from and its temporaries are there afterwards anyway)
   StateRef from = own_state(c, parity);
   const StateRef to = own_state(c, parity ^ 1);
-  from.el = slot_state(c, seg_slot(c, 0)).el;
+  from.el = slot_state(c, c->adj.final_state).el;
   rc = clear_err(c);
   if (!rc) {
     hipError_t e = launch_state_copy(c->stream, c->b.sc, c->b.f, E, 0, from.el.e, 1);
@@ -1363,7 +1354,7 @@ int shadow_move(lulesh_ctx *c, const char *field, double *host, int64_t n, bool 
   if (c->n != 1) return fail(c, LULESH_ERR_UNSUPPORTED, "the adjoint needs a one-domain context");
   if (!host) return fail(c, LULESH_ERR_INVALID_ARG, "null buffer");
   HIP_TRY(c, hipSetDevice(c->device));
-  int rc = adj_setup(c, 1, 1);
+  int rc = adj_setup(c, 0, 0, 0);
   if (rc) return rc;
   int64_t len = 0;
   double *p = shadow_field(c, field, &len);

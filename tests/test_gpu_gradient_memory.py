@@ -45,3 +45,23 @@ def test_an_interval_beyond_the_cycles_takes_their_slots_only():
         got.append(grad_run(d, 4, every)["grad_e"].view(np.uint64))
         d.close()
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+
+
+@pytest.mark.gpu
+def test_a_reversed_cycle_takes_the_adjoint_fields_only():
+    """vjp_cycle and the shadow's uploads reserve the adjoint arrays (9N + 118E
+    doubles and a state) and neither checkpoints nor cycle slots, which only
+    gradients over several cycles have."""
+    from lulesh_amd import timeIncrement, vjp_cycle
+    from lulesh_amd.domain import set_shadow
+    s = 96
+    print(f"[gradient memory] vjp s={s}", flush=True)
+    E, N = s ** 3, (s + 1) ** 3
+    d = domain(s)
+    timeIncrement(d)
+    before = free_bytes()
+    set_shadow(d, "e", np.ones(E))
+    vjp_cycle(d)
+    # (24 allocations, each rounded up to a page of 2 MiB)
+    assert before - free_bytes() < 8 * (15 * N + 123 * E) + 24 * 2 ** 21 + 2 ** 26
+    d.close()
