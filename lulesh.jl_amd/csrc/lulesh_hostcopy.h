@@ -1,5 +1,8 @@
 // Copies to (and from) the host through pinned staging memory, one per
-// context.
+// context.  What a small field takes is allocated with the context, in one
+// piece with its scalars: the first pinned allocation of its size takes up to
+// 500 us, and a context of s=20 that was read twice paid it twice (its first
+// two fields 327 and 339 us instead of 32 and 29).
 //
 // A copy straight into pageable memory costs the runtime a pass of its own
 // over the destination, page by page and on one thread: a fresh array's pages
@@ -34,49 +37,59 @@ class HostCopy {
   ~HostCopy() {
     for (hipEvent_t e : ev_)
       if (e) (void)hipEventDestroy(e);
-    if (pin_) (void)hipHostFree(pin_);
+    if (slots_) (void)hipHostFree(slots_);
+  }
+
+  // staging for a context that copies `bytes` at a time where it can
+  static size_t staging(size_t bytes) { return std::min(std::max(bytes, kLeast), kChunk); }
+  // pinned memory of that size, which the caller frees after its last call here
+  void use(void *pinned, size_t bytes) {
+    pin_ = (char *)pinned;
+    pinned_ = bytes;
   }
 
   // dst[0, bytes) = device src; on return the copy is done and `st` idle.
   hipError_t fetch(hipStream_t st, void *dst, const void *src, size_t bytes) {
     std::lock_guard<std::mutex> l(one_);
     if (bytes > kChunk) return fetch_chunks(st, (char *)dst, (const char *)src, bytes);
-    hipError_t e = ready(bytes, 0);
-    if (e == hipSuccess && bytes) e = hipMemcpyAsync(pin_, src, bytes, hipMemcpyDeviceToHost, st);
-    if (e == hipSuccess) e = hipStreamSynchronize(st);
-    if (e == hipSuccess && bytes) memcpy(dst, pin_, bytes);
-    return e;
+    hipError_t e = hipSuccess;
+    for (size_t o = 0, m; o < bytes && e == hipSuccess; o += m) {
+      m = std::min(bytes - o, pinned_);
+      e = hipMemcpyAsync(pin_, (const char *)src + o, m, hipMemcpyDeviceToHost, st);
+      if (e == hipSuccess) e = hipStreamSynchronize(st);
+      if (e == hipSuccess) memcpy((char *)dst + o, pin_, m);
+    }
+    return bytes ? e : hipStreamSynchronize(st);
   }
 
   // device dst = src[0, bytes); on return the copy is done and `st` idle.
-  // (Beyond a chunk the runtime's own copy does; below, it takes 60 us where
-  // this takes 15.)
+  // (Beyond the staging memory the runtime's own copy does; below, it takes 60
+  // us where this takes 15.)
   hipError_t send(hipStream_t st, void *dst, const void *src, size_t bytes) {
     std::lock_guard<std::mutex> l(one_);
-    const bool staged = bytes <= kChunk;
-    hipError_t e = staged ? ready(bytes, 0) : hipSuccess;
-    if (e == hipSuccess && staged && bytes) memcpy(pin_, src, bytes);
-    if (e == hipSuccess && bytes) e = hipMemcpyAsync(dst, staged ? pin_ : src, bytes, hipMemcpyHostToDevice, st);
+    const bool staged = bytes <= pinned_;
+    hipError_t e = hipSuccess;
+    if (staged && bytes) memcpy(pin_, src, bytes);
+    if (bytes) e = hipMemcpyAsync(dst, staged ? pin_ : src, bytes, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     return e;
   }
 
   // f(v, stride, m), in order, for the next m values of every one of
-  // `arrays` arrays of n values that follow one another on the device:
-  // v + k * stride holds array k's.  Nothing but staging memory is written.
+  // `arrays` arrays (at most three) of n values that follow one another on the
+  // device: v + k * stride holds array k's.  Nothing but staging memory is written.
   template <class F>
   hipError_t stream(hipStream_t st, const double *src, int arrays, int64_t n, F f) {
     std::lock_guard<std::mutex> l(one_);
     const int64_t m = (int64_t)(kChunk / sizeof(double)), chunks = (n + m - 1) / m;
-    if (arrays * n <= m) {
-      hipError_t e = ready((size_t)(arrays * n) * sizeof(double), 0);
-      if (e == hipSuccess && n > 0)
-        e = hipMemcpyAsync(pin_, src, (size_t)(arrays * n) * sizeof(double), hipMemcpyDeviceToHost, st);
+    if ((size_t)(arrays * n) * sizeof(double) <= pinned_) {
+      hipError_t e = hipSuccess;
+      if (n > 0) e = hipMemcpyAsync(pin_, src, (size_t)(arrays * n) * sizeof(double), hipMemcpyDeviceToHost, st);
       if (e == hipSuccess) e = hipStreamSynchronize(st);
       if (e == hipSuccess) f((const double *)pin_, n, n);
       return e;
     }
-    hipError_t e = ready((size_t)(2 * arrays) * kChunk, 2);
+    hipError_t e = ready();
     auto ask = [&](int64_t k) {
       for (int a = 0; a < arrays && e == hipSuccess; ++a)
         e = hipMemcpyAsync(slot((int)(k & 1) * arrays + a), src + a * n + k * m,
@@ -99,39 +112,33 @@ class HostCopy {
   // threads share a chunk by pieces, so that a few chunks occupy them all (57
   // MB with 4, 6, 16 chunks in flight 2.17, 1.95, 1.92 ms; six are pinned in
   // the time of one download of 7 MB).
-  static constexpr size_t kChunk = 1 << 20, kPiece = 1 << 17;
+  static constexpr size_t kChunk = 1 << 20, kPiece = 1 << 17, kLeast = 1 << 14;
   static constexpr int kSlots = 6;
   static_assert(kSlots * (int)(kChunk / kPiece) <= CopyPool::kPieces, "a queue holds what is in flight");
   std::mutex one_;  // threads that read one context's fields take turns
-  char *pin_ = nullptr;
-  size_t pinned_ = 0;  // bytes at pin_
+  char *pin_ = nullptr;    // the staging memory of small fields
+  size_t pinned_ = 0;
+  char *slots_ = nullptr;  // kSlots chunks
   hipEvent_t ev_[kSlots] = {};
   std::atomic<int> busy_[kSlots] = {};  // pieces that still read the slot
   std::shared_ptr<CopyPool> pool_;      // from the first large field on
   CopyPool::Queue queue_;
 
-  char *slot(int i) { return pin_ + (size_t)i * kChunk; }
+  char *slot(int i) { return slots_ + (size_t)i * kChunk; }
 
-  // at least `bytes` of pinned memory, and `events` events
-  hipError_t ready(size_t bytes, int events) {
+  // the chunks and their events
+  hipError_t ready() {
     hipError_t e = hipSuccess;
-    for (int i = 0; i < events && e == hipSuccess; ++i)
+    for (int i = 0; i < kSlots && e == hipSuccess; ++i)
       if (!ev_[i]) e = hipEventCreateWithFlags(&ev_[i], hipEventDisableTiming);
-    if (e != hipSuccess || bytes <= pinned_) return e;
-    size_t want = 1 << 16;  // (a power of two while it is less than a chunk)
-    while (want < bytes && want < kChunk) want *= 2;
-    want = std::max(want, bytes);
-    if (pin_) (void)hipHostFree(pin_);
-    pin_ = nullptr;
-    pinned_ = 0;
-    e = hipHostMalloc((void **)&pin_, want, hipHostMallocDefault);
-    if (e != hipSuccess) pin_ = nullptr;
-    else pinned_ = want;
+    if (e != hipSuccess || slots_) return e;
+    e = hipHostMalloc((void **)&slots_, kSlots * kChunk, hipHostMallocDefault);
+    if (e != hipSuccess) slots_ = nullptr;
     return e;
   }
 
   hipError_t fetch_chunks(hipStream_t st, char *dst, const char *src, size_t bytes) {
-    hipError_t e = ready(kSlots * kChunk, kSlots);
+    hipError_t e = ready();
     if (e != hipSuccess) return e;
     if (!pool_) pool_ = CopyPool::get();
     pool_->attach(queue_);

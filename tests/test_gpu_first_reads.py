@@ -1,0 +1,88 @@
+"""A context's first downloads: small fields go through staging memory that
+comes with the context, larger ones through chunks allocated for the first of
+them.  What was uploaded comes back on either side of each line, also for
+arrays longer than any field (a small domain's time steps)."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+REPO = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def domain(s):
+    from lulesh_amd import Domain, LuleshProblem
+    return Domain(LuleshProblem(10, True, s, 1, 1, 1))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("s", [1, 7, 8, 34, 35, 36, 49, 50, 51])
+def test_reads_of_a_fresh_context(s):
+    # staging of three node arrays, 16 KiB at least (s=7 12 KB, 8 17 KB) and
+    # 1 MiB at most (s=34 1.03 MB, 35 1.12); fields beyond it from s=50 (1.00
+    # and 1.06 MB) and 51 (1.06 and 1.12) on
+    print(f"[first reads] s={s}", flush=True)
+    g = np.random.default_rng(s)
+    d = domain(s)
+    want = {f: g.standard_normal(d.numNode if f in ("x", "zd") else d.numElem) for f in ("x", "e", "zd", "ss")}
+    for f, a in want.items():
+        d.set(f, a)
+    for _ in range(4):
+        for f, a in want.items():
+            assert np.array_equal(d.get(f).view(np.uint64), a.view(np.uint64)), (s, f)
+    d.close()
+
+
+@pytest.mark.gpu
+def test_more_time_steps_than_nodes():
+    from lulesh_amd import grad_run, run
+    print("[first reads] dt record", flush=True)
+    n = 2500  # 20 KB of time steps, staging of 16
+    d = domain(2)
+    d.stoptime = 1.0e9
+    r = grad_run(d, n, 500)
+    time = d.time
+    d.reset()
+    d.stoptime = 1.0e9
+    run(d, n)
+    assert d.time == time and r["dt"].size == n
+    t = 0.0
+    for dt in r["dt"]:
+        t = t + dt
+    assert t == time and r["dt"][-1] == d.deltatime
+    d.close()
+
+
+READS = """
+import time
+import numpy as np
+from lulesh_amd import Batch, run
+Batch([10]).close()
+times = []
+for _ in range(16):
+    b = Batch([20])
+    d = b.instance(0)
+    run(d, 10)
+    t = [time.perf_counter()]
+    for f in ("e", "x", "p"):
+        d.get(f)
+        t.append(time.perf_counter())
+    b.close()
+    times.append(np.diff(t))
+print(*np.median(times[1:], axis=0))
+"""
+
+
+@pytest.mark.gpu
+def test_first_reads_take_what_later_ones_do():
+    """A pinned allocation takes about 300 us where the process has none of its
+    size left over, a read of a small field about 15: medians over contexts,
+    each read three times, in a process of its own."""
+    print("[first reads] times", flush=True)
+    env = dict(os.environ, PYTHONPATH=os.path.join(REPO, "lulesh.jl_amd"))
+    r = subprocess.run([sys.executable, "-c", READS], capture_output=True, text=True, env=env, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    first, second, third = map(float, r.stdout.split())
+    assert max(first, second) < 8 * third, (first, second, third)
