@@ -303,7 +303,7 @@ int lulesh_set_timing(lulesh_ctx *ctx, int32_t on);
  * `depth` node planes of its node column (16x14 nodes for large domains);
  * in a single-domain context the first chunk takes one plane more, so
  * that every chunk but the last marches depth + 1 element planes.
-  * 0 restores the default: one domain whose tiles x node planes all fit on
+ * 0 restores the default: one domain whose tiles x node planes all fit on
  * the device at once (nx <= 34) is not marched at all, a workgroup computing
  * the two element planes around its node plane; larger ones take the chunk
  * count whose modelled time, start plus planes marched per round of CUs x the
@@ -311,7 +311,10 @@ int lulesh_set_timing(lulesh_ctx *ctx, int32_t on);
  * the depth that minimises (launch rounds x planes per workgroup).  Tile shape: per
  * instance the etx x (256/etx) element tile, etx in [lo, hi], that covers
  * the node columns with the fewest tiles (lulesh_set_nodal_tiles; 0, 0
- * restores the default 16..32; 2 <= lo <= hi <= 128); lulesh_nodal_tile
+ * restores the default 16..32; 2 <= lo <= hi <= 128; a tile with more than
+ * 297 nodes around it, etx <= 6 and some from 49 on, runs one workgroup to a
+ * CU instead of two: at s=90 291 us a cycle with etx 2, 120 with 24..32);
+ * lulesh_nodal_tile
  * reports an instance's {etx, ety, tiles along x, tiles along y}.  Neither
  * changes any result: every node sums its corners in the same order.
  * lulesh_autotune times k_nodal on the live state for five tile-width

@@ -381,8 +381,7 @@ int auto_depth(const lulesh_ctx *c) {
   pi.reserve(c->inst.size());
   for (const InstDesc &I : c->inst) pi.push_back({I.s, NodalTile{I.etx, I.ety, I.tx, I.ty}});
   if (c->n == 1) return auto_depth_one(pi[0], c->cus, c->nodal_per_cu);
-  return lulesh::auto_depth(pi.data(), pi.size(), (int64_t)c->cus * c->nodal_per_cu,
-                            balanced_cut(c));
+  return lulesh::auto_depth(pi.data(), pi.size(), (int64_t)c->cus * c->nodal_per_cu, false);
 }
 
 // k_nodal dispatch table (nodal_order) uploaded for the instances in

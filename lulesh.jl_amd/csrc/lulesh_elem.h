@@ -16,8 +16,9 @@
 
 #define LDEV __device__ __forceinline__
 // Keeps the compiler from computing ahead of here what these three values
-// do not need: a statement they pass through.  It emits no instruction but
-// aligns the ones after it to 8 bytes: a wave that issues alone takes five
+// do not need: a statement they pass through.  Where the code lies at 4 mod 8
+// it pads with one 4-byte s_nop, so that the instructions after it start at 0
+// mod 8: a wave that issues alone takes five
 // cycles for an 8-byte FP64 instruction at an address of 4 mod 8 and four
 // for one at 0 mod 8 (measured on chains of 2,048), and every 4-byte
 // instruction in between turns the one into the other.

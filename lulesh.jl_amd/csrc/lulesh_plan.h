@@ -132,10 +132,8 @@ struct NodalPlanInst {
 // `slots` (CUs x resident workgroups per CU): the estimate
 //   ceil(workgroups / slots) * (depth + 1)
 // is minimised over all depths (the smaller depth on ties, for balance),
-// each instance cut by depth_cut.  At s=192 on 256 CUs x 2 this picks 3
-// chunks (504 workgroups, one round; plain cut 65, 66 and 63 element planes,
-// balanced 65, 65 and 64) over 13 chunks of depth 15 (2184 workgroups, 4.3
-// rounds).
+// each instance cut by depth_cut.  The library asks for a batch's plain cut;
+// one domain's balanced one is auto_depth_one's.
 inline int auto_depth(const NodalPlanInst *insts, size_t n, int64_t slots, bool balanced) {
   int maxm = 2;
   for (size_t i = 0; i < n; ++i) maxm = insts[i].s + 1 > maxm ? insts[i].s + 1 : maxm;
@@ -166,7 +164,9 @@ inline int auto_depth(const NodalPlanInst *insts, size_t n, int64_t slots, bool 
 // auto_depth takes the two for equal and, with few blocks, doubles up CUs
 // where fewer, deeper chunks on a CU each are faster: launches at s=48 29.6
 // -> 26.9 us (depth 2, 288 workgroups -> depth 3, 192), s=52 30.6 -> 27.9,
-// s=40 23.0 -> 22.4; from s=56 on both choose alike.
+// s=40 23.0 -> 22.4; from s=56 on both choose alike, at s=192 3 chunks (504
+// workgroups, one round; 65, 65 and 64 element planes) over 13 of depth 15
+// (2184 workgroups, 4.3 rounds).
 inline int auto_depth_one(const NodalPlanInst &I, int64_t cus, int64_t per_cu) {
   if (cus < 1) cus = 1;
   const int64_t slots = per_cu > 1 ? cus * per_cu : cus;
