@@ -606,10 +606,9 @@ int create(int32_t n, const int32_t *nx, const double *einit_scale, const double
     if (he != hipSuccess) rc = hip_fail(c, he, "hipStreamCreate");
   }
   if (!rc) {
-    // the scalars' mirror and behind it the staging memory: for a field, or
-    // with one domain the three arrays of parameter gradients together
+    // the scalars' mirror and the staging memory behind it
     int64_t most = 0;
-    for (const InstDesc &I : c->inst) most = std::max<int64_t>(most, n == 1 ? 3 * I.N : I.N);
+    for (const InstDesc &I : c->inst) most = std::max<int64_t>(most, I.N);
     const size_t mirror = (sizeof(DevScalars) * n + 255) / 256 * 256;
     const size_t stage = HostCopy::staging((size_t)most * sizeof(double));
     he = hipHostMalloc((void **)&c->hsc, mirror + stage, hipHostMallocDefault);

@@ -1,8 +1,9 @@
 // Copies to (and from) the host through pinned staging memory, one per
 // context.  What a small field takes is allocated with the context, in one
-// piece with its scalars: the first pinned allocation of its size takes up to
-// 500 us, and a context of s=20 that was read twice paid it twice (its first
-// two fields 327 and 339 us instead of 32 and 29).
+// piece with its scalars: pinned memory that the process has none of left over
+// takes up to 350 us, a 2 MiB page of it, and a context of s=20 that was read
+// twice paid it twice (its first two fields 327 and 339 us instead of 32 and
+// 29).
 //
 // A copy straight into pageable memory costs the runtime a pass of its own
 // over the destination, page by page and on one thread: a fresh array's pages
@@ -38,9 +39,10 @@ class HostCopy {
     for (hipEvent_t e : ev_)
       if (e) (void)hipEventDestroy(e);
     if (slots_) (void)hipHostFree(slots_);
+    if (wide_) (void)hipHostFree(wide_);
   }
 
-  // staging for a context that copies `bytes` at a time where it can
+  // staging for a context whose largest field has `bytes`
   static size_t staging(size_t bytes) { return std::min(std::max(bytes, kLeast), kChunk); }
   // pinned memory of that size, which the caller frees after its last call here
   void use(void *pinned, size_t bytes) {
@@ -82,11 +84,17 @@ class HostCopy {
   hipError_t stream(hipStream_t st, const double *src, int arrays, int64_t n, F f) {
     std::lock_guard<std::mutex> l(one_);
     const int64_t m = (int64_t)(kChunk / sizeof(double)), chunks = (n + m - 1) / m;
-    if ((size_t)(arrays * n) * sizeof(double) <= pinned_) {
+    const size_t all = (size_t)(arrays * n) * sizeof(double);
+    if (all <= kChunk) {
+      char *to = pin_;
       hipError_t e = hipSuccess;
-      if (n > 0) e = hipMemcpyAsync(pin_, src, (size_t)(arrays * n) * sizeof(double), hipMemcpyDeviceToHost, st);
+      if (all > pinned_) {
+        if (all > wide_bytes_) e = widen(all);
+        to = wide_;
+      }
+      if (e == hipSuccess && n > 0) e = hipMemcpyAsync(to, src, all, hipMemcpyDeviceToHost, st);
       if (e == hipSuccess) e = hipStreamSynchronize(st);
-      if (e == hipSuccess) f((const double *)pin_, n, n);
+      if (e == hipSuccess) f((const double *)to, n, n);
       return e;
     }
     hipError_t e = ready();
@@ -118,6 +126,8 @@ class HostCopy {
   std::mutex one_;  // threads that read one context's fields take turns
   char *pin_ = nullptr;    // the staging memory of small fields
   size_t pinned_ = 0;
+  char *wide_ = nullptr;   // for several arrays at once, from the first such copy on
+  size_t wide_bytes_ = 0;
   char *slots_ = nullptr;  // kSlots chunks
   hipEvent_t ev_[kSlots] = {};
   std::atomic<int> busy_[kSlots] = {};  // pieces that still read the slot
@@ -125,6 +135,16 @@ class HostCopy {
   CopyPool::Queue queue_;
 
   char *slot(int i) { return slots_ + (size_t)i * kChunk; }
+
+  hipError_t widen(size_t bytes) {
+    if (wide_) (void)hipHostFree(wide_);
+    wide_ = nullptr;
+    wide_bytes_ = 0;
+    const hipError_t e = hipHostMalloc((void **)&wide_, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) wide_ = nullptr;
+    else wide_bytes_ = bytes;
+    return e;
+  }
 
   // the chunks and their events
   hipError_t ready() {
