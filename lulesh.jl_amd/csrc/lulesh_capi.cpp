@@ -607,10 +607,11 @@ int create(int32_t n, const int32_t *nx, const double *einit_scale, const double
   }
   if (!rc) {
     // the scalars' mirror and the staging memory behind it
-    int64_t most = 0;
-    for (const InstDesc &I : c->inst) most = std::max<int64_t>(most, I.N);
-    const size_t mirror = (sizeof(DevScalars) * n + 255) / 256 * 256;
-    const size_t stage = HostCopy::staging((size_t)most * sizeof(double));
+    size_t most = 0;
+    for (const InstDesc &I : c->inst)
+      for (const int64_t k : {I.N, I.E})
+        if (HostCopy::small((size_t)k * sizeof(double))) most = std::max(most, (size_t)k * sizeof(double));
+    const size_t mirror = (sizeof(DevScalars) * n + 255) / 256 * 256, stage = HostCopy::staging(most);
     he = hipHostMalloc((void **)&c->hsc, mirror + stage, hipHostMallocDefault);
     if (he != hipSuccess) rc = hip_fail(c, he, "hipHostMalloc");
     else c->host.use((char *)c->hsc + mirror, stage);

@@ -42,8 +42,10 @@ class HostCopy {
     if (wide_) (void)hipHostFree(wide_);
   }
 
-  // staging for a context whose largest field has `bytes`
-  static size_t staging(size_t bytes) { return std::min(std::max(bytes, kLeast), kChunk); }
+  // whether a field of `bytes` takes one copy through the staging memory
+  static bool small(size_t bytes) { return bytes <= kChunk; }
+  // staging for a context whose largest such field has `bytes`
+  static size_t staging(size_t bytes) { return std::max(bytes, kLeast); }
   // pinned memory of that size, which the caller frees after its last call here
   void use(void *pinned, size_t bytes) {
     pin_ = (char *)pinned;
@@ -53,26 +55,25 @@ class HostCopy {
   // dst[0, bytes) = device src; on return the copy is done and `st` idle.
   hipError_t fetch(hipStream_t st, void *dst, const void *src, size_t bytes) {
     std::lock_guard<std::mutex> l(one_);
-    if (bytes > kChunk) return fetch_chunks(st, (char *)dst, (const char *)src, bytes);
-    hipError_t e = hipSuccess;
-    for (size_t o = 0, m; o < bytes && e == hipSuccess; o += m) {
-      m = std::min(bytes - o, pinned_);
-      e = hipMemcpyAsync(pin_, (const char *)src + o, m, hipMemcpyDeviceToHost, st);
-      if (e == hipSuccess) e = hipStreamSynchronize(st);
-      if (e == hipSuccess) memcpy((char *)dst + o, pin_, m);
-    }
-    return bytes ? e : hipStreamSynchronize(st);
+    if (!small(bytes)) return fetch_chunks(st, (char *)dst, (const char *)src, bytes);
+    char *to = nullptr;
+    hipError_t e = room(bytes, &to);
+    if (e == hipSuccess && bytes) e = hipMemcpyAsync(to, src, bytes, hipMemcpyDeviceToHost, st);
+    if (e == hipSuccess) e = hipStreamSynchronize(st);
+    if (e == hipSuccess && bytes) memcpy(dst, to, bytes);
+    return e;
   }
 
   // device dst = src[0, bytes); on return the copy is done and `st` idle.
-  // (Beyond the staging memory the runtime's own copy does; below, it takes 60
-  // us where this takes 15.)
+  // (Beyond a chunk the runtime's own copy does; below, it takes 60 us where
+  // this takes 15.)
   hipError_t send(hipStream_t st, void *dst, const void *src, size_t bytes) {
     std::lock_guard<std::mutex> l(one_);
-    const bool staged = bytes <= pinned_;
-    hipError_t e = hipSuccess;
-    if (staged && bytes) memcpy(pin_, src, bytes);
-    if (bytes) e = hipMemcpyAsync(dst, staged ? pin_ : src, bytes, hipMemcpyHostToDevice, st);
+    const bool staged = small(bytes);
+    char *to = nullptr;
+    hipError_t e = staged ? room(bytes, &to) : hipSuccess;
+    if (e == hipSuccess && staged && bytes) memcpy(to, src, bytes);
+    if (e == hipSuccess && bytes) e = hipMemcpyAsync(dst, staged ? to : src, bytes, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     return e;
   }
@@ -85,13 +86,9 @@ class HostCopy {
     std::lock_guard<std::mutex> l(one_);
     const int64_t m = (int64_t)(kChunk / sizeof(double)), chunks = (n + m - 1) / m;
     const size_t all = (size_t)(arrays * n) * sizeof(double);
-    if (all <= kChunk) {
-      char *to = pin_;
-      hipError_t e = hipSuccess;
-      if (all > pinned_) {
-        if (all > wide_bytes_) e = widen(all);
-        to = wide_;
-      }
+    if (small(all)) {
+      char *to = nullptr;
+      hipError_t e = room(all, &to);
       if (e == hipSuccess && n > 0) e = hipMemcpyAsync(to, src, all, hipMemcpyDeviceToHost, st);
       if (e == hipSuccess) e = hipStreamSynchronize(st);
       if (e == hipSuccess) f((const double *)to, n, n);
@@ -120,13 +117,13 @@ class HostCopy {
   // threads share a chunk by pieces, so that a few chunks occupy them all (57
   // MB with 4, 6, 16 chunks in flight 2.17, 1.95, 1.92 ms; six are pinned in
   // the time of one download of 7 MB).
-  static constexpr size_t kChunk = 1 << 20, kPiece = 1 << 17, kLeast = 1 << 14;
+  static constexpr size_t kChunk = 1 << 20, kPiece = 1 << 17, kLeast = 1 << 16;
   static constexpr int kSlots = 6;
   static_assert(kSlots * (int)(kChunk / kPiece) <= CopyPool::kPieces, "a queue holds what is in flight");
   std::mutex one_;  // threads that read one context's fields take turns
   char *pin_ = nullptr;    // the staging memory of small fields
   size_t pinned_ = 0;
-  char *wide_ = nullptr;   // for several arrays at once, from the first such copy on
+  char *wide_ = nullptr;   // for what that does not hold, while there are no chunks
   size_t wide_bytes_ = 0;
   char *slots_ = nullptr;  // kSlots chunks
   hipEvent_t ev_[kSlots] = {};
@@ -136,14 +133,21 @@ class HostCopy {
 
   char *slot(int i) { return slots_ + (size_t)i * kChunk; }
 
-  hipError_t widen(size_t bytes) {
-    if (wide_) (void)hipHostFree(wide_);
-    wide_ = nullptr;
-    wide_bytes_ = 0;
-    const hipError_t e = hipHostMalloc((void **)&wide_, bytes, hipHostMallocDefault);
-    if (e != hipSuccess) wide_ = nullptr;
-    else wide_bytes_ = bytes;
-    return e;
+  // staging memory of at least `bytes`, at most a chunk
+  hipError_t room(size_t bytes, char **to) {
+    if (bytes > pinned_ && !slots_ && bytes > wide_bytes_) {
+      if (wide_) (void)hipHostFree(wide_);
+      wide_ = nullptr;
+      wide_bytes_ = 0;
+      const hipError_t e = hipHostMalloc((void **)&wide_, bytes, hipHostMallocDefault);
+      if (e != hipSuccess) {
+        wide_ = nullptr;
+        return e;
+      }
+      wide_bytes_ = bytes;
+    }
+    *to = bytes <= pinned_ ? pin_ : slots_ ? slots_ : wide_;
+    return hipSuccess;
   }
 
   // the chunks and their events

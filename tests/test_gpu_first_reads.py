@@ -18,20 +18,27 @@ def domain(s):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("s", [1, 11, 12, 49, 50, 51])
+@pytest.mark.parametrize("s", [1, 19, 20, 49, 50, 51, 63, 64])
 def test_reads_of_a_fresh_context(s):
-    # staging of a node array, 16 KiB at least (s=11 13.8 KB, 12 17.6) and 1
-    # MiB at most; fields beyond that from s=50 (1.00 and 1.06 MB) and 51 (1.06
-    # and 1.12) on
+    # staging of the largest field up to 1 MiB, 64 KiB at least (s=19 64.0 KB of
+    # nodes, 20 74): s=49 1.00 MB of nodes, 50 1.00 MB of elements, from 51 on
+    # none, where the masks still have less (s=63 1.00 MB, 64 1.05)
     print(f"[first reads] s={s}", flush=True)
     g = np.random.default_rng(s)
     d = domain(s)
     want = {f: g.standard_normal(d.numNode if f in ("x", "zd") else d.numElem) for f in ("x", "e", "zd", "ss")}
-    for f, a in want.items():
-        d.set(f, a)
-    for _ in range(4):
+    bc = g.integers(0, 2 ** 18, d.numElem).astype(np.uint32)
+    for first in ("elemBC", "e"):  # before there are chunks, and with them
+        d.set("elemBC", bc)
+        if first == "elemBC":
+            assert np.array_equal(d.get("elemBC"), bc)
+        for f, a in want.items():
+            d.set(f, a)
         for f, a in want.items():
             assert np.array_equal(d.get(f).view(np.uint64), a.view(np.uint64)), (s, f)
+        assert np.array_equal(d.get("elemBC"), bc)
+        from lulesh_amd import verify
+        assert verify(d)[0] == want["e"][0]
     d.close()
 
 
@@ -39,10 +46,10 @@ def test_reads_of_a_fresh_context(s):
 def test_more_time_steps_than_nodes():
     from lulesh_amd import grad_run, run
     print("[first reads] dt record", flush=True)
-    n = 2500  # 20 KB of time steps, staging of 16
+    n = 9000  # 72 KB of time steps, staging of 64 KiB
     d = domain(2)
     d.stoptime = 1.0e9
-    r = grad_run(d, n, 500)
+    r = grad_run(d, n, 1000)
     time = d.time
     d.reset()
     d.stoptime = 1.0e9
@@ -56,10 +63,10 @@ def test_more_time_steps_than_nodes():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("s", [1, 6, 9, 20, 35, 36])
+@pytest.mark.parametrize("s", [1, 13, 14, 20, 35, 36])
 def test_parameter_sums_through_each_staging(s):
     """The three arrays of parameter gradients in the field's staging memory
-    (s=6 5.2 of 16 KiB), in their own (s=9 17 KB, 35 1.03 MB) and in chunks
+    (s=13 52.7 of 64 KiB), in their own (s=14 65.9 KB, 35 1.03 MB) and in chunks
     (s=36 1.12 MB): vjp_cycle's sums are those of a one-cycle gradient, and are
     the same when the memory is there already."""
     from lulesh_amd import grad_run, timeIncrement, vjp_cycle
